@@ -109,7 +109,7 @@ struct tg_ctx {
   int* thin_count = nullptr;
   // tiles taking the full path of the update / adjoint (compacted by their
   // classifying pass) and the list length
-  int* act_list = nullptr;
+  TileRef* act_list = nullptr;  // (the FP32 adjoint lists bare tile indices in it)
   int* act_count = nullptr;
 
   // adaptive mesh (TG_MESH_LEAVES): leaf tables and reverse-step buffers
@@ -544,7 +544,7 @@ void enqueue_adjoint_m(tg_ctx* ctx, void* const U[3], void* const lnext[3], void
   a.thin_count = ctx->thin_count;
   a.s64 = (ctx->ses == 8) ? (const double*)ctx->statics : nullptr;
   a.ncell = ctx->ncell;
-  a.tile_list = ctx->act_list;
+  a.tile_list = (int*)ctx->act_list;
   a.tile_count = ctx->act_count;
   a.mk_U = marks_of(ctx, U);
   a.mk_lnext = marks_of(ctx, lnext);
@@ -1364,7 +1364,7 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
     if (params) params_into(I, &params[0]);
     for (int v = 0; v < NSHAPE; v++)
       for (int x = 0; x < meshes[0].n; x += BLOCK)
-        ctx->tiles_h[v].push_back(TileDev{0, x, 0, 0, -1, -1, -1, -1});
+        ctx->tiles_h[v].push_back(TileDev{0, x, 0, 0, -1, -1, -1, -1, meshes[0].n, 1, 0});
     off = meshes[0].n;
   }
   // leaf chunks (the BLOCK leaves of one workgroup) carry one zero-mark word
@@ -1412,7 +1412,8 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
           ctx->tiles_h[v].push_back(TileDev{b, tx, ty, mw, bx > 0 ? mw - 1 : -1,
                                             bx + 1 < I.nsx ? mw + 1 : -1,
                                             by > 0 ? mw - I.nsx : -1,
-                                            by + 1 < I.nsy ? mw + I.nsx : -1});
+                                            by + 1 < I.nsy ? mw + I.nsx : -1, m->nx, m->ny,
+                                            off});
         }
     }
     off += (long long)m->nx * m->ny;
@@ -1490,7 +1491,7 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
   if (!rc && ctx->mode != TG_FP64)
     rc = dalloc(ctx, (void**)&ctx->thin_list, sizeof(int2) * (size_t)n);
   if (!rc && ctx->mode != TG_FP64) rc = dalloc(ctx, (void**)&ctx->thin_count, sizeof(int));
-  if (!rc) rc = dalloc(ctx, (void**)&ctx->act_list, sizeof(int) * (size_t)ctx->ntiles);
+  if (!rc) rc = dalloc(ctx, (void**)&ctx->act_list, sizeof(TileRef) * (size_t)ctx->ntiles);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->act_count, sizeof(int));
   if (!rc) rc = dalloc(ctx, (void**)&ctx->inst_d, sizeof(InstDev) * nm);
   for (int v = 0; v < NSHAPE && !rc; v++)

@@ -44,10 +44,20 @@ __device__ __forceinline__ MatDev mat_of(const InstDev& I, const uint8_t* mat, c
 // A launch tile: TX x (BLOCK / TX) cells of instance `inst` starting at
 // (x0, y0).  One workgroup per tile.  mw: the zero-mark word of the tile's
 // block; mwW, mwE, mwS, mwN: those of the four side blocks (-1 outside the
-// member).
+// member).  nx, ny, off: the member's extent and first cell (InstDev), so a
+// workgroup addresses its cells without the member record.
 struct TileDev {
   int inst, x0, y0, mw;
   int mwW, mwE, mwS, mwN;
+  int nx, ny;
+  long long off;
+};
+
+// An entry of the compacted list of full-path tiles: what the listed tile's
+// workgroup needs before it can address its cells, in one load.
+struct TileRef {
+  int inst, tile, x0, y0, mw, nx, ny, pad;
+  long long off;
 };
 
 // A run of at most BOX_CHUNK listed box cells [begin, end) of member inst
@@ -115,8 +125,8 @@ __device__ __forceinline__ int list_band(int p, int n) {
   return x * q + (x < r ? x : r) + p / NXCD;
 }
 // the byte of its block's word that a tile of width TX owns
-template <int TX>
-__device__ __forceinline__ int mark_byte(const TileDev& t) {
+template <int TX, class T>
+__device__ __forceinline__ int mark_byte(const T& t) {
   constexpr int TY = BLOCK / TX;
   return ((t.y0 % MARK_H) / TY) * (MARK_W / TX) + (t.x0 % MARK_W) / TX;
 }
@@ -163,7 +173,7 @@ struct StepArgs {
   unsigned long long* active;
   // compacted list of the tiles that take the update's full path (written
   // by the classifying pass, walked by the update) and its length
-  int* tile_list;
+  TileRef* tile_list;
   int* tile_count;
   // 1: k_dt clears tile_count (the update pass then launches no fill)
   int dt_clears_count;
@@ -204,7 +214,7 @@ struct AdjArgs {
   double* lam_hv;
   double* dphi_part;     // [ntiles] running sum of lambda^{s+1}.dU/dphi, or null
   unsigned long long* active;  // null, or counter of cells in non-void tiles
-  int* tile_list;        // compacted non-void tiles (classifying pass) and count
+  TileRef* tile_list;    // compacted non-void tiles (classifying pass) and count
   int* tile_count;
   // zero marks of U^s, lambda^{s+1} and lambda^s (all null: no marks) and
   // the short-path cell counter, as in StepArgs
@@ -311,6 +321,9 @@ constexpr int THIN_GRID = 1024;
 // the listed tiles spread over every CU (1024, 2048, 4096 and 8192 measured
 // on the 256-member ensemble: 4096 about 1 % ahead)
 constexpr int LIST_GRID = 4096;
+// workgroups of the FP64 adjoint's list walk, and its waves per SIMD
+constexpr int ADJ_GRID = 2048;
+constexpr int ADJ_WAVES = 3;
 
 template <class S>
 void launch_coef_m(const StepArgsM<S>& a, bool reduce, hipStream_t s);

@@ -67,6 +67,20 @@ __device__ __forceinline__ Cell cell_of(const TileDev& t, const InstDev& I) {
   return q;
 }
 
+template <int TX>
+__device__ __forceinline__ Cell cell_of(const TileRef& t) {
+  Cell q;
+  q.i = t.x0 + (int)(threadIdx.x % TX);
+  q.j = t.y0 + (int)(threadIdx.x / TX);
+  q.act = q.i < t.nx && q.j < t.ny;
+  q.c = t.off + (long long)q.j * t.nx + q.i;
+  q.hasE = q.i + 1 < t.nx;
+  q.hasW = q.i > 0;
+  q.hasN = q.j + 1 < t.ny;
+  q.hasS = q.j > 0;
+  return q;
+}
+
 // ------------------------------------------------------------- zero marks --
 
 __device__ __forceinline__ bool bitzero3(double a, double b, double c) {
@@ -75,8 +89,8 @@ __device__ __forceinline__ bool bitzero3(double a, double b, double c) {
 // Records in the output marks whether the tile holds +0.0 only (all: the
 // workgroup's reduction of "this cell is +0.0 in all three fields or
 // outside the member").  Thread 0 stores the tile's byte.
-template <int TX>
-__device__ __forceinline__ void mark_store(uint32_t* mk, const TileDev& t, bool all) {
+template <int TX, class T>
+__device__ __forceinline__ void mark_store(uint32_t* mk, const T& t, bool all) {
   if (threadIdx.x == 0) ((unsigned char*)(mk + t.mw))[mark_byte<TX>(t)] = all ? 1 : 0;
 }
 
@@ -107,6 +121,13 @@ __device__ __forceinline__ bool adjoint_skip(const uint32_t* mu, const uint32_t*
 // the byte of block word mw that tile byte b owns
 __device__ __forceinline__ void mark_byte_store(uint32_t* mk, int mw, int b, bool zero) {
   ((unsigned char*)(mk + mw))[b] = zero ? 1 : 0;
+}
+// the list entry of tile byte b of a block
+template <int TX>
+__device__ __forceinline__ TileRef tile_ref(const BlockDev& B, int b) {
+  constexpr int TY = BLOCK / TX, PER_ROW = MARK_W / TX;
+  return TileRef{B.inst, B.tile[b], B.x0 + (b % PER_ROW) * TX, B.y0 + (b / PER_ROW) * TY,
+                 B.mw, B.nx, B.ny, 0, B.off};
 }
 // The cells of a block's four tiles this thread handles (one per tile).
 template <int TX>
@@ -404,7 +425,7 @@ __global__ __launch_bounds__(BLOCK) void k_update_classify(StepArgs a) {
     int k = atomicAdd(a.tile_count, __popc(W));
 #pragma unroll
     for (int b = 0; b < 4; b++)
-      if ((W >> b) & 1u) a.tile_list[k++] = B.tile[b];
+      if ((W >> b) & 1u) a.tile_list[k++] = tile_ref<TX>(B, b);
   }
   // the momenta of the dry tiles that hold something (a wet tile's cells are
   // read again by the full path)
@@ -462,7 +483,7 @@ __global__ __launch_bounds__(BLOCK) void k_update_classify(StepArgs a) {
 // update_tile's per-cell part: slopes from the staged differences, the four
 // face fluxes with outflow copies, update_states; z: the new state is +0.0.
 template <int TX>
-__device__ __forceinline__ void update_cell(const StepArgs& a, const TileDev& t,
+__device__ __forceinline__ void update_cell(const StepArgs& a, const TileRef& t,
                                             const InstDev& I, const Cell& q, FaceLds<TX>& L,
                                             bool& z) {
   const int tx = (int)(threadIdx.x % TX), ty = (int)(threadIdx.x / TX);
@@ -505,11 +526,10 @@ __device__ __forceinline__ void update_cell(const StepArgs& a, const TileDev& t,
 // Update pass 2, one listed tile: face fluxes staged in LDS, slopes,
 // update_states.
 template <int TX>
-__device__ __forceinline__ void update_tile(const StepArgs& a, int tile, FaceLds<TX>& L) {
+__device__ __forceinline__ void update_tile(const StepArgs& a, const TileRef& t, FaceLds<TX>& L) {
   constexpr int TY = BLOCK / TX;
-  const TileDev t = a.tiles[tile];
   const InstDev I = a.inst[t.inst];
-  const Cell q = cell_of<TX>(t, I);
+  const Cell q = cell_of<TX>(t);
   const long long nx = I.nx;
   if (a.active) {
     const int cnt = __syncthreads_count(q.act);
@@ -695,264 +715,291 @@ __global__ __launch_bounds__(BLOCK) void k_member_reduce(const double* sum_part,
 
 // ---------------------------------------------------------------- adjoint --
 
-// Everything the Jacobian blocks need about one cell at U^s
-// (DualElem after update_dual_grid + update_states in calc_jacobian).
-struct DualInfo {
-  double h, hu, hv, g2;
-  double k;              // kact from the dual slopes (dual_grid_routines.C:68-84)
-  double dk;             // d kact / d phi_bed
-  double d[6];           // dual slopes hx, hux, hvx, hy, huy, hvy
-  double hsx[3], hsy[3]; // hslope_sens(dir, self/minus/plus)
-  SrcInfo si;
-};
+// A double from the other thread of a pair (two 32-bit DPP moves, no LDS).
+__device__ __forceinline__ double swap_pair(double v) {
+  constexpr int ctrl = 1 | (0 << 2) | (3 << 4) | (2 << 6);
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
 
-__device__ __forceinline__ DualInfo dual_info(const AdjArgs& a, const InstDev& I, int i, int j,
-                                              bool want_dk) {
-  DualInfo r;
-  const long long nx = I.nx, c = I.off + (long long)j * nx + i;
-  r.h = a.U.h[c]; r.hu = a.U.hu[c]; r.hv = a.U.hv[c]; r.g2 = a.S.gz[c];
+// Reverse step, one tile of 256 cells by 512 threads.
+//
+// Phase 1, one thread per record (the tile's cells and the four side
+// strips of its halo): the dual slopes, kact, source switches and what the
+// faces and blocks read of a cell, staged in LDS with its lambda^{s+1}.  Every
+// load of a record is issued before any of it is looked at.
+// Phase 2, two threads per cell, one its y faces and one its x faces: the
+// faces' Jacobians with respect to the cell (dual_riemannflux,
+// dualmesh.C:1628-1843) in the face's own frame -- 0 depth, n normal and t
+// tangential momentum -- where seven of the nine entries can differ from
+// zero (rows 0 and n have no t column), then the gather lambda^s = g -
+// sum_j J_j^T lambda_j, whose running sum the pair hands back and forth in the
+// reference's order self, S, E, N, W (neighbor[0..3] with positive_x_side =
+// 1).  The products left out are exact zeros, and adding a zero to a running
+// sum that starts at +0.0 changes nothing, so the result is the reference's
+// bit for bit.  The bed-friction gradient's face fluxes come out of the same
+// evaluation.
+//
+// What bounds it: FP64 instruction issue (52 % of the issue slots at 128
+// VGPRs, four waves per SIMD) and, per tile, three round trips to memory (list
+// entry, records, results).  A 64-member ensemble of 5.8 M cells: 51 us per
+// step against 81 us for one thread per cell with every face's forward and
+// dual flux evaluated apart (26.0 M wave instructions, now 15.6 M); one
+// tile alone: 13.8 against 27 us.  One thread per cell needs 168 VGPRs (81
+// us), four per cell repeat the self block (75 us).
+template <int TX, bool DPHI>
+struct DualLds {
+  static constexpr int RX = TX + 2, RN = (TX + 2) * (BLOCK / TX + 2);
+  // records: the state, +0.0 where h < tiny (the flux functions' void side),
+  // 1/h and sqrt(kact h g2)
+  double h[RN], hu[RN], hv[RN], inv[RN], sq[RN];
+  // the source term that the cell's block as x- / x+ / y- / y+ neighbour's
+  // neighbour subtracts (compute_jacobian_elem.C:44-51)
+  double src[4][RN];
+  double lam[3][RN];  // lambda^{s+1}
+  // bed-friction gradient: d kact / d phi_bed times d F_n / d kact and
+  // d sqrt(kact h g2) / d kact
+  double dF[DPHI ? RN : 1], dw[DPHI ? RN : 1];
+  // the tile's cells: what the self block subtracts from its entries 10, 10,
+  // 11, 20, 20, 22 (compute_jacobian_elem.C:55-110), the sources' phi_bed
+  // derivatives, and whether h != 0
+  double self[6][BLOCK];
+  double dsrc[2][DPHI ? BLOCK : 1];
+  double sp[2 * BLOCK / 64];
+  unsigned char nz[BLOCK];
+};
+constexpr int ADJ_THREADS = 2 * BLOCK;
+
+// .5 * c_sgn and f_sgn (tg_math.h) by the sign bit
+__device__ __forceinline__ double half_sgn(double z, double tiny) {
+  return fabs(z) > tiny ? copysign(.5, z) : 0.;
+}
+// slope_dual (tg_math.h); hs: its sensitivities for the cell itself and its
+// minus and plus neighbour
+__device__ __forceinline__ double dslope(double up, double uc, double um, double dx, double inv,
+                                         double inv_s, double gamma, double tiny,
+                                         double* hs = nullptr) {
+  const double dp = (up - uc) * inv, dm = (uc - um) * inv;
+  const double dc = (dp * dx + dm * dx) * inv_s;
+  const double gp = gamma * fabs(dp), gm = gamma * fabs(dm);
+  const double mn = fmin(fmin(gp, gm), fabs(dc));
+  const double sg = half_sgn(dp, tiny) + half_sgn(dm, tiny);
+  if (hs) {
+    const bool on = sg != 0., P = mn == gp, M = !P && mn == gm, C = !P && !M;
+    const double cen = inv * (dx * inv_s), one = on ? inv : 0.;
+    hs[0] = P ? -one : M ? one : 0.;
+    hs[1] = M ? -one : (on && C) ? -cen : 0.;
+    hs[2] = P ? one : (on && C) ? cen : 0.;
+  }
+  return sg * mn;
+}
+
+// The record of cell (i, j) in slot r; own >= 0: also the self terms of the
+// tile's cell `own` (DualElem after update_dual_grid, dual_grid_routines.C:
+// 68-84, and update_states in calc_jacobian).  Returns whether the cell is not
+// void (h != 0, or with the gradient lambda^{s+1} != 0).
+template <int TX, bool DPHI>
+__device__ __forceinline__ bool dual_record(const AdjArgs& a, const TileRef& t, const InstDev& I,
+                                            int i, int j, double dt, DualLds<TX, DPHI>& L, int r,
+                                            int own) {
+  const long long c = t.off + (long long)j * t.nx + i;
+  // cells on the domain boundary have zero slopes: with themselves as
+  // neighbours every difference is 0, and so are slope and sensitivities
+  const bool inner = i + 1 < t.nx && i > 0 && j + 1 < t.ny && j > 0;
+  const long long ox = inner ? 1 : 0, oy = inner ? t.nx : 0;
+  double h = a.U.h[c], hu = a.U.hu[c], hv = a.U.hv[c];
+  double hE = a.U.h[c + ox], hW = a.U.h[c - ox], hN = a.U.h[c + oy], hS = a.U.h[c - oy];
+  double uE = a.U.hu[c + ox], uW = a.U.hu[c - ox], uN = a.U.hu[c + oy], uS = a.U.hu[c - oy];
+  double vE = a.U.hv[c + ox], vW = a.U.hv[c - ox], vN = a.U.hv[c + oy], vS = a.U.hv[c - oy];
+  double g2 = a.S.gz[c], k0 = a.S.kx[c], k1 = a.S.ky[c];
+  double l0 = a.lam_next.h[c], l1 = a.lam_next.hu[c], l2 = a.lam_next.hv[c];
+  double g0 = 0., g1 = 0., dg0 = 0., dg1 = 0.;
+  if (own >= 0) { g0 = a.S.gx[c]; g1 = a.S.gy[c]; dg0 = a.S.dgx[c]; dg1 = a.S.dgy[c]; }
+  // all of them in flight together (used only below a test of h, they
+  // would be loaded after it)
+  asm volatile("" : "+v"(hE), "+v"(hW), "+v"(hN), "+v"(hS), "+v"(uE), "+v"(uW), "+v"(uN),
+                    "+v"(uS), "+v"(vE), "+v"(vW), "+v"(vN), "+v"(vS));
+  asm volatile("" : "+v"(g2), "+v"(k0), "+v"(k1), "+v"(g0), "+v"(g1), "+v"(dg0), "+v"(dg1),
+                    "+v"(l0), "+v"(l1), "+v"(l2));
+  L.lam[0][r] = l0; L.lam[1][r] = l1; L.lam[2][r] = l2;
+  const bool busy = h != 0. || (DPHI && !(l0 == 0. && l1 == 0. && l2 == 0.));
+  if (own >= 0) L.nz[own] = h != 0.;
+  if (!(h > a.tiny)) {
+    // void side of every flux, or (h = tiny, or not a number) a dry cell:
+    // kact = epsilon, no slopes and no sources
+    const bool flows = !(h < a.tiny);
+    L.h[r] = flows ? h : 0.;
+    L.hu[r] = flows ? hu : 0.;
+    L.hv[r] = flows ? hv : 0.;
+    L.inv[r] = flows ? 1. / h : 0.;
+    L.sq[r] = flows ? sqrt(1. * I.eps * h * g2) : 0.;
 #pragma unroll
-  for (int k = 0; k < 6; k++) r.d[k] = 0.;
+    for (int k = 0; k < 4; k++) L.src[k][r] = 0.;
+    if (DPHI) L.dF[r] = L.dw[r] = 0.;
+    if (own >= 0) {
 #pragma unroll
-  for (int k = 0; k < 3; k++) r.hsx[k] = r.hsy[k] = 0.;
-  if (i + 1 < I.nx && i > 0 && j + 1 < I.ny && j > 0) {
-    const double ix = I.inv_dx, isx = I.inv_sx;
-    const double iy = I.inv_dy, isy = I.inv_sy;
-    DualSlope s = slope_dual(a.U.h[c + 1], r.h, a.U.h[c - 1], I.dx, ix, isx, a.gamma, a.tiny, true);
-    r.d[0] = s.d; r.hsx[0] = s.s0; r.hsx[1] = s.s1; r.hsx[2] = s.s2;
-    r.d[1] = slope_dual(a.U.hu[c + 1], r.hu, a.U.hu[c - 1], I.dx, ix, isx, a.gamma, a.tiny, false).d;
-    r.d[2] = slope_dual(a.U.hv[c + 1], r.hv, a.U.hv[c - 1], I.dx, ix, isx, a.gamma, a.tiny, false).d;
-    s = slope_dual(a.U.h[c + nx], r.h, a.U.h[c - nx], I.dy, iy, isy, a.gamma, a.tiny, true);
-    r.d[3] = s.d; r.hsy[0] = s.s0; r.hsy[1] = s.s1; r.hsy[2] = s.s2;
-    r.d[4] = slope_dual(a.U.hu[c + nx], r.hu, a.U.hu[c - nx], I.dy, iy, isy, a.gamma, a.tiny, false).d;
-    r.d[5] = slope_dual(a.U.hv[c + nx], r.hv, a.U.hv[c - nx], I.dy, iy, isy, a.gamma, a.tiny, false).d;
+      for (int k = 0; k < 6; k++) L.self[k][own] = 0.;
+      if (DPHI) L.dsrc[0][own] = L.dsrc[1][own] = 0.;
+    }
+    return busy;
   }
   const MatDev M = mat_of(I, a.mat, a.mtab, c);
-  r.k = getcoef(r.h, r.hu, r.hv, r.d[0], r.d[1], r.d[3], r.d[5], I.kc1, M.kroot, I.eps, a.tiny);
-  r.dk = want_dk ? dgetcoef_dphi(r.h, r.hu, r.hv, r.d[0], r.d[1], r.d[3], r.d[5], I.kc1, M.kroot,
-                                 M.dkroot, I.eps, a.tiny)
-                 : 0.;
-  r.si = src_switches(r.h, r.hu, r.hv, r.d[0], r.d[2], r.d[3], r.d[4], a.S.kx[c], a.S.ky[c],
-                      M.tan_bed, r.g2, a.ft, a.tiny);
-  return r;
-}
-
-// J = dtdx*(px - nx) + dtdy*(py - ny), calc_jacobian_elem
-// (compute_jacobian_elem.C:21-24); an operand whose flag is false is
-// ZERO_MATRIX.  Operands are taken by value and selected element by element
-// so the blocks stay in registers.
-__device__ __forceinline__ M3 flux_block(const M3& px, bool ux, const M3& nxm, bool unx,
-                                         const M3& py, bool uy, const M3& nym, bool uny,
-                                         double dtdx, double dtdy) {
-  M3 J;
-#pragma unroll
-  for (int i = 0; i < 3; i++)
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-      double a = ux ? px.a[i][j] : 0., b = unx ? nxm.a[i][j] : 0.;
-      double c = uy ? py.a[i][j] : 0., d = uny ? nym.a[i][j] : 0.;
-      J.a[i][j] = +dtdx * (a - b) + dtdy * (c - d);
-    }
-  return J;
-}
-
-// Source-term part of a neighbour block (compute_jacobian_elem.C:44-51).
-__device__ __forceinline__ void nbr_source(M3& J, const DualInfo& n, double sin_int, double dt,
-                                           double dh0, double dh1, double tiny) {
-  if (n.h > tiny) {
-    double alpha = sin_int * n.si.sgn[0] * n.k;
-    double betta = sin_int * n.si.sgn[1] * n.k;
-    if (!n.si.stop[0]) J.a[1][0] -= -dt * n.h * alpha * n.g2 * dh1;
-    if (!n.si.stop[1]) J.a[2][0] -= -dt * n.h * betta * n.g2 * dh0;
+  const double ix = I.inv_dx, isx = I.inv_sx, iy = I.inv_dy, isy = I.inv_sy;
+  double sx[3], sy[3];
+  const double hx = dslope(hE, h, hW, I.dx, ix, isx, a.gamma, a.tiny, sx);
+  const double hy = dslope(hN, h, hS, I.dy, iy, isy, a.gamma, a.tiny, sy);
+  const double hux = dslope(uE, hu, uW, I.dx, ix, isx, a.gamma, a.tiny);
+  const double hvx = dslope(vE, hv, vW, I.dx, ix, isx, a.gamma, a.tiny);
+  const double huy = dslope(uN, hu, uS, I.dy, iy, isy, a.gamma, a.tiny);
+  const double hvy = dslope(vN, hv, vS, I.dy, iy, isy, a.gamma, a.tiny);
+  const double inv = 1. / h;
+  const double vx = div_r(hu, h, inv), vy = div_r(hv, h, inv);
+  L.h[r] = h; L.hu[r] = hu; L.hv[r] = hv; L.inv[r] = inv;
+  // getcoef (tg_math.h) and its phi_bed derivative
+  const double hh = h * h, ihh = 1. / hh;
+  const double vel = div_r(hux, h, inv) - div_r(hu * hx, hh, ihh) + div_r(hvy, h, inv) -
+                     div_r(hv * hy, hh, ihh);
+  const double sg = fabs(vel) < a.tiny ? 0. : copysign(1., vel);
+  const bool still = fabs(vx) < a.tiny && fabs(vy) < a.tiny;
+  const double kf = I.kc1 * (1. - sg * M.kroot) - 1.;
+  const double k = (still ? 1. : (kf < 0. ? 0. : kf)) * I.eps;
+  const double sq = sqrt(k * h * g2);
+  L.sq[r] = sq;
+  // src_switches (tg_math.h)
+  const double tb = M.tan_bed;
+  const double sgn0 = tiny_sgn(inv * (huy - vx * hy), a.ft), sgn2 = tiny_sgn(vx, a.ft);
+  const double sgn1 = tiny_sgn(inv * (hvx - vy * hx), a.ft), sgn3 = tiny_sgn(vy, a.ft);
+  const double fx = umax(g2 * h + vx * hu * k0, 0.0), fy = umax(g2 * h + vy * hv * k1, 0.0);
+  const bool stop0 = sgn2 * fx * tb == 0. && sgn2 != 0.;
+  const bool stop1 = sgn3 * fy * tb == 0. && sgn3 != 0.;
+  const double alpha = I.sin_int * sgn0 * k, betta = I.sin_int * sgn1 * k;
+  const double bx = stop1 ? 0. : -dt * h * betta * g2, by = stop0 ? 0. : -dt * h * alpha * g2;
+  L.src[0][r] = bx * sx[1]; L.src[1][r] = bx * sx[2];
+  L.src[2][r] = by * sy[1]; L.src[3][r] = by * sy[2];
+  double dk = 0.;
+  if (DPHI) {
+    dk = (still || kf < 0.) ? 0. : -I.kc1 * sg * M.dkroot * I.eps;
+    L.dw[r] = (sq > 0.) ? dk * ((h * g2) / (2. * sq)) : 0.;
+    L.dF[r] = dk * (0.5 * h * g2 * h);
   }
+  if (own >= 0) {
+    L.self[0][own] = dt * (g0 - alpha * h * (2 * dg1 + g2 * sy[0]) - alpha * g2 * hy);
+    L.self[3][own] = dt * (g1 - betta * h * (2 * dg0 + g2 * sx[0]) - betta * g2 * hx);
+    const double f0 = (sgn2 != 0. && !stop0) ? -dt * sgn2 * tb : 0.;
+    const double f1 = (sgn3 != 0. && !stop1) ? -dt * sgn3 * tb : 0.;
+    L.self[1][own] = f0 * (g2 - vx * vx * k0);
+    L.self[2][own] = f0 * (2 * vx * k0);
+    L.self[4][own] = f1 * (g2 - vy * vy * k1);
+    L.self[5][own] = f1 * (2 * vy * k1);
+    if (DPHI) {
+      const double sec2 = 1. + tb * tb;
+      L.dsrc[0][own] = dt * (-(sgn0 * h * dk * (g2 * hy + dg1 * h) * I.sin_int) - sgn2 * fx * sec2);
+      L.dsrc[1][own] = dt * (-(sgn1 * h * dk * (g2 * hx + dg0 * h) * I.sin_int) - sgn3 * fy * sec2);
+    }
+  }
+  return busy;
 }
 
-__device__ __forceinline__ void accum_T(double adj[3], const M3& J, const double lam[3]) {
-#pragma unroll
-  for (int k = 0; k < 3; k++)
-#pragma unroll
-    for (int l = 0; l < 3; l++) adj[k] += lam[l] * J.a[l][k];
-}
-
-
-// The part of a cell's dual record its neighbours read, staged in LDS for the
-// tile plus a one-cell halo: each record is computed once per workgroup
-// instead of once per reading cell.
-// LDS record slots: the largest tile plus halo over the built tile widths
-// ((TX + 2) * (BLOCK / TX + 2) is largest at TX = 64)
-constexpr int RN = (64 + 2) * (BLOCK / 64 + 2);
-struct DualLds {
-  double h[RN], hu[RN], hv[RN], g2[RN], k[RN], dk[RN];
-  double hsx1[RN], hsx2[RN], hsy1[RN], hsy2[RN];
-  int flags[RN];  // sgn0+1 | (sgn1+1)<<2 | stop0<<4 | stop1<<5
-  // per record, for h >= tiny: 1/h and sqrt(k h g2) (dual_hfv, hfv_fwd,
-  // dhfv_dk), hu/h and hv/h (hfv_fwd), dhfv_dk's da -- each evaluated once
-  // with the expression the flux functions use, instead of once per face
-  double inv[RN], sq[RN], vx[RN], vy[RN], da[RN];
+// One face's Jacobian with respect to the cell, in the face's frame: the
+// entries 00, 0n, n0, nn, t0, tn, tt.
+struct FaceJac {
+  double a00, a0n, an0, ann, at0, atn, att;
+};
+// The face's mass flux, and the derivative of its flux along d kact /
+// d phi_bed on both sides.
+struct FaceDk {
+  double flux0, d0, dn, dt;
 };
 
-__device__ __forceinline__ void lds_put(DualLds& L, int r, const DualInfo& d, double tiny) {
-  L.h[r] = d.h; L.hu[r] = d.hu; L.hv[r] = d.hv; L.g2[r] = d.g2; L.k[r] = d.k; L.dk[r] = d.dk;
-  double inv = 0., sq = 0., vx = 0., vy = 0., da = 0.;
-  if (!(d.h < tiny)) {
-    inv = 1. / d.h;
-    sq = sqrt(d.k * d.h * d.g2);
-    vx = d.hu / d.h;
-    vy = d.hv / d.h;
-    da = (sq > 0.) ? (d.h * d.g2) / (2. * sq) : 0.;
+// dual_riemann_side (tg_math.h) of the face between the cell's record rc and
+// its neighbour's rn, along x (isx) or y, towards plus or minus.  The normal
+// axis points from the cell to the neighbour, so the cell is the left side
+// of every face: where the axis is reversed (plus false) normal momenta and
+// velocities, the mass and the tangential flux change sign and sl, sr become
+// -sr, -sl.  All of it rounds the same, so the caller takes the signs back
+// (of a00, ann, at0, att; flux0, d0, dt).  Only the choice between equal
+// sides depends on the direction.
+template <int TX, bool DPHI>
+__device__ __forceinline__ FaceJac face_jac(const DualLds<TX, DPHI>& L, bool isx, bool plus,
+                                            int rc, int rn, FaceDk& D) {
+  const double* Q = isx ? L.hu : L.hv;  // normal and tangential momentum
+  const double* T = isx ? L.hv : L.hu;
+  const double ch = L.h[rc], ct = T[rc], ci = L.inv[rc], ca = L.sq[rc];
+  const double nh = L.h[rn], nt = T[rn], ni = L.inv[rn], na = L.sq[rn];
+  double cq = Q[rc], nq = Q[rn];
+  if (!plus) { cq = -cq; nq = -nq; }
+  const bool cvoid = ch == 0., nvoid = nh == 0.;
+  const double cv = cq * ci, nv = nq * ni;
+  // wave speeds; next to a void side 2 w - vel of the other one (a void
+  // side's own are 0, so it drops out of the minimum and maximum with 0)
+  const double cw0 = cv - ca, cw2 = cv + ca, nw0 = nv - na, nw2 = nv + na;
+  const double c0 = nvoid ? 2. * cw0 - cv : cw0, c2 = nvoid ? 2. * cw2 - cv : cw2;
+  const double n0 = cvoid ? 2. * nw0 - nv : nw0, n2 = cvoid ? 2. * nw2 - nv : nw2;
+  const double sl = fmin(0., fmin(c0, n0)), sr = fmax(0., fmax(c2, n2));
+  // the cell's flux Jacobian
+  const double cvi = cv * ci, fn0 = ca * ca - cv * cv, ft0 = -cv * ct * ci, ftn = ct * ci;
+  double dwc = 0., dwn = 0., dFc = 0., dFn = 0., dsl = 0., dsr = 0.;
+  if (DPHI) {
+    dwc = L.dw[rc]; dwn = L.dw[rn]; dFc = L.dF[rc]; dFn = L.dF[rn];
+    const double dv = 2. * (cvoid ? dwn : dwc);
+    const bool one = cvoid || nvoid;
+    if (sl < 0.) dsl = -(one ? dv : (c0 > n0 ? dwn : dwc));
+    if (sr > 0.) dsr = one ? dv : (c2 > n2 ? dwc : dwn);
   }
-  L.inv[r] = inv; L.sq[r] = sq; L.vx[r] = vx; L.vy[r] = vy; L.da[r] = da;
-  L.hsx1[r] = d.hsx[1]; L.hsx2[r] = d.hsx[2]; L.hsy1[r] = d.hsy[1]; L.hsy2[r] = d.hsy[2];
-  L.flags[r] = (int)(d.si.sgn[0] + 1.) | ((int)(d.si.sgn[1] + 1.) << 2) | (d.si.stop[0] << 4) |
-               (d.si.stop[1] << 5);
-}
-
-// Rebuilds the fields a neighbour block and the face Jacobians use; the
-// other fields (own slopes, sgn[2..3]) belong to the owning cell only.
-__device__ __forceinline__ DualInfo lds_get(const DualLds& L, int r) {
-  DualInfo d;
-  d.h = L.h[r]; d.hu = L.hu[r]; d.hv = L.hv[r]; d.g2 = L.g2[r]; d.k = L.k[r]; d.dk = L.dk[r];
-  d.hsx[0] = d.hsy[0] = 0.;
-  d.hsx[1] = L.hsx1[r]; d.hsx[2] = L.hsx2[r]; d.hsy[1] = L.hsy1[r]; d.hsy[2] = L.hsy2[r];
-  const int f = L.flags[r];
-  d.si.sgn[0] = (double)((f & 3) - 1);
-  d.si.sgn[1] = (double)(((f >> 2) & 3) - 1);
-  d.si.sgn[2] = d.si.sgn[3] = 0.;
-  d.si.stop[0] = (f >> 4) & 1;
-  d.si.stop[1] = (f >> 5) & 1;
-#pragma unroll
-  for (int k = 0; k < 6; k++) d.d[k] = 0.;
-  return d;
-}
-
-// dual_hfv of record r (tg_math.h), with its staged 1/h and sqrt(k h g2)
-__device__ __forceinline__ DualHfv lds_dual_hfv(const DualLds& L, int dir, int r, double tiny) {
-  DualHfv o;
-  const double h = L.h[r], hu = L.hu[r], hv = L.hv[r];
-  if (h < tiny) {
-#pragma unroll
-    for (int i = 0; i < 3; i++) o.u[i] = o.f[i] = o.w[i] = 0.;
-    o.fj = zero3(); o.sj = zero3();
-    return o;
+  FaceJac J;
+  if (sl >= 0. || sr <= 0.) {  // upwind: one side's flux
+    const bool own = plus ? sl >= 0. : !(sr <= 0.);
+    J.a00 = 0.;
+    J.a0n = (own && !cvoid) ? 1. : 0.;
+    J.an0 = own ? fn0 : 0.; J.ann = own ? 2 * cv : 0.;
+    J.at0 = own ? ft0 : 0.; J.atn = own ? ftn : 0.; J.att = own ? cv : 0.;
+    if (DPHI) {
+      D.flux0 = own ? cq : nq;
+      D.d0 = D.dt = 0.;
+      D.dn = own ? dFc : dFn;
+    }
+    return J;
   }
-  const double h_inv = L.inv[r], a = L.sq[r];
-  o.u[0] = h; o.u[1] = hu; o.u[2] = hv;
-  if (dir == 0) {
-    double vel = hu * h_inv;
-    o.f[0] = hu; o.f[1] = hu * vel + 0.5 * a * a * h; o.f[2] = hv * vel;
-    o.w[0] = vel - a; o.w[1] = vel; o.w[2] = vel + a;
-    o.fj.a[0][0] = 0.; o.fj.a[0][1] = 1.; o.fj.a[0][2] = 0.;
-    o.fj.a[1][0] = a * a - vel * vel; o.fj.a[1][1] = 2 * vel; o.fj.a[1][2] = 0.;
-    o.fj.a[2][0] = -vel * hv * h_inv; o.fj.a[2][1] = hv * h_inv; o.fj.a[2][2] = vel;
-    o.sj.a[0][0] = -.5 * a * h_inv - vel * h_inv; o.sj.a[0][1] = h_inv; o.sj.a[0][2] = 0.;
-    o.sj.a[1][0] = -vel * h_inv; o.sj.a[1][1] = h_inv; o.sj.a[1][2] = 0.;
-    o.sj.a[2][0] = .5 * a * h_inv - vel * h_inv; o.sj.a[2][1] = h_inv; o.sj.a[2][2] = 0.;
-  } else {
-    double vel = hv * h_inv;
-    o.f[0] = hv; o.f[1] = hu * vel; o.f[2] = hv * vel + 0.5 * a * a * h;
-    o.w[0] = vel - a; o.w[1] = vel; o.w[2] = vel + a;
-    o.fj.a[0][0] = 0.; o.fj.a[0][1] = 0.; o.fj.a[0][2] = 1.;
-    o.fj.a[1][0] = -vel * hu * h_inv; o.fj.a[1][1] = vel; o.fj.a[1][2] = hu * h_inv;
-    o.fj.a[2][0] = a * a - vel * vel; o.fj.a[2][1] = 0.; o.fj.a[2][2] = 2 * vel;
-    o.sj.a[0][0] = -.5 * a * h_inv - vel * h_inv; o.sj.a[0][1] = 0.; o.sj.a[0][2] = h_inv;
-    o.sj.a[1][0] = -vel * h_inv; o.sj.a[1][1] = 0.; o.sj.a[1][2] = h_inv;
-    o.sj.a[2][0] = .5 * a * h_inv - vel * h_inv; o.sj.a[2][1] = 0.; o.sj.a[2][2] = h_inv;
+  // d sl, d sr by the cell (0, n entries; 2 ci - ci = ci)
+  const double hai = .5 * ca * ci;
+  const double e0 = -hai - cvi, e2 = hai - cvi;
+  const bool usel = sl != 0. && (plus ? sl == c0 : sl != n0);
+  const bool user = sr != 0. && (plus ? sr == c2 : sr != n2);
+  const double dsl0 = usel ? (nvoid ? 2 * e0 - -cvi : e0) : 0., dsln = usel ? ci : 0.;
+  const double dsr0 = user ? (nvoid ? 2 * e2 - -cvi : e2) : 0., dsrn = user ? ci : 0.;
+  const double g = 1. / (sr - sl), ss = sl * sr;
+  const double slg = -sl * g, srg = sr * g, jv = -sr * sl * g;
+  {
+    const double vd = nh - ch;
+    const double fx = (sr * cq - sl * nq + ss * vd) * g;
+    const double p = (cq + sl * vd - fx) * g, m = (-nq + sr * vd + fx) * g;
+    J.a00 = p * dsr0 + m * dsl0 + jv;
+    J.a0n = p * dsrn + m * dsln + (cvoid ? 0. : srg);
+    if (DPHI) {
+      D.flux0 = fx;
+      D.d0 = p * dsr + m * dsl;
+    }
   }
-  return o;
-}
-
-// hfv_fwd and dhfv_dk (tg_math.h) of record r, with its staged values
-__device__ __forceinline__ Hfv lds_hfv(const DualLds& L, int dir, int r, double tiny) {
-  Hfv o;
-  const double h = L.h[r], hu = L.hu[r], hv = L.hv[r];
-  if (h < tiny) {
-#pragma unroll
-    for (int i = 0; i < 3; i++) o.u[i] = o.f[i] = o.w[i] = 0.;
-    return o;
+  {
+    const double cf = cq * cv + 0.5 * ca * ca * ch, nf = nq * nv + 0.5 * na * na * nh;
+    const double vd = nq - cq;
+    const double fx = (sr * cf - sl * nf + ss * vd) * g;
+    const double p = (cf + sl * vd - fx) * g, m = (-nf + sr * vd + fx) * g;
+    J.an0 = p * dsr0 + m * dsl0 + srg * fn0;
+    J.ann = p * dsrn + m * dsln + srg * (2 * cv) + jv;
+    if (DPHI) D.dn = p * dsr + m * dsl + srg * dFc + slg * dFn;
   }
-  const double a = L.sq[r];
-  o.u[0] = h; o.u[1] = hu; o.u[2] = hv;
-  if (dir == 0) {
-    const double vel = L.vx[r];
-    o.f[0] = hu; o.f[1] = hu * vel + 0.5 * a * a * h; o.f[2] = hv * vel;
-    o.w[0] = vel - a; o.w[1] = vel; o.w[2] = vel + a;
-  } else {
-    const double vel = L.vy[r];
-    o.f[0] = hv; o.f[1] = hu * vel; o.f[2] = hv * vel + 0.5 * a * a * h;
-    o.w[0] = vel - a; o.w[1] = vel; o.w[2] = vel + a;
+  {
+    const double cf = ct * cv, nf = nt * nv, vd = nt - ct;
+    const double fx = (sr * cf - sl * nf + ss * vd) * g;
+    const double p = (cf + sl * vd - fx) * g, m = (-nf + sr * vd + fx) * g;
+    J.at0 = p * dsr0 + m * dsl0 + srg * ft0;
+    J.atn = p * dsrn + m * dsln + srg * ftn;
+    J.att = srg * cv + jv;
+    if (DPHI) D.dt = p * dsr + m * dsl;
   }
-  return o;
-}
-__device__ __forceinline__ void lds_dhfv_dk(const DualLds& L, int dir, int r, double tiny,
-                                            double dF[3], double dW[3]) {
-  dF[0] = dF[1] = dF[2] = dW[0] = dW[1] = dW[2] = 0.;
-  const double h = L.h[r];
-  if (h < tiny) return;
-  const double g3 = L.g2[r], da = L.da[r];
-  if (dir == 0) dF[1] = 0.5 * h * g3 * h;
-  else dF[2] = 0.5 * h * g3 * h;
-  dW[0] = -da;
-  dW[2] = da;
-}
-
-// face flux and its derivative along d kact/d phi_bed (both sides) between
-// records rl and rr
-__device__ __forceinline__ void face_dk(const AdjArgs& a, int side, const DualLds& L, int rl,
-                                        int rr, double flux[3], double dflux[3]) {
-  Hfv hl = lds_hfv(L, side, rl, a.tiny);
-  Hfv hr = lds_hfv(L, side, rr, a.tiny);
-  riemann(hl, hr, flux);
-  double dFl[3], dWl[3], dFr[3], dWr[3];
-  lds_dhfv_dk(L, side, rl, a.tiny, dFl, dWl);
-  lds_dhfv_dk(L, side, rr, a.tiny, dFr, dWr);
-  const double dkl = L.dk[rl], dkr = L.dk[rr];
-#pragma unroll
-  for (int v = 0; v < 3; v++) {
-    dFl[v] *= dkl; dWl[v] *= dkl; dFr[v] *= dkr; dWr[v] *= dkr;
-  }
-  driemann(hl, hr, dFl, dWl, dFr, dWr, dflux);
-}
-
-// lambda^{s+1}_c . d U^{s+1}_c / d phi_bed at frozen dt (bed-friction
-// gradient; no reference counterpart).  C: the cell's own record; rc, rE,
-// rN, rW, rS: the LDS records of the cell and its neighbours (absent
-// neighbours' slots are passed but not read).  Faces with no neighbour copy
-// the opposite face (outflow), as in the forward step.
-__device__ double dphi_term(const AdjArgs& a, const InstDev& I, const Cell& q,
-                            const DualInfo& C, const DualLds& L, int rc, int rE, int rN, int rW,
-                            int rS, double dt, const double lam[3]) {
-  double fE[3] = {0., 0., 0.}, fN[3] = {0., 0., 0.}, fW[3] = {0., 0., 0.}, fS[3] = {0., 0., 0.};
-  double dE[3] = {0., 0., 0.}, dN[3] = {0., 0., 0.}, dW[3] = {0., 0., 0.}, dS[3] = {0., 0., 0.};
-  if (q.hasE) face_dk(a, 0, L, rc, rE, fE, dE);
-  if (q.hasW) face_dk(a, 0, L, rW, rc, fW, dW);
-  if (q.hasN) face_dk(a, 1, L, rc, rN, fN, dN);
-  if (q.hasS) face_dk(a, 1, L, rS, rc, fS, dS);
-#pragma unroll
-  for (int v = 0; v < 3; v++) {
-    if (!q.hasE) { fE[v] = fW[v]; dE[v] = dW[v]; }
-    if (!q.hasW) { fW[v] = fE[v]; dW[v] = dE[v]; }
-    if (!q.hasN) { fN[v] = fS[v]; dN[v] = dS[v]; }
-    if (!q.hasS) { fS[v] = fN[v]; dS[v] = dN[v]; }
-  }
-  const double dtdx = dt / I.dx, dtdy = dt / I.dy;
-  double out[3];
-#pragma unroll
-  for (int v = 0; v < 3; v++) out[v] = -dtdx * (dE[v] - dW[v]) - dtdy * (dN[v] - dS[v]);
-  if (C.h - dtdx * (fE[0] - fW[0]) - dtdy * (fN[0] - fS[0]) < 0.) out[0] = 0.;
-  if (C.h > a.tiny) {
-    const long long c = q.c;
-    const double tbc = mat_of(I, a.mat, a.mtab, c).tan_bed;
-    const double sec2 = 1. + tbc * tbc;
-    const double vx = L.vx[rc], vy = L.vy[rc];  // hu / h, hv / h (staged)
-    const double g2 = C.g2, dg0 = a.S.dgx[c], dg1 = a.S.dgy[c], k0 = a.S.kx[c], k1 = a.S.ky[c];
-    double ds2x = C.si.sgn[0] * C.h * C.dk * (g2 * C.d[3] + dg1 * C.h) * I.sin_int;
-    double ds3x = C.si.sgn[2] * umax(g2 * C.h + vx * C.hu * k0, 0.0) * sec2;
-    double ds2y = C.si.sgn[1] * C.h * C.dk * (g2 * C.d[0] + dg0 * C.h) * I.sin_int;
-    double ds3y = C.si.sgn[3] * umax(g2 * C.h + vy * C.hv * k1, 0.0) * sec2;
-    out[1] += dt * (-ds2x - ds3x);
-    out[2] += dt * (-ds2y - ds3y);
-  }
-  return lam[0] * out[0] + lam[1] * out[1] + lam[2] * out[2];
+  return J;
 }
 
 // Adjoint pass 1 (one workgroup per mark block, one cell of each of its four
@@ -1000,7 +1047,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_classify(AdjArgs a) {
     int k = atomicAdd(a.tile_count, __popc(W));
 #pragma unroll
     for (int b = 0; b < 4; b++)
-      if ((W >> b) & 1u) a.tile_list[k++] = B.tile[b];
+      if ((W >> b) & 1u) a.tile_list[k++] = tile_ref<TX>(B, b);
   }
   int nshort = 0;
 #pragma unroll
@@ -1024,185 +1071,197 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_classify(AdjArgs a) {
 }
 
 
-// Adjoint pass 2, one listed tile.
-template <int TX>
-__device__ __forceinline__ void adjoint_tile(const AdjArgs& a, int tile, DualLds& L,
-                                             double* sp) {
-  const TileDev t = a.tiles[tile];
+// Adjoint pass 2, one tile.  MAYBE_VOID: the tile is not known to hold
+// anything; a void one is written here as the classifying pass would.
+template <int TX, bool DPHI, bool MAYBE_VOID>
+__device__ __forceinline__ void adjoint_tile(const AdjArgs& a, const TileRef& t,
+                                             DualLds<TX, DPHI>& L) {
   const InstDev I = a.inst[t.inst];
-  const Cell q = cell_of<TX>(t, I);
-  double dphi = 0.;
-  bool zero_out = true;
-  const bool want_dphi = a.dphi_part != nullptr;
-  // the halo is the four side strips: the 5-point stencil reads no corner
   constexpr int TY = BLOCK / TX, RX = TX + 2, RY = TY + 2, NHALO = 2 * TX + 2 * TY;
-  static_assert(RX * RY <= RN && NHALO <= BLOCK, "tile does not fit the LDS records");
-  if (a.active) {
-    const int cnt = __syncthreads_count(q.act);
-    if (threadIdx.x == 0) atomicAdd(a.active, (unsigned long long)cnt);
-  }
-  const int tx = (int)(threadIdx.x % TX), ty = (int)(threadIdx.x / TX);
-  const int rself = (ty + 1) * RX + tx + 1;
-  // phase 1: dual records of the tile (kept in registers) and of the halo
-  DualInfo self;
-  if (q.act) {
-    self = dual_info(a, I, q.i, q.j, want_dphi);
-    lds_put(L, rself, self, a.tiny);
-  }
-  if ((int)threadIdx.x < NHALO) {
-    const int h = (int)threadIdx.x;
-    int rx, ry;
-    if (h < TX) { rx = h + 1; ry = 0; }
+  static_assert(BLOCK + NHALO <= ADJ_THREADS, "one thread per record");
+  int tid = (int)threadIdx.x;
+  asm volatile("" : "+v"(tid));  // indexes rebuilt per tile, not held over the tile loop
+  const double dt = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
+  // phase 1: the halo is the four side strips (the stencil reads no corner)
+  bool busy = false;
+  if (tid < BLOCK + NHALO) {
+    int rx, ry, own = -1;
+    const int h = tid - BLOCK;
+    if (h < 0) { rx = tid % TX + 1; ry = tid / TX + 1; own = tid; }
+    else if (h < TX) { rx = h + 1; ry = 0; }
     else if (h < 2 * TX) { rx = h - TX + 1; ry = RY - 1; }
     else if (h < 2 * TX + TY) { rx = 0; ry = h - 2 * TX + 1; }
     else { rx = RX - 1; ry = h - 2 * TX - TY + 1; }
-    const int gi = t.x0 - 1 + rx, gj = t.y0 - 1 + ry;
-    if (gi >= 0 && gi < I.nx && gj >= 0 && gj < I.ny)
-      lds_put(L, ry * RX + rx, dual_info(a, I, gi, gj, want_dphi), a.tiny);
+    const int i = t.x0 - 1 + rx, j = t.y0 - 1 + ry;
+    if (i >= 0 && i < t.nx && j >= 0 && j < t.ny)
+      busy = dual_record<TX, DPHI>(a, t, I, i, j, dt, L, ry * RX + rx, own) && own >= 0;
   }
-  __syncthreads();
-  if (q.act) {
-    const long long c = q.c, nx = I.nx;
-    const double dt = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
-    const double dtdx = dt / I.dx, dtdy = dt / I.dy;
-    const double hc = self.h;
-    double adj[3] = {0., 0., 0.};
-    // slots: 0 self, 1 E, 2 N, 3 W, 4 S
-    const bool has[5] = {true, q.hasE, q.hasN, q.hasW, q.hasS};
-    const long long nb[5] = {c, c + 1, c + nx, c - 1, c - nx};
-    const int rn[5] = {rself, rself + 1, rself + RX, rself - 1, rself - RX};
-    // Neighbour records are re-read from LDS at each use (not held in
-    // registers across the phases); the empty asm statements keep the
-    // compiler from merging the re-reads into long-lived registers.
-    auto nbr_hfv = [&](int dir, int r) { return lds_dual_hfv(L, dir, r, a.tiny); };
-    if (hc != 0.) {  // a void cell receives nothing (calc_jacobain.C:117-122)
-      // c-side Jacobians of the four faces (dual_riemannflux)
-      M3 JE = zero3(), JN = zero3(), JW = zero3(), JS = zero3();
-      {
-        const DualHfv cx = lds_dual_hfv(L, 0, rself, a.tiny);
-        if (has[1]) JE = dual_riemann_side(cx, nbr_hfv(0, rn[1]), true);
-        if (has[3]) JW = dual_riemann_side(nbr_hfv(0, rn[3]), cx, false);
+  const int p = tid & 1, q = tid >> 1;
+  const bool isx = p;
+  const int gi = t.x0 + q % TX, gj = t.y0 + q / TX;
+  const bool act = gi < t.nx && gj < t.ny;
+  const long long c = t.off + (long long)gj * t.nx + gi;
+  if (MAYBE_VOID) {
+    if (!__syncthreads_or(busy)) {
+      const bool keep = a.mk_out && a.l_bytes && (a.mk_out[t.mw] >> (8 * mark_byte<TX>(t))) & 1u;
+      if (act && isx && !keep) { a.lam_h[c] = 0.; a.lam_hu[c] = 0.; a.lam_hv[c] = 0.; }
+      if (a.short_cells) {
+        const int cnt = __syncthreads_count(act && isx);
+        if (tid == 0) atomicAdd(a.short_cells, (unsigned long long)cnt);
       }
-      {
-        const DualHfv cy = lds_dual_hfv(L, 1, rself, a.tiny);
-        if (has[2]) JN = dual_riemann_side(cy, nbr_hfv(1, rn[2]), true);
-        if (has[4]) JS = dual_riemann_side(nbr_hfv(1, rn[4]), cy, false);
+      if (a.mk_out) {
+        __syncthreads();  // every thread has read the byte
+        mark_store<TX>(a.mk_out, t, true);
       }
-      asm volatile("" ::: "memory");
-
-      // ---- self block (effelement 0): fjc(.,.,0) with boundary copies
-      {
-        M3 J;
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-          for (int j = 0; j < 3; j++) {
-            const double pE = has[1] ? JE.a[i][j] : (has[3] ? JW.a[i][j] : 0.);
-            const double nW = has[3] ? JW.a[i][j] : (has[1] ? JE.a[i][j] : 0.);
-            const double pN = has[2] ? JN.a[i][j] : (has[4] ? JS.a[i][j] : 0.);
-            const double nS = has[4] ? JS.a[i][j] : (has[2] ? JN.a[i][j] : 0.);
-            J.a[i][j] = +dtdx * (pE - nW) + dtdy * (pN - nS);
-          }
-        for (int i = 0; i < 3; i++) J.a[i][i] -= 1.;
-        const DualInfo& C = self;
-        if (C.h > a.tiny) {
-          const double alpha = I.sin_int * C.si.sgn[0] * C.k;
-          const double betta = I.sin_int * C.si.sgn[1] * C.k;
-          const double vx = L.vx[rself], vy = L.vy[rself];  // hu / h, hv / h (staged)
-          const double vx_sq = vx * vx, vy_sq = vy * vy;
-          const double tb = mat_of(I, a.mat, a.mtab, c).tan_bed;
-          const double g0 = a.S.gx[c], g1 = a.S.gy[c], g2 = C.g2;
-          const double dg0 = a.S.dgx[c], dg1 = a.S.dgy[c], k0 = a.S.kx[c], k1 = a.S.ky[c];
-          const double dh0 = C.hsx[0], dh1 = C.hsy[0];
-          J.a[1][0] -= dt * (g0 - alpha * C.h * (2 * dg1 + g2 * dh1) - alpha * g2 * C.d[3]);
-          if (C.si.sgn[2] != 0. && !C.si.stop[0]) {
-            J.a[1][0] -= -dt * C.si.sgn[2] * tb * (g2 - vx_sq * k0);
-            J.a[1][1] -= -dt * C.si.sgn[2] * tb * (2 * vx * k0);
-            J.a[1][2] -= 0.;
-          }
-          J.a[2][0] -= dt * (g1 - betta * C.h * (2 * dg0 + g2 * dh0) - betta * g2 * C.d[0]);
-          if (C.si.sgn[3] != 0. && !C.si.stop[1]) {
-            J.a[2][0] -= -dt * C.si.sgn[3] * tb * (g2 - vy_sq * k1);
-            J.a[2][1] -= 0.;
-            J.a[2][2] -= -dt * C.si.sgn[3] * tb * (2 * vy * k1);
-          }
-        }
-        const double lam[3] = {a.lam_next.h[c], a.lam_next.hu[c], a.lam_next.hv[c]};
-        accum_T(adj, J, lam);
-      }
-      // ---- neighbour blocks in the reference's visiting order S, E, N, W
-      // (neighbor[0..3] with positive_x_side = 1).
-      const int order[4] = {4, 1, 2, 3};
-#pragma unroll
-      for (int o = 0; o < 4; o++) {
-        const int s = order[o];
-        if (!has[s]) continue;
-        const DualInfo N = lds_get(L, rn[s]);
-        const long long n = nb[s];
-        M3 J;
-        if (s == 1) {         // c is the xm neighbour of n
-          const bool bnd = !(q.i + 2 < I.nx);
-          J = flux_block(JE, bnd, JE, true, JE, false, JE, false, dtdx, dtdy);
-          nbr_source(J, N, I.sin_int, dt, N.hsx[1], 0., a.tiny);
-        } else if (s == 3) {  // c is the xp neighbour of n
-          const bool bnd = !(q.i - 2 >= 0);
-          J = flux_block(JW, true, JW, bnd, JW, false, JW, false, dtdx, dtdy);
-          nbr_source(J, N, I.sin_int, dt, N.hsx[2], 0., a.tiny);
-        } else if (s == 2) {  // c is the ym neighbour of n
-          const bool bnd = !(q.j + 2 < I.ny);
-          J = flux_block(JN, false, JN, false, JN, bnd, JN, true, dtdx, dtdy);
-          nbr_source(J, N, I.sin_int, dt, 0., N.hsy[1], a.tiny);
-        } else {              // c is the yp neighbour of n
-          const bool bnd = !(q.j - 2 >= 0);
-          J = flux_block(JS, false, JS, false, JS, true, JS, bnd, dtdx, dtdy);
-          nbr_source(J, N, I.sin_int, dt, 0., N.hsy[2], a.tiny);
-        }
-        const double lam[3] = {a.lam_next.h[n], a.lam_next.hu[n], a.lam_next.hv[n]};
-        accum_T(adj, J, lam);
-      }
+      return;
     }
-    double out[3];
-    for (int j = 0; j < 3; j++) {
-      double v = 0. - adj[j];
-      if (fabs(v) < 1e-16) v = 0.;  // calc_adjoint.C:150-152
-      out[j] = v;
-    }
-    a.lam_h[c] = out[0];
-    a.lam_hu[c] = out[1];
-    a.lam_hv[c] = out[2];
-    zero_out = bitzero3(out[0], out[1], out[2]);
-    if (want_dphi) {
-      const double lam[3] = {a.lam_next.h[c], a.lam_next.hu[c], a.lam_next.hv[c]};
-      asm volatile("" ::: "memory");
-      // every rn[] slot lies inside the LDS tile; records of absent
-      // neighbours are passed but not read (dphi_term checks q.has*).  A
-      // cell with lambda^{s+1} = 0 adds lambda . dU/dphi = 0 (dU/dphi is
-      // finite): not evaluated (the tile's sum may then hold +0.0 where the
-      // full evaluation would give -0.0)
-      if (!(lam[0] == 0. && lam[1] == 0. && lam[2] == 0.))
-        dphi = dphi_term(a, I, q, self, L, rself, rn[1], rn[2], rn[3], rn[4], dt, lam);
-    }
-  }
-  if (want_dphi) {
-    dphi = wave_sum(dphi);
-    if (threadIdx.x % 64 == 0) sp[threadIdx.x / 64] = dphi;
+  } else {
     __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int k = 1; k < BLOCK / 64; k++) dphi += sp[k];
-      a.dphi_part[tile] += dphi;
+  }
+  double dphi = 0.;
+  bool zero_out = true;
+  if (act) {
+    const bool full = L.nz[q];  // a void cell receives nothing (calc_jacobain.C:117-122)
+    const int rc = (q / TX + 1) * RX + q % TX + 1;
+    const double* LN = isx ? L.lam[1] : L.lam[2];  // normal and tangential adjoint
+    const double* LT = isx ? L.lam[2] : L.lam[1];
+    const double lc0 = L.lam[0][rc], lcn = LN[rc], lct = LT[rc];
+    double out[3] = {0., 0., 0.};
+    // a cell with lambda^{s+1} = 0 adds lambda . dU/dphi = 0 to the gradient
+    if (full || (DPHI && !(lc0 == 0. && lcn == 0. && lct == 0.))) {
+      const double dtd = isx ? dt / I.dx : dt / I.dy, dts = isx ? dtd : -dtd;
+      // faces in visiting order: A is S (y) or E (x), B is N or W; the
+      // neighbours beyond them up to the member's edge
+      const int pos = isx ? gi : gj, last = (isx ? t.nx : t.ny) - 1;
+      const int aheadA = isx ? last - pos : pos, aheadB = last - aheadA;
+      const bool hasA = aheadA > 0, hasB = aheadB > 0;
+      const int stepA = isx ? 1 : -RX;
+      // (a missing neighbour: any face, its entries are replaced below)
+      const int rA = hasA ? rc + stepA : rc, rB = hasB ? rc - stepA : rc;
+      FaceDk D;
+      // lambda^{s+1}_c . d U^{s+1}_c / d phi_bed at frozen dt (no reference
+      // counterpart): an outflow face copies the opposite face, so the
+      // pair's difference vanishes; h clamped at 0 does not vary
+      const double pair = hasA && hasB ? dtd : 0.;
+      double mass = 0., d0 = 0.;
+      FaceJac A = face_jac<TX, DPHI>(L, isx, isx, rc, rA, D);
+      if (DPHI) {
+        mass = pair * D.flux0; d0 = pair * D.d0;
+        dphi -= lcn * ((isx ? pair : -pair) * D.dn) + lct * (pair * D.dt);
+      }
+      FaceJac B = face_jac<TX, DPHI>(L, isx, !isx, rc, rB, D);
+      if (DPHI) {
+        mass += pair * D.flux0; d0 += pair * D.d0;
+        dphi -= lcn * ((isx ? -pair : pair) * D.dn) + lct * (pair * D.dt);
+        if (!(L.h[rc] - (mass + swap_pair(mass)) < 0.)) dphi -= lc0 * d0;
+        if (isx) dphi += lcn * L.dsrc[0][q] + lct * L.dsrc[1][q];
+      }
+      if (full) {
+        // an outflow face copies the opposite face (boundary_flux): its
+        // mirrored entries are the opposite's with the signs taken back
+        if (!hasA || !hasB) {
+          auto flip = [](const FaceJac& J) {
+            return FaceJac{-J.a00, J.a0n, J.an0, -J.ann, -J.at0, J.atn, -J.att};
+          };
+          const FaceJac Z = {0., 0., 0., 0., 0., 0., 0.};
+          if (!hasA) A = hasB ? flip(B) : Z;
+          if (!hasB) B = hasA ? flip(A) : Z;
+        }
+        // the neighbours' blocks (calc_jacobian_elem): -dtd J of a plus face
+        // (it is the neighbour's minus face), +dtd J of a minus face; zero
+        // where the neighbour's other side is a domain boundary (both its
+        // sides then carry this face); with the source term on the
+        // tangential row, times the neighbour's lambda
+        const double sA = aheadA > 1 ? -dtd : 0., pA = isx ? sA : -sA;
+        const double sB = aheadB > 1 ? -dtd : 0., pB = isx ? -sB : sB;
+        const double a0 = hasA ? L.lam[0][rA] : 0., an = hasA ? LN[rA] : 0.,
+                     at = hasA ? LT[rA] : 0.;
+        const double b0 = hasB ? L.lam[0][rB] : 0., bn = hasB ? LN[rB] : 0.,
+                     bt = hasB ? LT[rB] : 0.;
+        const double At0 = sA * A.at0 - L.src[isx ? 0 : 3][rA];
+        const double Bt0 = sB * B.at0 - L.src[isx ? 1 : 2][rB];
+        // rows 1 and 2 in order: x faces n, t; y faces t, n
+        const double An0 = an * (pA * A.an0), Ann = an * (sA * A.ann);
+        const double Bn0 = bn * (pB * B.an0), Bnn = bn * (sB * B.ann);
+        const double At0l = at * At0, Atn = at * (pA * A.atn);
+        const double Bt0l = bt * Bt0, Btn = bt * (pB * B.atn);
+        // self block: dtd * (plus face - minus face) of both directions - 1,
+        // minus the sources; the y thread (n = 2, t = 1) forms it
+        auto other = [](double v) { return swap_pair(v); };
+        const double D00 = dtd * (A.a00 + B.a00), D0n = dts * (A.a0n - B.a0n);
+        const double Dn0 = dts * (A.an0 - B.an0), Dnn = dtd * (A.ann + B.ann);
+        const double Dt0 = dtd * (A.at0 + B.at0), Dtn = dts * (A.atn - B.atn);
+        const double Dtt = dtd * (A.att + B.att);
+        double r0 = 0. + lc0 * ((D00 + other(D00)) - 1.);
+        double rt = 0. + lc0 * other(D0n), rn = 0. + lc0 * D0n;
+        r0 += lct * ((other(Dn0) + Dt0) - L.self[0][q] - L.self[1][q]);
+        rt += lct * ((other(Dnn) + Dtt) - 1. - L.self[2][q]);
+        rn += lct * Dtn;
+        r0 += lcn * ((other(Dt0) + Dn0) - L.self[3][q] - L.self[4][q]);
+        rt += lcn * other(Dtn);
+        rn += lcn * ((other(Dtt) + Dnn) - 1. - L.self[5][q]);
+        // the pair hands the sum back and forth: n and t change roles
+        auto pass = [&]() {
+          r0 = swap_pair(r0);
+          const double x = swap_pair(rt);
+          rt = swap_pair(rn);
+          rn = x;
+        };
+        const double A1 = isx ? An0 : At0l, A2 = isx ? At0l : An0;
+        const double A1n = isx ? Ann : Atn, A2n = isx ? Atn : Ann;
+        const double A0 = a0 * (sA * A.a00), A0n = a0 * (pA * A.a0n), Att = at * (sA * A.att);
+        auto addA = [&]() {
+          r0 += A0; rn += A0n; rt += Att;
+          r0 += A1; rn += A1n;
+          r0 += A2; rn += A2n;
+        };
+        const double B1 = isx ? Bn0 : Bt0l, B2 = isx ? Bt0l : Bn0;
+        const double B1n = isx ? Bnn : Btn, B2n = isx ? Btn : Bnn;
+        const double B0 = b0 * (sB * B.a00), B0n = b0 * (pB * B.a0n), Btt = bt * (sB * B.att);
+        auto addB = [&]() {
+          r0 += B0; rn += B0n; rt += Btt;
+          r0 += B1; rn += B1n;
+          r0 += B2; rn += B2n;
+        };
+        addA(); pass(); addA(); pass();  // S, E
+        addB(); pass(); addB();          // N, W
+        // the x thread holds the sum (n = 1, t = 2)
+        out[0] = 0. - r0; out[1] = 0. - rn; out[2] = 0. - rt;
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+          if (fabs(out[k]) < 1e-16) out[k] = 0.;  // calc_adjoint.C:150-152
+      }
+    }
+    if (isx) {
+      a.lam_h[c] = out[0];
+      a.lam_hu[c] = out[1];
+      a.lam_hv[c] = out[2];
+      zero_out = bitzero3(out[0], out[1], out[2]);
     }
   }
-  if (a.mk_out) mark_store<TX>(a.mk_out, t, __syncthreads_and(zero_out));
+  if (a.active) {
+    const int cnt = __syncthreads_count(act && isx);
+    if (tid == 0) atomicAdd(a.active, (unsigned long long)cnt);
+  }
+  const bool all = a.mk_out || DPHI ? __syncthreads_and(zero_out) : false;
+  if (DPHI) {
+    dphi = wave_sum(dphi);
+    if (tid % 64 == 0) L.sp[tid / 64] = dphi;
+    __syncthreads();
+    if (tid == 0) {
+      for (int k = 1; k < ADJ_THREADS / 64; k++) dphi += L.sp[k];
+      unsafeAtomicAdd(a.dphi_part + t.tile, dphi);  // the tile's only writer: nothing waits for it
+    }
+  }
+  if (a.mk_out) mark_store<TX>(a.mk_out, t, all);
 }
 
-
-template <int TX>
-__global__ __launch_bounds__(BLOCK) void k_adjoint(AdjArgs a) {
-  __shared__ DualLds L;
-  __shared__ double sp[BLOCK / 64];
+template <int TX, bool DPHI>
+__global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint(AdjArgs a) {
+  __shared__ DualLds<TX, DPHI> L;
   const int n = *a.tile_count;
   for (int i = (int)blockIdx.x; i < n; i += (int)gridDim.x) {
-    adjoint_tile<TX>(a, a.tile_list[list_band(i, n)], L, sp);
+    adjoint_tile<TX, DPHI, false>(a, a.tile_list[list_band(i, n)], L);
     __syncthreads();  // LDS reused by the next tile
   }
 }
@@ -1235,7 +1294,16 @@ void launch_update(const StepArgs& a, hipStream_t s) {
 void launch_adjoint(const AdjArgs& a, hipStream_t s) {
   launch_zero(a.tile_count, sizeof(int), s);
   TG_LAUNCH_TX(a.shape, k_adjoint_classify, dim3(a.nblocks), s, a);
-  TG_LAUNCH_TX(a.shape, k_adjoint, dim3(a.ntiles < LIST_GRID ? a.ntiles : LIST_GRID), s, a);
+  const dim3 g(a.ntiles < ADJ_GRID ? a.ntiles : ADJ_GRID);
+#define TG_ADJ(TX)                                                                        \
+  if (a.dphi_part) hipLaunchKernelGGL((k_adjoint<TX, true>), g, dim3(ADJ_THREADS), 0, s, a); \
+  else hipLaunchKernelGGL((k_adjoint<TX, false>), g, dim3(ADJ_THREADS), 0, s, a)
+  switch (SHAPE_TX[a.shape]) {
+    case 64: TG_ADJ(64); break;
+    case 32: TG_ADJ(32); break;
+    default: TG_ADJ(16); break;
+  }
+#undef TG_ADJ
 }
 static unsigned grid_for(long long n) {
   const long long b = (n + 255) / 256;

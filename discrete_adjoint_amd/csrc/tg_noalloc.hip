@@ -37,7 +37,7 @@ constexpr size_t OFF_MISC = OFF_RED + align256(sizeof(RedDev));  // dt, time, er
 constexpr size_t OFF_TILES = OFF_MISC + 256;
 constexpr size_t OFF_BLOCKS = OFF_TILES + align256(sizeof(TileDev) * NA_MAX_TILES);
 constexpr size_t OFF_LIST = OFF_BLOCKS + align256(sizeof(BlockDev) * NA_MAX_BLOCKS);
-constexpr size_t OFF_KACT = OFF_LIST + align256(sizeof(int) * NA_MAX_TILES);
+constexpr size_t OFF_KACT = OFF_LIST + align256(sizeof(TileRef) * NA_MAX_TILES);
 constexpr size_t NA_BYTES = OFF_KACT + align256(sizeof(double) * NA_MAX_CELLS);
 
 __device__ __align__(256) unsigned char scratch[NA_BYTES];
@@ -75,7 +75,7 @@ void build_tables(int nx, int ny, int* ntiles, int* nblocks) {
     for (int tx = 0; tx < nx; tx += TX) {
       const int bx = tx / MARK_W, by = ty / MARK_H, mw = by * nsx + bx;
       g_tiles[nt++] = TileDev{0, tx, ty, mw, bx > 0 ? mw - 1 : -1, bx + 1 < nsx ? mw + 1 : -1,
-                              by > 0 ? mw - nsx : -1, by + 1 < nsy ? mw + nsx : -1};
+                              by > 0 ? mw - nsx : -1, by + 1 < nsy ? mw + nsx : -1, nx, ny, 0};
     }
   const int nb = nsx * nsy;
   for (int by = 0; by < nsy; by++)
@@ -188,7 +188,7 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.h_out = d_h_out; a.hu_out = d_hu_out; a.hv_out = d_hv_out;
   a.err = &md->err;
   a.active = nullptr;
-  a.tile_list = (int*)(base + OFF_LIST);
+  a.tile_list = (TileRef*)(base + OFF_LIST);
   a.tile_count = &md->tile_count;
   a.dt_clears_count = 1;
   a.mk_in = nullptr;   // no zero marks: every tile is classified from its cells
