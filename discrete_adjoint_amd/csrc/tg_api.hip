@@ -50,6 +50,7 @@ struct tg_ctx {
   BlockDev* blocks_d[NSHAPE] = {};
   int nb[NSHAPE] = {};
   int sel[3] = {0, 0, 0};
+  bool sel_chosen = false;  // by the configuration, the autotuner or the caller
   int ninst = 0, ntiles = 0;
   long long ncell = 0;
 
@@ -86,9 +87,13 @@ struct tg_ctx {
   bool box_on = false;  // a region is set (it may hold no cell)
   long long box_version = 0;  // changes with every tg_set_maxh_region
   double* box_rec = nullptr;
-  RedDev* red = nullptr;
+  RedDev* red = nullptr;     // 2 * ninst: the FP64 uniform steps alternate
   double* dt_rec = nullptr;  // ninst * max_steps
   double* time_d = nullptr;  // ninst
+  // ninst * (max_steps + 1): each member's time before each recorded step of
+  // the FP64 uniform path; clock_at: the step whose slot is current (-1: none)
+  double* clock_d = nullptr;
+  int clock_at = -1;
   int* err_d = nullptr;
   double* part_mass = nullptr;
   double* part_hmax = nullptr;
@@ -311,6 +316,8 @@ void free_fields(tg_ctx* ctx) {
   dfree(ctx->red);
   dfree(ctx->time_d);
   dfree(ctx->dt_rec);
+  dfree(ctx->clock_d);
+  ctx->clock_at = -1;
   for (auto& p : ctx->ckpt) dfree(p);
   for (auto& p : ctx->seg) dfree(p);
   dfree(ctx->traj_block);
@@ -382,12 +389,23 @@ Statics32 statics32(tg_ctx* ctx) {
                    at<float>(b, 6, n)};
 }
 
+// Every pass of a mesh launches its tiles the same way, whatever variants
+// the passes use: directly when the largest tile table is small.
+int tile_launch(const tg_ctx* ctx, int v) {
+  return ctx->ntiles > TILE_LAUNCH_MAX ? 0 : SHAPE_XCD[v] ? 2 : 1;
+}
+void set_by_tile(const tg_ctx* ctx, int v, StepArgs& a) { a.by_tile = tile_launch(ctx, v); }
+void set_by_tile(const tg_ctx* ctx, int v, AdjArgs& a) { a.by_tile = tile_launch(ctx, v); }
+template <class A>
+void set_by_tile(const tg_ctx*, int, A&) {}
+
 // points a kernel's arguments at the tile table of its selected variant
 template <class A>
 void use_tiles(const tg_ctx* ctx, int kernel, A& a) {
   a.mat = ctx->mat_d;
   a.mtab = ctx->mtab_d;
   const int v = ctx->sel[kernel];
+  set_by_tile(ctx, v, a);
   a.tiles = ctx->tiles_d[v];
   a.ntiles = ctx->nt[v];
   a.blocks = ctx->blocks_d[v];
@@ -569,6 +587,7 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
                   at<double>(ctx->statics, 4, n), at<double>(ctx->statics, 5, n),
                   at<double>(ctx->statics, 6, n)};
     a.kact = (double*)ctx->kact; a.red = ctx->red; a.dt_rec = ctx->dt_rec; a.time = ctx->time_d;
+    a.clock = ctx->clock_d;
     a.max_steps = ctx->cfg.max_steps; a.step = s; a.ft = frict_tiny(ctx, s);
     a.tiny = ctx->cfg.tiny; a.gamma = ctx->cfg.gamma;
     a.cfl_inner = ctx->cfg.cfl_inner; a.cfl_outer = ctx->cfg.cfl_outer;
@@ -595,6 +614,9 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
       inst_mark(ctx, 1, false);
       return;
     }
+    a.fold = compute_dt;
+    a.red = ctx->red + (s & 1) * ctx->ninst;
+    a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst;
     use_tiles(ctx, 0, a);
     a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[0]] == ctx->mk_tx[0];
     a.active = inst_counter(ctx, 0, true);
@@ -602,10 +624,6 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
     inst_mark(ctx, 0, true);
     launch_coef(a, compute_dt, ctx->stream);
     inst_mark(ctx, 0, false);
-    if (compute_dt) {
-      a.dt_clears_count = 1;
-      launch_dt(a, ctx->ninst, ctx->stream);
-    }
     use_tiles(ctx, 1, a);
     a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[1]] == ctx->mk_tx[0];
     a.active = inst_counter(ctx, 1, true);
@@ -890,6 +908,12 @@ int stored_steps(const tg_ctx* ctx, int nsteps) {
   return (int)(m < nsteps ? (m < 0 ? 0 : m) : nsteps);
 }
 
+// The reduction cells cleared and every member's clock set for step s.
+void start_clock(tg_ctx* ctx, int s) {
+  launch_reset_red(ctx->red, ctx->ninst, ctx->time_d, ctx->clock_d + s,
+                   (long long)ctx->cfg.max_steps + 1, ctx->stream);
+}
+
 int forward_loop(tg_ctx* ctx, const tg_params* prm, int nsteps, const double* dt_seq,
                  tg_stats* stats, int nstats) {
   if (!ctx->have_mesh || !ctx->have_state) return set_err(ctx, TG_ERR_STATE, "mesh/state not set");
@@ -916,7 +940,7 @@ int forward_loop(tg_ctx* ctx, const tg_params* prm, int nsteps, const double* dt
   void* A[3] = {ctx->U[0], ctx->U[1], ctx->U[2]};
   void* B[3] = {ctx->Ut[0], ctx->Ut[1], ctx->Ut[2]};
   auto body = [&]() -> void** {
-    launch_reset_red(ctx->red, ctx->ninst, ctx->stream);
+    start_clock(ctx, 0);
     zero_box_record(ctx);
     void** cur = A;
     void* slot[3];
@@ -970,6 +994,7 @@ int forward_loop(tg_ctx* ctx, const tg_params* prm, int nsteps, const double* dt
   HIPCHK(ctx, hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
   ctx->fwd_ms = ms;
   ctx->rec_steps = ctx->run_steps = nsteps;
+  ctx->clock_at = dt_seq ? -1 : nsteps;
   ctx->traj_s0 = s0;
   if (dt_seq) {  // time advances by the prescribed sequence
     std::vector<double> t(ctx->ninst);
@@ -1452,6 +1477,13 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
   for (int v = 0; v < NSHAPE; v++) {
     ctx->nb[v] = (int)ctx->blocks_h[v].size();
   }
+  // Nobody chose: on a large mesh the FP64 forward passes take the square tiles
+  // (a fifth fewer records in the halo; 64 members, 5.8 M cells: update 20
+  // against 26 us).  The reverse step keeps the plain table, whose order the
+  // gradient's partial sums have, and so do small meshes, where a workgroup per
+  // tile runs and the time is one tile's.
+  if (!ctx->sel_chosen && ctx->mode == TG_FP64 && !leaves)
+    ctx->sel[0] = ctx->sel[1] = ctx->ntiles > TILE_LAUNCH_MAX ? LARGE_VARIANT : DEFAULT_VARIANT;
   const long long n = ctx->ncell;
   const size_t fb = (size_t)ctx->es * n;
   auto align256 = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -1503,9 +1535,12 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
   for (int b = 0; b < nm; b++) any_mat |= meshes[b].mat != nullptr;
   if (!rc && any_mat) rc = dalloc(ctx, (void**)&ctx->mat_d, (size_t)n);
   if (!rc && any_mat) rc = dalloc(ctx, (void**)&ctx->mtab_d, sizeof(MatDev) * MAX_MAT * nm);
-  if (!rc) rc = dalloc(ctx, (void**)&ctx->red, sizeof(RedDev) * nm);
+  if (!rc) rc = dalloc(ctx, (void**)&ctx->red, sizeof(RedDev) * 2 * nm);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->time_d, sizeof(double) * nm);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->dt_rec, sizeof(double) * nm * ctx->cfg.max_steps);
+  if (!rc)
+    rc = dalloc(ctx, (void**)&ctx->clock_d,
+                sizeof(double) * nm * ((size_t)ctx->cfg.max_steps + 1));
   if (leaves) {
     if (!rc) rc = dalloc(ctx, (void**)&ctx->leaf_nbr, sizeof(int) * 8 * (size_t)n);
     if (!rc) rc = dalloc(ctx, (void**)&ctx->leaf_meta, sizeof(uint32_t) * (size_t)n);
@@ -1608,6 +1643,7 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
 }
 
 int reset_time(tg_ctx* ctx) {
+  ctx->clock_at = -1;
   std::vector<double> z(ctx->ninst, 0.);
   HIPCHK(ctx, hipMemcpyAsync(ctx->time_d, z.data(), sizeof(double) * ctx->ninst,
                              hipMemcpyHostToDevice, ctx->stream));
@@ -1873,6 +1909,7 @@ int tg_create(const tg_config* cfg, tg_ctx** out) {
       return TG_ERR_UNSUPPORTED;
     }
     ctx->sel[0] = ctx->sel[1] = ctx->sel[2] = v;
+    ctx->sel_chosen = true;
   } else {
     ctx->sel[0] = ctx->sel[1] = ctx->sel[2] = DEFAULT_VARIANT;
   }
@@ -1973,6 +2010,7 @@ int tg_set_clock(tg_ctx* ctx, int step0, double time) {
   if (!ctx || step0 < 0 || !(time >= 0) || !std::isfinite(time)) return TG_ERR_ARG;
   if (!ctx->have_state) return set_err(ctx, TG_ERR_STATE, "no state");
   ctx->step0 = step0;
+  ctx->clock_at = -1;
   std::vector<double> t(ctx->ninst, time);
   HIPCHK(ctx, hipMemcpyAsync(ctx->time_d, t.data(), sizeof(double) * ctx->ninst,
                              hipMemcpyHostToDevice, ctx->stream));
@@ -2027,17 +2065,16 @@ int tg_forward_step(tg_ctx* ctx, const tg_params* prm, tg_stats* stats) {
   if (ctx->rec_steps >= ctx->cfg.max_steps) return set_err(ctx, TG_ERR_ARG, "dt record full");
   int rc = upload_params(ctx, prm);
   if (rc) return rc;
-  if (ctx->rec_steps == 0) {
-    launch_reset_red(ctx->red, ctx->ninst, ctx->stream);
-    zero_box_record(ctx);
-  }
+  if (ctx->rec_steps == 0) zero_box_record(ctx);
+  if (ctx->rec_steps == 0 || ctx->clock_at != ctx->rec_steps) start_clock(ctx, ctx->rec_steps);
+  ctx->clock_at = -1;  // until this step has been taken
   enqueue_step(ctx, ctx->U, ctx->Ut, ctx->rec_steps, true);
   enqueue_box_max(ctx, ctx->Ut, ctx->rec_steps);
   for (int c = 0; c < 3; c++) std::swap(ctx->U[c], ctx->Ut[c]);
   HIPCHK(ctx, hipGetLastError());
   rc = check_err(ctx);
   if (rc) return rc;
-  ctx->rec_steps++;
+  ctx->clock_at = ++ctx->rec_steps;
   ctx->run_steps = 0;  // single steps keep no checkpoints
   return fill_stats(ctx, stats, 1);
 }
@@ -2359,6 +2396,7 @@ int time_kernel_variant(tg_ctx* ctx, int which, int v, int reps, double* avg_ms)
       } else if (w == 0) {
         launch_coef(a, false, ctx->stream);
       } else {
+        if (!a.by_tile) launch_zero(ctx->act_count, sizeof(int), ctx->stream);
         launch_update(a, ctx->stream);
       }
       inst_mark(ctx, w, false);
@@ -2435,6 +2473,7 @@ int tg_autotune(tg_ctx* ctx, const tg_params* prm, int reps, int* variant_out, d
       if (ms < best) { best = ms; bv = v; }
     }
     ctx->sel[w] = bv;
+    ctx->sel_chosen = true;
     if (variant_out) variant_out[w] = bv;
   }
   return TG_OK;
@@ -2465,6 +2504,7 @@ int tg_set_tile_selection(tg_ctx* ctx, const int* variant) {
   for (int k = 0; k < 3; k++)
     if (variant[k] < 0 || variant[k] >= NSHAPE) return TG_ERR_ARG;
   for (int k = 0; k < 3; k++) ctx->sel[k] = variant[k];
+  ctx->sel_chosen = true;
   return TG_OK;
 }
 

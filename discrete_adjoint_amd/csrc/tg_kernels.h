@@ -83,7 +83,7 @@ struct BlockDev {
 // Per-instance CFL reduction cells: bit patterns of non-negative doubles
 // (IEEE order of non-negative doubles equals unsigned-integer order, so
 // integer atomic min/max is an exact FP64 min/max).
-struct RedDev {
+struct alignas(128) RedDev {  // a cache line each: members' atomics do not share one
   unsigned long long min_ev;  // min over wet cells of min(dx,dy)/evalue
   unsigned long long hmax;    // max over wet cells of h
 };
@@ -98,7 +98,7 @@ constexpr int NSHAPE = 4;
 constexpr int SHAPE_TX[NSHAPE] = {64, 64, 32, 16};
 constexpr bool SHAPE_XCD[NSHAPE] = {false, true, true, true};
 constexpr int NXCD = 8;
-constexpr int DEFAULT_VARIANT = 0;
+constexpr int DEFAULT_VARIANT = 0, LARGE_VARIANT = 3;
 
 // Zero marks.  A state (h, hu, hv) or adjoint buffer can carry one 32-bit
 // word per MARK_W x MARK_H block of a member's cells.  Every tile shape cuts
@@ -123,6 +123,15 @@ static_assert(MARK_W % 64 == 0 && MARK_H % (BLOCK / 16) == 0 && MARK_W * MARK_H 
 __device__ __forceinline__ int list_band(int p, int n) {
   const int q = n / NXCD, r = n % NXCD, x = p % NXCD;
   return x * q + (x < r ? x : r) + p / NXCD;
+}
+// The entry of a banded table (SHAPE_XCD; n entries) that holds the tile at
+// position p of the mesh's row-major order: a launch of a workgroup per tile
+// takes the tiles in that order, so that the few tiles of a pile, which lie
+// in one band, spread over every XCD instead of queueing on one.
+__device__ __forceinline__ int unbanded(int p, int n) {
+  const int q = n / NXCD, r = n % NXCD, long_runs = r * (q + 1);
+  if (p < long_runs) return (p % (q + 1)) * NXCD + p / (q + 1);
+  return ((p - long_runs) % q) * NXCD + r + (p - long_runs) / q;
 }
 // the byte of its block's word that a tile of width TX owns
 template <int TX, class T>
@@ -156,9 +165,12 @@ struct StepArgs {
   Fields U;
   Statics S;
   double* kact;          // [n] forward kact of U
-  RedDev* red;           // [ninst]
+  RedDev* red;           // [ninst] of this step
+  RedDev* red_next;      // [ninst] of the next step (fold)
   double* dt_rec;        // [ninst * max_steps]
-  double* time;          // [ninst]
+  double* time;          // [ninst] after the last step taken
+  double* clock;         // [ninst * (max_steps + 1)]: before each step (fold)
+  int fold;              // 1: the update's passes make dt (step_dt)
   int max_steps;
   int step;              // step index s (U = U^s)
   double ft;             // frict_tiny of step s
@@ -175,8 +187,6 @@ struct StepArgs {
   // by the classifying pass, walked by the update) and its length
   TileRef* tile_list;
   int* tile_count;
-  // 1: k_dt clears tile_count (the update pass then launches no fill)
-  int dt_clears_count;
   // zero marks of U and of the output state (both null: no marks); a tile
   // the marks show to need nothing is skipped by the coefficient and the
   // classifying pass
@@ -184,6 +194,9 @@ struct StepArgs {
   uint32_t* mk_out;
   // null, or a counter the launch adds the cells it writes on a short path to
   unsigned long long* short_cells;
+  // 0: block passes and a tile list; else a workgroup per tile in every
+  // pass, of a table in row-major order (1) or banded by XCD (2)
+  int by_tile;
   // per-cell material index and the material table (mat null: one material
   // per member, the InstDev fields)
   const uint8_t* mat;
@@ -222,6 +235,7 @@ struct AdjArgs {
   const uint32_t* mk_lnext;
   uint32_t* mk_out;
   unsigned long long* short_cells;
+  int by_tile;            // as in StepArgs
   const uint8_t* mat;     // as in StepArgs
   const MatDev* mtab;
   // as StepArgs::zbytes, for the marks of U^s (u_bytes) and of the adjoint
@@ -321,6 +335,13 @@ constexpr int THIN_GRID = 1024;
 // the listed tiles spread over every CU (1024, 2048, 4096 and 8192 measured
 // on the 256-member ensemble: 4096 about 1 % ahead)
 constexpr int LIST_GRID = 4096;
+// Up to this many tiles each FP64 pass launches a workgroup per tile: two
+// launches per forward and one per reverse step instead of four and three
+// (512 x 512 cells, 1024 tiles: 14.4 us of kernels per forward step against
+// 34, 13 against 40 per reverse step).  Beyond it the workgroups of empty
+// tiles, held to three a CU by their LDS, queue: the block passes leave a
+// block after a few words and only listed tiles take that LDS.
+constexpr int TILE_LAUNCH_MAX = 1024;
 // workgroups of the FP64 adjoint's list walk, and its waves per SIMD
 constexpr int ADJ_GRID = 2048;
 constexpr int ADJ_WAVES = 3;
@@ -411,7 +432,10 @@ void launch_coef(const StepArgs& a, bool reduce, hipStream_t s);
 void launch_dt(const StepArgs& a, int ninst, hipStream_t s);
 void launch_update(const StepArgs& a, hipStream_t s);
 void launch_adjoint(const AdjArgs& a, hipStream_t s);
-void launch_reset_red(RedDev* red, int ninst, hipStream_t s);
+// clears both sets of reduction cells (red [2 * ninst]); clock (or null):
+// clock[b * stride] = time[b]
+void launch_reset_red(RedDev* red, int ninst, const double* time, double* clock, long long stride,
+                      hipStream_t s);
 // rec[member * max_steps + step] = max(itself, largest h > 0 over the listed
 // box cells); rec holds FP64 values >= +0.0
 template <class S>

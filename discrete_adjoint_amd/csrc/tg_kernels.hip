@@ -104,8 +104,9 @@ __device__ __forceinline__ bool coef_skip(const uint32_t* mk, int mw) {
 // and side neighbour has h < tiny, so the fluxes are zero and there are no
 // sources, and U^{s+1} = U^s - dtdx*(0 - 0) - dtdy*(0 - 0) = +0.0 for a
 // finite dt -- and the block of the output already holds +0.0.
+template <class Blk>
 __device__ __forceinline__ bool update_skip(const uint32_t* in, const uint32_t* out,
-                                            const BlockDev& B, double dt) {
+                                            const Blk& B, double dt) {
   return in[B.mw] == MARK_FULL && out[B.mw] == MARK_FULL &&
          (B.mwW < 0 || in[B.mwW] == MARK_FULL) && (B.mwE < 0 || in[B.mwE] == MARK_FULL) &&
          (B.mwS < 0 || in[B.mwS] == MARK_FULL) && (B.mwN < 0 || in[B.mwN] == MARK_FULL) &&
@@ -152,24 +153,95 @@ __device__ __forceinline__ void block_cells(const BlockDev& B, Cell q[4]) {
 
 // Limited slope from its two one-sided differences dp = (u+ - u)/dx and
 // dm = (u - u-)/dx (Element::get_slopes, element2.C:886-897; same operands
-// as slope_fwd).
-__device__ __forceinline__ double slope_from(double dp, double dm, double dx, double gamma,
-                                             double tiny) {
-  double dc = (dp * dx + dm * dx) / (dx + dx);
+// as slope_fwd); inv_s = 1 / (dx + dx).
+__device__ __forceinline__ double slope_from(double dp, double dm, double dx, double inv_s,
+                                             double gamma, double tiny) {
+  const double dc = div_r(dp * dx + dm * dx, dx + dx, inv_s);
   return .5 * (c_sgn(dp, tiny) + c_sgn(dm, tiny)) *
          dmin3(gamma * dabs(dp), gamma * dabs(dm), dabs(dc));
 }
+__device__ __forceinline__ double slope3(double up, double uc, double um, double dx, double inv,
+                                         double inv_s, double gamma, double tiny) {
+  return slope_from(div_r(up - uc, dx, inv), div_r(uc - um, dx, inv), dx, inv_s, gamma, tiny);
+}
 
+// Coefficients of one cell above tiny: kact from its forward slopes
+// (getcoef.f), written, and its terms of the CFL reduction
+// (get_coef_and_eigen.C:29-180).  Every load is issued before the first use.
+__device__ __forceinline__ void coef_cell(const StepArgs& a, const InstDev& I, int i, int j,
+                                          double h, int reduce, double& minev, double& hmax) {
+  const long long c = I.off + (long long)j * I.nx + i;
+  // cells on the domain boundary have zero slopes: with themselves as
+  // neighbours every difference is 0
+  const bool inner = i + 1 < I.nx && i > 0 && j + 1 < I.ny && j > 0;
+  const long long ox = inner ? 1 : 0, oy = inner ? I.nx : 0;
+  const double hu = a.U.hu[c], hv = a.U.hv[c], g3 = a.S.gz[c];
+  const double hE = a.U.h[c + ox], hW = a.U.h[c - ox], hN = a.U.h[c + oy], hS = a.U.h[c - oy];
+  const double uE = a.U.hu[c + ox], uW = a.U.hu[c - ox];
+  const double vN = a.U.hv[c + oy], vS = a.U.hv[c - oy];
+  const double kroot = mat_of(I, a.mat, a.mtab, c).kroot;
+  const double hx = slope3(hE, h, hW, I.dx, I.inv_dx, I.inv_sx, a.gamma, a.tiny);
+  const double hux = slope3(uE, hu, uW, I.dx, I.inv_dx, I.inv_sx, a.gamma, a.tiny);
+  const double hy = slope3(hN, h, hS, I.dy, I.inv_dy, I.inv_sy, a.gamma, a.tiny);
+  const double hvy = slope3(vN, hv, vS, I.dy, I.inv_dy, I.inv_sy, a.gamma, a.tiny);
+  // getcoef and eigen (tg_math.h) for h > tiny
+  const double inv = 1. / h, hh = h * h, ihh = 1. / hh;
+  const double vx = div_r(hu, h, inv), vy = div_r(hv, h, inv);
+  const double vel = div_r(hux, h, inv) - div_r(hu * hx, hh, ihh) + div_r(hvy, h, inv) -
+                     div_r(hv * hy, hh, ihh);
+  double k = I.kc1 * (1. - f_sgn(vel, a.tiny) * kroot) - 1.;
+  if (fabs(vx) < a.tiny && fabs(vy) < a.tiny) k = 1.;
+  if (k < 0.) k = 0.;
+  k = k * I.eps;
+  a.kact[c] = k;
+  if (reduce) {
+    const double w = sqrt(k * g3 * h);
+    const double ex = fabs(vx) + w, ey = fabs(vy) + w;
+    const double ev = (ex > ey) ? ex : ey;
+    if (ev > 1000000000.) atomicOr(a.err, 2);
+    const double mdx = (I.dx > I.dy) ? I.dy : I.dx;
+    const double m = mdx / ev;
+    minev = (m < minev) ? m : minev;
+    hmax = (h > hmax) ? h : hmax;
+  }
+}
 
-// Coefficient pass, one workgroup per mark block (one cell of each of its
-// four tiles per thread): forward slopes -> kact (getcoef.f) and the
-// per-instance CFL min / hmax reduction (get_coef_and_eigen.C:29-180).
+// The workgroup's CFL terms into the member's reduction cells (every thread
+// calls it; any: some thread has one).
+__device__ __forceinline__ void coef_reduce(RedDev* red, double minev, double hmax, bool any) {
+  if (!__syncthreads_or(any)) return;
+  __shared__ double smin[BLOCK / 64], smax[BLOCK / 64];
+  minev = wave_min(minev);
+  hmax = wave_max(hmax);
+  const int w = threadIdx.x / 64, l = threadIdx.x % 64;
+  if (l == 0) { smin[w] = minev; smax[w] = hmax; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < BLOCK / 64; k++) {
+      minev = (smin[k] < minev) ? smin[k] : minev;
+      hmax = (smax[k] > hmax) ? smax[k] : hmax;
+    }
+    if (minev < HUGE_VAL) atomicMin(&red->min_ev, dbits(minev));
+    if (hmax > 0.) atomicMax(&red->hmax, dbits(hmax));
+  }
+}
+
+// Coefficient pass on large meshes, one workgroup per mark block: forward
+// slopes -> kact (getcoef.f) and the per-instance CFL min / hmax reduction
+// (get_coef_and_eigen.C:29-180).  The block's wet cells are listed in LDS and
+// worked off 256 at a time, so a block that a front crosses takes as many
+// rounds as it has wet cells, not one for each of its four tiles (64 members,
+// 5.8 M cells: 15.5 us, a round per tile 23 us).
 template <int TX>
 __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.tile_count = 0;  // the update's list starts empty
   // (the block table is indexed by mark word)
   if (a.mk_in && coef_skip(a.mk_in, (int)blockIdx.x)) return;
   const BlockDev B = a.blocks[blockIdx.x];
-  const InstDev I = a.inst[B.inst];
+  __shared__ int s_n;
+  __shared__ unsigned short s_cell[4 * BLOCK];
+  __shared__ double s_h[4 * BLOCK];
+  if (threadIdx.x == 0) s_n = 0;
   Cell q[4];
   block_cells<TX>(B, q);
   // a tile the marks show to hold +0.0 has h < tiny everywhere: nothing to
@@ -181,39 +253,33 @@ __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
   double h[4];
 #pragma unroll
   for (int b = 0; b < 4; b++) h[b] = q[b].act ? a.U.h[q[b].c] : 0.;
-  double minev = HUGE_VAL, hmax = 0.;
+  const InstDev I = a.inst[B.inst];
+  __syncthreads();  // s_n set
   int nwet = 0, nshort = 0;
+  const int lane = threadIdx.x % 64;
 #pragma unroll
   for (int b = 0; b < 4; b++) {
+    const bool wet = q[b].act && h[b] > a.tiny;
+    const unsigned long long m = __ballot(wet);
+    if (m) {
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&s_n, __popcll(m));
+      base = __shfl(base, 0, 64);
+      if (wet) {
+        const int k = base + __popcll(m & ((1ull << lane) - 1ull));
+        s_cell[k] = (unsigned short)((q[b].j - B.y0) * MARK_W + q[b].i - B.x0);
+        s_h[k] = h[b];
+      }
+    }
     if (!q[b].act) continue;
-    const long long c = q[b].c, nx = I.nx;
-    if (h[b] > a.tiny) {
+    if (wet) {
       nwet++;
-      const double hc = h[b], hu = a.U.hu[c], hv = a.U.hv[c];
-      double hx = 0., hux = 0., hy = 0., hvy = 0.;
-      if (q[b].hasE && q[b].hasW && q[b].hasN && q[b].hasS) {  // boundary cells: zero slopes
-        hx = slope_fwd(a.U.h[c + 1], hc, a.U.h[c - 1], I.dx, a.gamma, a.tiny);
-        hux = slope_fwd(a.U.hu[c + 1], hu, a.U.hu[c - 1], I.dx, a.gamma, a.tiny);
-        hy = slope_fwd(a.U.h[c + nx], hc, a.U.h[c - nx], I.dy, a.gamma, a.tiny);
-        hvy = slope_fwd(a.U.hv[c + nx], hv, a.U.hv[c - nx], I.dy, a.gamma, a.tiny);
-      }
-      const double kroot = mat_of(I, a.mat, a.mtab, c).kroot;
-      const double k = getcoef(hc, hu, hv, hx, hux, hy, hvy, I.kc1, kroot, I.eps, a.tiny);
-      if (reduce) {
-        double ev = eigen(hc, hu, hv, k, a.S.gz[c], a.tiny);
-        if (ev > 1000000000.) atomicOr(a.err, 2);
-        double mdx = (I.dx > I.dy) ? I.dy : I.dx;
-        const double m = mdx / ev;
-        minev = (m < minev) ? m : minev;
-        hmax = (hc > hmax) ? hc : hmax;
-      }
-      a.kact[c] = k;
     } else {
       nshort++;
       // kact is read only where h >= tiny (the physical flux is zero below
       // tiny, update_states uses kact only above it): at or below tiny the
       // value is epsilon, and below tiny it is not written
-      if (!(h[b] < a.tiny)) a.kact[c] = I.eps;
+      if (!(h[b] < a.tiny)) a.kact[q[b].c] = I.eps;
     }
   }
   if (a.active) {
@@ -224,29 +290,58 @@ __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
     const int cnt = (int)wave_sum((double)nshort);
     if (threadIdx.x % 64 == 0 && cnt) atomicAdd(a.short_cells, (unsigned long long)cnt);
   }
-  if (reduce && __syncthreads_or(nwet > 0)) {
-    __shared__ double smin[BLOCK / 64], smax[BLOCK / 64];
-    minev = wave_min(minev);
-    hmax = wave_max(hmax);
-    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-    if (l == 0) { smin[w] = minev; smax[w] = hmax; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int k = 1; k < BLOCK / 64; k++) {
-        minev = (smin[k] < minev) ? smin[k] : minev;
-        hmax = (smax[k] > hmax) ? smax[k] : hmax;
-      }
-      if (minev < HUGE_VAL) atomicMin(&a.red[B.inst].min_ev, dbits(minev));
-      if (hmax > 0.) atomicMax(&a.red[B.inst].hmax, dbits(hmax));
-    }
-  }
+  __syncthreads();  // the list is complete
+  const int n = s_n;
+  double minev = HUGE_VAL, hmax = 0.;
+  for (int k = (int)threadIdx.x; k < n; k += BLOCK)
+    coef_cell(a, I, B.x0 + s_cell[k] % MARK_W, B.y0 + s_cell[k] / MARK_W, s_h[k], reduce, minev,
+              hmax);
+  if (reduce) coef_reduce(&a.red[B.inst], minev, hmax, (int)threadIdx.x < n);
 }
 
-__global__ void k_reset_red(RedDev* red, int ninst) {
+// the tile of a workgroup of the passes over every tile
+template <class A>
+__device__ __forceinline__ int tile_of(const A& a) {
+  const int p = (int)blockIdx.x;
+  return a.by_tile == 2 ? unbanded(p, a.ntiles) : p;
+}
+
+// Coefficient pass on small meshes, one workgroup per tile (128 x 128 cells:
+// 5 us; a workgroup per mark block, four tiles in turn, 12 us).
+template <int TX>
+__global__ __launch_bounds__(BLOCK) void k_coef_tile(StepArgs a, int reduce) {
+  const TileDev t = a.tiles[tile_of(a)];
+  const uint32_t z = a.mk_in ? a.mk_in[t.mw] : 0u;
+  if (z == MARK_FULL || (a.zbytes && ((z >> (8 * mark_byte<TX>(t))) & 1u))) return;
+  const InstDev I = a.inst[t.inst];
+  const int i = t.x0 + (int)(threadIdx.x % TX), j = t.y0 + (int)(threadIdx.x / TX);
+  const bool act = i < t.nx && j < t.ny;
+  const long long c = t.off + (long long)j * t.nx + i;
+  const double h = act ? a.U.h[c] : 0.;
+  const bool wet = act && h > a.tiny;
+  double minev = HUGE_VAL, hmax = 0.;
+  if (wet) coef_cell(a, I, i, j, h, reduce, minev, hmax);
+  else if (act && !(h < a.tiny)) a.kact[c] = I.eps;  // (as in k_coef)
+  if (a.active) {
+    const int cnt = __syncthreads_count(wet);
+    if (threadIdx.x == 0 && cnt) atomicAdd(a.active, (unsigned long long)cnt);
+  }
+  if (a.short_cells) {
+    const int cnt = __syncthreads_count(act && !wet);
+    if (threadIdx.x == 0 && cnt) atomicAdd(a.short_cells, (unsigned long long)cnt);
+  }
+  if (reduce) coef_reduce(&a.red[t.inst], minev, hmax, wet);
+}
+
+// Both sets of reduction cells, and each member's clock slot of the step about
+// to be taken.
+__global__ void k_reset_red(RedDev* red, int ninst, const double* time, double* clock,
+                            long long stride) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b < ninst) {
-    red[b].min_ev = dbits(10000000.);  // get_coef_and_eigen.C:35
-    red[b].hmax = dbits(0.);
+    red[b].min_ev = red[ninst + b].min_ev = dbits(10000000.);  // get_coef_and_eigen.C:35
+    red[b].hmax = red[ninst + b].hmax = dbits(0.);
+    if (clock) clock[b * stride] = time[b];
   }
 }
 
@@ -309,30 +404,54 @@ __global__ void k_member_fill(const uint32_t* __restrict__ src, uint32_t* __rest
     for (long long i = t0; i < nmw; i += stride) mk[mw0 + i] = 0u;
 }
 
-__global__ void k_dt(StepArgs a, int ninst) {
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b == 0 && a.dt_clears_count) *a.tile_count = 0;  // the update's list starts empty
-  if (b >= ninst) return;
-  const InstDev I = a.inst[b];
-  double min_ev = bitsd(a.red[b].min_ev), hmax = bitsd(a.red[b].hmax);
-  double dt0 = a.cfl_inner * min_ev;
-  double dt1 = -0.9 * sqrt(hmax * I.eps * I.gscale / 9.8);
-  double m = (dt0 > -dt1) ? -dt1 : dt0;
+// dt = 0.5 * min(0.5 * min(dx / ev), 0.9 * sqrt(hmax eps Gs / 9.8)) clamped as
+// TimeProps::incrtime does (properties.h:397-410)
+__device__ __forceinline__ double cfl_dt(const StepArgs& a, const InstDev& I, const RedDev& R,
+                                         double time) {
+  const double min_ev = bitsd(R.min_ev), hmax = bitsd(R.hmax);
+  const double dt0 = a.cfl_inner * min_ev;
+  const double dt1 = -0.9 * sqrt(hmax * I.eps * I.gscale / 9.8);
+  const double m = (dt0 > -dt1) ? -dt1 : dt0;
   double dt = a.cfl_outer * m;
   if (dt == 0.0) dt = 0.5 * HUGE_VAL;
-  // TimeProps::incrtime, properties.h:397-410
-  double time = a.time[b];
   if (time + dt > I.nextoutput) dt = I.nextoutput - time;
   if (time + dt > I.nextsave) dt = I.nextsave - time;
   if (time + dt > I.maxtime) dt = I.maxtime - time;
+  return dt;
+}
+
+__global__ void k_dt(StepArgs a, int ninst) {
+  int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= ninst) return;
+  const double time = a.time[b];
+  const double dt = cfl_dt(a, a.inst[b], a.red[b], time);
   a.time[b] = time + dt;
   a.dt_rec[(long long)b * a.max_steps + a.step] = dt;
   a.red[b].min_ev = dbits(10000000.);
   a.red[b].hmax = dbits(0.);
 }
 
-__device__ __forceinline__ Hfv hfv_at(const StepArgs& a, int dir, long long c) {
-  return hfv_fwd(dir, a.U.h[c], a.U.hu[c], a.U.hv[c], a.kact[c], a.S.gz[c], a.tiny);
+// The dt of member b at this step.  a.fold: it is made here, by every workgroup
+// alike, from the reduction cells the coefficient pass filled (k_dt's
+// arithmetic), instead of in a launch of its own; one workgroup of the member
+// (`own`) also records it, moves the member's clock on and clears the
+// reduction cells of the next step, which nothing else touches meanwhile
+// (steps alternate between two sets, and the clock has a slot per step).
+// Otherwise it was prescribed or recorded before.
+__device__ __forceinline__ double step_dt(const StepArgs& a, int b, bool own) {
+  double* rec = a.dt_rec + (long long)b * a.max_steps + a.step;
+  if (!a.fold) return *rec;
+  const InstDev& I = a.inst[b];
+  const RedDev R = a.red[b];
+  double* clock = a.clock + (long long)b * (a.max_steps + 1) + a.step;
+  const double dt = cfl_dt(a, I, R, *clock);
+  if (own && threadIdx.x == 0) {
+    *rec = dt;
+    clock[1] = a.time[b] = *clock + dt;
+    a.red_next[b].min_ev = dbits(10000000.);
+    a.red_next[b].hmax = dbits(0.);
+  }
+  return dt;
 }
 
 // Face records of one tile: every face flux and every one-sided difference
@@ -344,34 +463,68 @@ struct FaceLds {
   double fx[3][TY][TX + 1], fy[3][TY + 1][TX];
   double dxh[TY][TX + 1], dxhv[TY][TX + 1];  // (U_right - U_left) / dx of h, hv
   double dyh[TY + 1][TX], dyhu[TY + 1][TX];  // (U_top - U_bottom) / dy of h, hu
-  // records of the tile and its one-cell frame: the state and, for h >=
-  // tiny, hu/h, hv/h and sqrt(kact h g2) -- hfv_fwd's values, evaluated
-  // once per cell instead of once per face
+  // records of the tile and its side strips: the state and, for h >= tiny,
+  // hu/h, hv/h and sqrt(kact h g2) -- hfv_fwd's values, evaluated once per
+  // cell instead of once per face
   double h[RXY], hu[RXY], hv[RXY], vx[RXY], vy[RXY], sq[RXY];
 };
-
-// hfv_fwd (tg_math.h) of record r
+// threads of the update: one for every face of a tile, or one for every record
+// (the faces then take two rounds)
 template <int TX>
-__device__ __forceinline__ Hfv rec_hfv(const FaceLds<TX>& L, int dir, int r, double tiny) {
-  Hfv o;
-  const double h = L.h[r], hu = L.hu[r], hv = L.hv[r];
-  if (h < tiny) {
-#pragma unroll
-    for (int i = 0; i < 3; i++) o.u[i] = o.f[i] = o.w[i] = 0.;
-    return o;
-  }
-  const double a = L.sq[r];
-  o.u[0] = h; o.u[1] = hu; o.u[2] = hv;
-  if (dir == 0) {
-    const double vel = L.vx[r];
-    o.f[0] = hu; o.f[1] = hu * vel + 0.5 * a * a * h; o.f[2] = hv * vel;
-    o.w[0] = vel - a; o.w[1] = vel; o.w[2] = vel + a;
+constexpr int face_threads() {
+  return ((TX + 1) * (BLOCK / TX) + TX * (BLOCK / TX + 1) + 63) / 64 * 64;
+}
+template <int TX>
+constexpr int record_threads() {
+  return BLOCK + (2 * TX + 2 * (BLOCK / TX) + 63) / 64 * 64;
+}
+
+// riemannflux (tg_math.h) of the face between records l and r along dir
+// (0 x, 1 y) and their one-sided differences: the three quotients share the
+// reciprocal of their denominator
+template <int TX>
+__device__ __forceinline__ void face_flux(const FaceLds<TX>& L, int dir, int l, int r,
+                                          double tiny, double flux[3]) {
+  const double lh = L.h[l] < tiny ? 0. : L.h[l], rh = L.h[r] < tiny ? 0. : L.h[r];
+  flux[0] = flux[1] = flux[2] = 0.;
+  if (lh == 0. && rh == 0.) return;
+  const double* V = dir ? L.vy : L.vx;
+  const bool lz = L.h[l] < tiny, rz = L.h[r] < tiny;
+  const double lu[3] = {lh, lz ? 0. : L.hu[l], lz ? 0. : L.hv[l]};
+  const double ru[3] = {rh, rz ? 0. : L.hu[r], rz ? 0. : L.hv[r]};
+  const double lv = V[l], rv = V[r], la = L.sq[l], ra = L.sq[r];  // 0 below tiny
+  double lf[3], rf[3];
+  lf[0] = dir ? lu[2] : lu[1];
+  rf[0] = dir ? ru[2] : ru[1];
+  const double lp = 0.5 * la * la * lh, rp = 0.5 * ra * ra * rh;
+  lf[1] = lu[1] * lv; lf[2] = lu[2] * lv;
+  rf[1] = ru[1] * rv; rf[2] = ru[2] * rv;
+  if (dir) { lf[2] += lp; rf[2] += rp; }
+  else { lf[1] += lp; rf[1] += rp; }
+  const double lw0 = lv - la, lw2 = lv + la, rw0 = rv - ra, rw2 = rv + ra;
+  double sl, sr;
+  if (lh == 0.) {
+    sl = umin(0, 2.0 * rw0 - rv);
+    sr = umax(0, 2.0 * rw2 - rv);
+  } else if (rh == 0.) {
+    sl = umin(0, 2.0 * lw0 - lv);
+    sr = umax(0, 2.0 * lw2 - lv);
   } else {
-    const double vel = L.vy[r];
-    o.f[0] = hv; o.f[1] = hu * vel; o.f[2] = hv * vel + 0.5 * a * a * h;
-    o.w[0] = vel - a; o.w[1] = vel; o.w[2] = vel + a;
+    sl = umin(0, umin(lw0, rw0));
+    sr = umax(0, umax(lw2, rw2));
   }
-  return o;
+  if (sl >= 0.0) {
+#pragma unroll
+    for (int v = 0; v < 3; v++) flux[v] = lf[v];
+  } else if (sr <= 0.0) {
+#pragma unroll
+    for (int v = 0; v < 3; v++) flux[v] = rf[v];
+  } else {
+    const double d = sr - sl, g = 1. / d, ss = sl * sr;
+#pragma unroll
+    for (int v = 0; v < 3; v++)
+      flux[v] = div_r(sr * lf[v] - sl * rf[v] + ss * (ru[v] - lu[v]), d, g);
+  }
 }
 
 // Update pass 1 (one workgroup per mark block, one cell of each of its four
@@ -388,7 +541,7 @@ template <int TX>
 __global__ __launch_bounds__(BLOCK) void k_update_classify(StepArgs a) {
   constexpr int TY = BLOCK / TX;
   const BlockDev B = a.blocks[blockIdx.x];
-  const double dt = a.dt_rec[(long long)B.inst * a.max_steps + a.step];
+  const double dt = step_dt(a, B.inst, B.x0 == 0 && B.y0 == 0);
   if (a.mk_in && update_skip(a.mk_in, a.mk_out, B, dt)) return;
   const InstDev I = a.inst[B.inst];
   // tiles of the block holding +0.0 in the input / output state (mark bytes)
@@ -480,24 +633,28 @@ __global__ __launch_bounds__(BLOCK) void k_update_classify(StepArgs a) {
   }
 }
 
+// What the corrector reads of a tile's own cell besides the faces.
+struct CellIn {
+  double h, hu, hv, k, gx, gy, gz, dgx, dgy, kx, ky;
+};
+
 // update_tile's per-cell part: slopes from the staged differences, the four
 // face fluxes with outflow copies, update_states; z: the new state is +0.0.
 template <int TX>
 __device__ __forceinline__ void update_cell(const StepArgs& a, const TileRef& t,
-                                            const InstDev& I, const Cell& q, FaceLds<TX>& L,
-                                            bool& z) {
+                                            const InstDev& I, const Cell& q, const CellIn& u,
+                                            double dt, const FaceLds<TX>& L, bool& z) {
   const int tx = (int)(threadIdx.x % TX), ty = (int)(threadIdx.x / TX);
   const long long c = q.c;
-  const double dt = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
-  const double prev[3] = {a.U.h[c], a.U.hu[c], a.U.hv[c]};
+  const double prev[3] = {u.h, u.hu, u.hv};
   // Element::get_slopes, element2.C:830-939 (only the components the
   // corrector reads: hx, hvx, hy, huy); boundary cells keep zero slopes
   double hx = 0., hvx = 0., hy = 0., huy = 0.;
   if (q.hasE && q.hasW && q.hasN && q.hasS) {
-    hx = slope_from(L.dxh[ty][tx + 1], L.dxh[ty][tx], I.dx, a.gamma, a.tiny);
-    hvx = slope_from(L.dxhv[ty][tx + 1], L.dxhv[ty][tx], I.dx, a.gamma, a.tiny);
-    hy = slope_from(L.dyh[ty + 1][tx], L.dyh[ty][tx], I.dy, a.gamma, a.tiny);
-    huy = slope_from(L.dyhu[ty + 1][tx], L.dyhu[ty][tx], I.dy, a.gamma, a.tiny);
+    hx = slope_from(L.dxh[ty][tx + 1], L.dxh[ty][tx], I.dx, I.inv_sx, a.gamma, a.tiny);
+    hvx = slope_from(L.dxhv[ty][tx + 1], L.dxhv[ty][tx], I.dx, I.inv_sx, a.gamma, a.tiny);
+    hy = slope_from(L.dyh[ty + 1][tx], L.dyh[ty][tx], I.dy, I.inv_sy, a.gamma, a.tiny);
+    huy = slope_from(L.dyhu[ty + 1][tx], L.dyhu[ty][tx], I.dy, I.inv_sy, a.gamma, a.tiny);
   }
   // a face on the domain boundary takes the flux of the opposite face
   // (boundary_flux, element2.C:3374-3411)
@@ -509,13 +666,13 @@ __device__ __forceinline__ void update_cell(const StepArgs& a, const TileRef& t,
     fS[v] = q.hasS ? L.fy[v][ty][tx] : fN[v];
   }
   // correct() -> update_states (corrector.C:36-140, residual.C:162-275)
-  const double kc = (prev[0] > a.tiny) ? a.kact[c] : I.eps;
+  const double kc = (prev[0] > a.tiny) ? u.k : I.eps;
   double out[3];
   SrcInfo si;
-  update_states(prev, out, fE, fN, fW, fS, dt / I.dx, dt / I.dy, dt, hx, hvx, hy, huy,
-                a.S.kx[c], a.S.ky[c], I.sin_int, mat_of(I, a.mat, a.mtab, c).tan_bed,
-                a.S.gx[c], a.S.gy[c], a.S.gz[c],
-                a.S.dgx[c], a.S.dgy[c], kc, a.ft, a.tiny, &si);
+  update_states(prev, out, fE, fN, fW, fS, div_r(dt, I.dx, I.inv_dx), div_r(dt, I.dy, I.inv_dy),
+                dt, hx, hvx, hy, huy, u.kx, u.ky, I.sin_int,
+                mat_of(I, a.mat, a.mtab, c).tan_bed, u.gx, u.gy, u.gz, u.dgx, u.dgy, kc, a.ft,
+                a.tiny, &si);
   if (!isfinite(out[0]) || !isfinite(out[1]) || !isfinite(out[2])) atomicOr(a.err, 1);
   a.h_out[c] = out[0];
   a.hu_out[c] = out[1];
@@ -523,77 +680,153 @@ __device__ __forceinline__ void update_cell(const StepArgs& a, const TileRef& t,
   z = bitzero3(out[0], out[1], out[2]);
 }
 
-// Update pass 2, one listed tile: face fluxes staged in LDS, slopes,
-// update_states.
-template <int TX>
-__device__ __forceinline__ void update_tile(const StepArgs& a, const TileRef& t, FaceLds<TX>& L) {
-  constexpr int TY = BLOCK / TX;
+// Update of one tile: records of the tile and its side strips (the first 256
+// threads the tile's own cells, whose corrector inputs stay in registers),
+// every face once, update_states per cell.  MAYBE_DRY: the tile is not known
+// to be wet; a dry one is written here as the classifying pass would.
+// What bounds it is the chain of one tile: one round trip to memory, then
+// records, faces and cells; so each phase has a thread per item where a tile
+// is all a CU has (576 to 640 threads, 9 to 7 us for 128 x 128 cells, the
+// list walk's 256 threads 9.5 us), and a thread per record, two rounds of
+// faces, where several tiles share a CU (64 members, 5.8 M cells: 20 us;
+// one thread per face 40 us, 256 threads on 64 x 4 tiles 27.5 us).
+template <int TX, int NT, bool MAYBE_DRY>
+__device__ __forceinline__ void update_tile(const StepArgs& a, const TileRef& t, double dt,
+                                            FaceLds<TX>& L) {
+  constexpr int TY = BLOCK / TX, RX = FaceLds<TX>::RX, RY = TY + 2, NHALO = 2 * TX + 2 * TY;
+  constexpr int NFX = (TX + 1) * TY, NFY = TX * (TY + 1);
+  static_assert(BLOCK + NHALO <= NT, "one thread per record");
   const InstDev I = a.inst[t.inst];
-  const Cell q = cell_of<TX>(t);
-  const long long nx = I.nx;
-  if (a.active) {
-    const int cnt = __syncthreads_count(q.act);
-    if (threadIdx.x == 0) atomicAdd(a.active, (unsigned long long)cnt);
-  }
-  // phase 0: records of the tile and its frame (cells of the member only)
-  constexpr int RX = FaceLds<TX>::RX, RXY = FaceLds<TX>::RXY;
-  for (int r = (int)threadIdx.x; r < RXY; r += BLOCK) {
-    const int gi = t.x0 - 1 + r % RX, gj = t.y0 - 1 + r / RX;
-    if (gi >= 0 && gi < I.nx && gj >= 0 && gj < I.ny) {
-      const long long c = I.off + (long long)gj * nx + gi;
-      const double h = a.U.h[c], hu = a.U.hu[c], hv = a.U.hv[c];
+  int tid = (int)threadIdx.x;
+  asm volatile("" : "+v"(tid));  // indexes rebuilt per tile, not held over the tile loop
+  Cell q = cell_of<TX>(t);
+  q.act = q.act && tid < BLOCK;
+  CellIn u = {};
+  bool wet = false;
+  if (tid < BLOCK + NHALO) {
+    int rx, ry;
+    const int h0 = tid - BLOCK;
+    if (h0 < 0) { rx = tid % TX + 1; ry = tid / TX + 1; }
+    else if (h0 < TX) { rx = h0 + 1; ry = 0; }
+    else if (h0 < 2 * TX) { rx = h0 - TX + 1; ry = RY - 1; }
+    else if (h0 < 2 * TX + TY) { rx = 0; ry = h0 - 2 * TX + 1; }
+    else { rx = RX - 1; ry = h0 - 2 * TX - TY + 1; }
+    const int gi = t.x0 - 1 + rx, gj = t.y0 - 1 + ry;
+    if (gi >= 0 && gi < t.nx && gj >= 0 && gj < t.ny) {
+      const long long c = t.off + (long long)gj * t.nx + gi;
+      double h = a.U.h[c], hu = a.U.hu[c], hv = a.U.hv[c], k = a.kact[c], gz = a.S.gz[c];
+      if (h0 < 0) {
+        u.gx = a.S.gx[c]; u.gy = a.S.gy[c]; u.dgx = a.S.dgx[c]; u.dgy = a.S.dgy[c];
+        u.kx = a.S.kx[c]; u.ky = a.S.ky[c];
+      }
+      // all of them in flight together, not each where it is used
+      asm volatile("" : "+v"(hu), "+v"(hv), "+v"(k), "+v"(gz), "+v"(u.gx), "+v"(u.gy),
+                        "+v"(u.dgx), "+v"(u.dgy), "+v"(u.kx), "+v"(u.ky));
+      u.h = h; u.hu = hu; u.hv = hv; u.k = k; u.gz = gz;
+      wet = !(h < a.tiny);
+      const int r = ry * RX + rx;
       L.h[r] = h; L.hu[r] = hu; L.hv[r] = hv;
       double vx = 0., vy = 0., sq = 0.;
-      if (!(h < a.tiny)) {
-        vx = hu / h;
-        vy = hv / h;
-        sq = sqrt(a.kact[c] * h * a.S.gz[c]);
+      if (wet) {
+        const double inv = 1. / h;
+        vx = div_r(hu, h, inv);
+        vy = div_r(hv, h, inv);
+        sq = sqrt(k * h * gz);
       }
       L.vx[r] = vx; L.vy[r] = vy; L.sq[r] = sq;
     }
   }
-  __syncthreads();
-  // phase 1: faces with a cell of the member on both sides
-  // (calc_edge_states, element2.C:2744-3072)
-  for (int f = (int)threadIdx.x; f < (TX + 1) * TY; f += BLOCK) {
-    const int fi = f % (TX + 1), fj = f / (TX + 1);
-    const int gi = t.x0 + fi, gj = t.y0 + fj;
-    if (gi > 0 && gi < I.nx && gj < I.ny) {
-      const int r = (fj + 1) * RX + fi + 1;  // record of the right cell
-      double fl[3];
-      riemann(rec_hfv<TX>(L, 0, r - 1, a.tiny), rec_hfv<TX>(L, 0, r, a.tiny), fl);
-      for (int v = 0; v < 3; v++) L.fx[v][fj][fi] = fl[v];
-      L.dxh[fj][fi] = (L.h[r] - L.h[r - 1]) / I.dx;
-      L.dxhv[fj][fi] = (L.hv[r] - L.hv[r - 1]) / I.dx;
+  if (MAYBE_DRY) {
+    if (!__syncthreads_or(wet)) {
+      // every face flux is zero and there are no sources: update_states'
+      // own arithmetic with zero fluxes
+      const bool zin = a.mk_in && a.zbytes && (a.mk_in[t.mw] >> (8 * mark_byte<TX>(t))) & 1u;
+      const bool keep = zin && a.mk_out && isfinite(dt) &&
+                        (a.mk_out[t.mw] >> (8 * mark_byte<TX>(t))) & 1u;
+      bool z = true;
+      if (q.act) {
+        const double dtdx = dt / I.dx, dtdy = dt / I.dy, zero = 0.;
+        double out[3] = {u.h, u.hu, u.hv};
+#pragma unroll
+        for (int v = 0; v < 3; v++)
+          out[v] = out[v] - dtdx * (zero - zero) - dtdy * (zero - zero);
+        if (out[0] < 0.) out[0] = 0;
+        if (!isfinite(out[0]) || !isfinite(out[1]) || !isfinite(out[2])) atomicOr(a.err, 1);
+        z = bitzero3(out[0], out[1], out[2]);
+        if (!keep) {
+          a.h_out[q.c] = out[0];
+          a.hu_out[q.c] = out[1];
+          a.hv_out[q.c] = out[2];
+        }
+      }
+      if (a.short_cells) {
+        const int cnt = __syncthreads_count(q.act);
+        if (tid == 0) atomicAdd(a.short_cells, (unsigned long long)cnt);
+      }
+      if (a.mk_out) mark_store<TX>(a.mk_out, t, __syncthreads_and(z));
+      return;
     }
+  } else {
+    __syncthreads();
   }
-  for (int f = (int)threadIdx.x; f < TX * (TY + 1); f += BLOCK) {
-    const int fi = f % TX, fj = f / TX;
+  if (a.active) {
+    const int cnt = __syncthreads_count(q.act);
+    if (tid == 0) atomicAdd(a.active, (unsigned long long)cnt);
+  }
+  // faces with a cell of the member on both sides (calc_edge_states,
+  // element2.C:2744-3072)
+#pragma unroll 1
+  for (int k = tid; k < NFX + NFY; k += NT) {
+    const bool isx = k < NFX;
+    const int f = isx ? k : k - NFX, W = isx ? TX + 1 : TX;
+    const int fi = f % W, fj = f / W;
     const int gi = t.x0 + fi, gj = t.y0 + fj;
-    if (gj > 0 && gj < I.ny && gi < I.nx) {
-      const int r = (fj + 1) * RX + fi + 1;  // record of the upper cell
+    if (gi < t.nx && gj < t.ny && (isx ? gi > 0 : gj > 0)) {
+      const int r = (fj + 1) * RX + fi + 1, l = isx ? r - 1 : r - RX;  // upper cell, lower cell
       double fl[3];
-      riemann(rec_hfv<TX>(L, 1, r - RX, a.tiny), rec_hfv<TX>(L, 1, r, a.tiny), fl);
-      for (int v = 0; v < 3; v++) L.fy[v][fj][fi] = fl[v];
-      L.dyh[fj][fi] = (L.h[r] - L.h[r - RX]) / I.dy;
-      L.dyhu[fj][fi] = (L.hu[r] - L.hu[r - RX]) / I.dy;
+      if (isx) {
+        face_flux<TX>(L, 0, l, r, a.tiny, fl);
+        for (int v = 0; v < 3; v++) L.fx[v][fj][fi] = fl[v];
+        L.dxh[fj][fi] = div_r(L.h[r] - L.h[l], I.dx, I.inv_dx);
+        L.dxhv[fj][fi] = div_r(L.hv[r] - L.hv[l], I.dx, I.inv_dx);
+      } else {
+        face_flux<TX>(L, 1, l, r, a.tiny, fl);
+        for (int v = 0; v < 3; v++) L.fy[v][fj][fi] = fl[v];
+        L.dyh[fj][fi] = div_r(L.h[r] - L.h[l], I.dy, I.inv_dy);
+        L.dyhu[fj][fi] = div_r(L.hu[r] - L.hu[l], I.dy, I.inv_dy);
+      }
     }
   }
   __syncthreads();
   bool z = true;
-  if (q.act) update_cell<TX>(a, t, I, q, L, z);
+  if (q.act) update_cell<TX>(a, t, I, q, u, dt, L, z);
   if (a.mk_out) mark_store<TX>(a.mk_out, t, __syncthreads_and(z));
 }
 
-
 template <int TX>
-__global__ __launch_bounds__(BLOCK) void k_update(StepArgs a) {
+__global__ __launch_bounds__(record_threads<TX>(), 5) void k_update(StepArgs a) {
   __shared__ FaceLds<TX> L;
   const int n = *a.tile_count;
   for (int i = (int)blockIdx.x; i < n; i += (int)gridDim.x) {
-    update_tile<TX>(a, a.tile_list[list_band(i, n)], L);
+    const TileRef t = a.tile_list[list_band(i, n)];
+    update_tile<TX, record_threads<TX>(), false>(a, t, a.dt_rec[(long long)t.inst * a.max_steps + a.step], L);
     __syncthreads();  // LDS reused by the next tile
   }
+}
+
+__device__ __forceinline__ TileRef ref_of(const TileDev& t, int tile) {
+  return TileRef{t.inst, tile, t.x0, t.y0, t.mw, t.nx, t.ny, 0, t.off};
+}
+
+// Update on small meshes, one workgroup per tile, nothing listed.
+template <int TX>
+__global__ __launch_bounds__(face_threads<TX>()) void k_update_tile(StepArgs a) {
+  __shared__ FaceLds<TX> L;
+  const int tile = tile_of(a);
+  const TileDev t = a.tiles[tile];
+  const double dt = step_dt(a, t.inst, t.x0 == 0 && t.y0 == 0);
+  if (a.mk_in && update_skip(a.mk_in, a.mk_out, t, dt)) return;
+  update_tile<TX, face_threads<TX>(), true>(a, ref_of(t, tile), dt, L);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_stats(const InstDev* inst, const TileDev* tiles,
@@ -743,11 +976,11 @@ __device__ __forceinline__ double swap_pair(double v) {
 //
 // What bounds it: FP64 instruction issue (52 % of the issue slots at 128
 // VGPRs, four waves per SIMD) and, per tile, three round trips to memory (list
-// entry, records, results).  A 64-member ensemble of 5.8 M cells: 51 us per
+// entry, records, results).  A 64-member ensemble of 5.8 M cells: 60 us per
 // step against 81 us for one thread per cell with every face's forward and
-// dual flux evaluated apart (26.0 M wave instructions, now 15.6 M); one
-// tile alone: 13.8 against 27 us.  One thread per cell needs 168 VGPRs (81
-// us), four per cell repeat the self block (75 us).
+// dual flux evaluated apart; one tile alone (128 x 128 cells): 12 against 27
+// us.  One thread per cell needs 168 VGPRs (81 us), four per cell repeat the
+// self block (75 us).
 template <int TX, bool DPHI>
 struct DualLds {
   static constexpr int RX = TX + 2, RN = (TX + 2) * (BLOCK / TX + 2);
@@ -758,15 +991,15 @@ struct DualLds {
   // neighbour subtracts (compute_jacobian_elem.C:44-51)
   double src[4][RN];
   double lam[3][RN];  // lambda^{s+1}
-  // bed-friction gradient: d kact / d phi_bed times d F_n / d kact and
-  // d sqrt(kact h g2) / d kact
-  double dF[DPHI ? RN : 1], dw[DPHI ? RN : 1];
+  // bed-friction gradient: hu/h and hv/h, and d kact / d phi_bed times d F_n /
+  // d kact and d sqrt(kact h g2) / d kact
+  double vx[DPHI ? RN : 1], vy[DPHI ? RN : 1], dF[DPHI ? RN : 1], dw[DPHI ? RN : 1];
   // the tile's cells: what the self block subtracts from its entries 10, 10,
   // 11, 20, 20, 22 (compute_jacobian_elem.C:55-110), the sources' phi_bed
   // derivatives, and whether h != 0
   double self[6][BLOCK];
   double dsrc[2][DPHI ? BLOCK : 1];
-  double sp[2 * BLOCK / 64];
+  double sp[BLOCK / 64];
   unsigned char nz[BLOCK];
 };
 constexpr int ADJ_THREADS = 2 * BLOCK;
@@ -836,7 +1069,11 @@ __device__ __forceinline__ bool dual_record(const AdjArgs& a, const TileRef& t, 
     L.sq[r] = flows ? sqrt(1. * I.eps * h * g2) : 0.;
 #pragma unroll
     for (int k = 0; k < 4; k++) L.src[k][r] = 0.;
-    if (DPHI) L.dF[r] = L.dw[r] = 0.;
+    if (DPHI) {
+      L.vx[r] = flows ? hu / h : 0.;
+      L.vy[r] = flows ? hv / h : 0.;
+      L.dF[r] = L.dw[r] = 0.;
+    }
     if (own >= 0) {
 #pragma unroll
       for (int k = 0; k < 6; k++) L.self[k][own] = 0.;
@@ -882,6 +1119,8 @@ __device__ __forceinline__ bool dual_record(const AdjArgs& a, const TileRef& t, 
     dk = (still || kf < 0.) ? 0. : -I.kc1 * sg * M.dkroot * I.eps;
     L.dw[r] = (sq > 0.) ? dk * ((h * g2) / (2. * sq)) : 0.;
     L.dF[r] = dk * (0.5 * h * g2 * h);
+    L.vx[r] = vx;
+    L.vy[r] = vy;
   }
   if (own >= 0) {
     L.self[0][own] = dt * (g0 - alpha * h * (2 * dg1 + g2 * sy[0]) - alpha * g2 * hy);
@@ -906,10 +1145,10 @@ __device__ __forceinline__ bool dual_record(const AdjArgs& a, const TileRef& t, 
 struct FaceJac {
   double a00, a0n, an0, ann, at0, atn, att;
 };
-// The face's mass flux, and the derivative of its flux along d kact /
-// d phi_bed on both sides.
+// The derivative of the face's momentum fluxes along d kact / d phi_bed on both
+// sides.
 struct FaceDk {
-  double flux0, d0, dn, dt;
+  double dn, dt;
 };
 
 // dual_riemann_side (tg_math.h) of the face between the cell's record rc and
@@ -955,8 +1194,7 @@ __device__ __forceinline__ FaceJac face_jac(const DualLds<TX, DPHI>& L, bool isx
     J.an0 = own ? fn0 : 0.; J.ann = own ? 2 * cv : 0.;
     J.at0 = own ? ft0 : 0.; J.atn = own ? ftn : 0.; J.att = own ? cv : 0.;
     if (DPHI) {
-      D.flux0 = own ? cq : nq;
-      D.d0 = D.dt = 0.;
+      D.dt = 0.;
       D.dn = own ? dFc : dFn;
     }
     return J;
@@ -976,10 +1214,6 @@ __device__ __forceinline__ FaceJac face_jac(const DualLds<TX, DPHI>& L, bool isx
     const double p = (cq + sl * vd - fx) * g, m = (-nq + sr * vd + fx) * g;
     J.a00 = p * dsr0 + m * dsl0 + jv;
     J.a0n = p * dsrn + m * dsln + (cvoid ? 0. : srg);
-    if (DPHI) {
-      D.flux0 = fx;
-      D.d0 = p * dsr + m * dsl;
-    }
   }
   {
     const double cf = cq * cv + 0.5 * ca * ca * ch, nf = nq * nv + 0.5 * na * na * nh;
@@ -1071,6 +1305,37 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_classify(AdjArgs a) {
 }
 
 
+// The face's mass flux and its derivative along d kact / d phi_bed on both
+// sides (riemann and driemann, tg_math.h, component 0), mirrored as in
+// face_jac.  It has the forward flux's own velocities hu/h, not the dual
+// flux's hu (1/h): where the functional is the whole mass the terms of all
+// faces cancel, and what is left is the rounding of exactly these values.
+template <int TX>
+__device__ __forceinline__ void face_mass_dk(const DualLds<TX, true>& L, bool isx, bool plus,
+                                             int rc, int rn, double& flux, double& d0) {
+  const double* Q = isx ? L.hu : L.hv;
+  const double* V = isx ? L.vx : L.vy;
+  const double ch = L.h[rc], ca = L.sq[rc], nh = L.h[rn], na = L.sq[rn];
+  double cq = Q[rc], nq = Q[rn], cv = V[rc], nv = V[rn];
+  if (!plus) { cq = -cq; nq = -nq; cv = -cv; nv = -nv; }
+  const bool cvoid = ch == 0., nvoid = nh == 0.;
+  const double cw0 = cv - ca, cw2 = cv + ca, nw0 = nv - na, nw2 = nv + na;
+  const double c0 = nvoid ? 2. * cw0 - cv : cw0, c2 = nvoid ? 2. * cw2 - cv : cw2;
+  const double n0 = cvoid ? 2. * nw0 - nv : nw0, n2 = cvoid ? 2. * nw2 - nv : nw2;
+  const double sl = fmin(0., fmin(c0, n0)), sr = fmax(0., fmax(c2, n2));
+  if (sl >= 0. || sr <= 0.) {
+    flux = (plus ? sl >= 0. : !(sr <= 0.)) ? cq : nq;
+    d0 = 0.;
+    return;
+  }
+  const double dwc = L.dw[rc], dwn = L.dw[rn], dv = 2. * (cvoid ? dwn : dwc);
+  const bool one = cvoid || nvoid;
+  const double dsl = -(one ? dv : (c0 > n0 ? dwn : dwc)), dsr = one ? dv : (c2 > n2 ? dwc : dwn);
+  const double g = 1. / (sr - sl), vd = nh - ch;
+  flux = (sr * cq - sl * nq + sl * sr * vd) * g;
+  d0 = (cq + sl * vd - flux) * g * dsr + (-nq + sr * vd + flux) * g * dsl;
+}
+
 // Adjoint pass 2, one tile.  MAYBE_VOID: the tile is not known to hold
 // anything; a void one is written here as the classifying pass would.
 template <int TX, bool DPHI, bool MAYBE_VOID>
@@ -1126,6 +1391,7 @@ __device__ __forceinline__ void adjoint_tile(const AdjArgs& a, const TileRef& t,
     const double* LN = isx ? L.lam[1] : L.lam[2];  // normal and tangential adjoint
     const double* LT = isx ? L.lam[2] : L.lam[1];
     const double lc0 = L.lam[0][rc], lcn = LN[rc], lct = LT[rc];
+    const double hraw = L.h[rc];
     double out[3] = {0., 0., 0.};
     // a cell with lambda^{s+1} = 0 adds lambda . dU/dphi = 0 to the gradient
     if (full || (DPHI && !(lc0 == 0. && lcn == 0. && lct == 0.))) {
@@ -1138,23 +1404,30 @@ __device__ __forceinline__ void adjoint_tile(const AdjArgs& a, const TileRef& t,
       const int stepA = isx ? 1 : -RX;
       // (a missing neighbour: any face, its entries are replaced below)
       const int rA = hasA ? rc + stepA : rc, rB = hasB ? rc - stepA : rc;
-      FaceDk D;
-      // lambda^{s+1}_c . d U^{s+1}_c / d phi_bed at frozen dt (no reference
-      // counterpart): an outflow face copies the opposite face, so the
-      // pair's difference vanishes; h clamped at 0 does not vary
-      const double pair = hasA && hasB ? dtd : 0.;
-      double mass = 0., d0 = 0.;
-      FaceJac A = face_jac<TX, DPHI>(L, isx, isx, rc, rA, D);
-      if (DPHI) {
-        mass = pair * D.flux0; d0 = pair * D.d0;
-        dphi -= lcn * ((isx ? pair : -pair) * D.dn) + lct * (pair * D.dt);
-      }
-      FaceJac B = face_jac<TX, DPHI>(L, isx, !isx, rc, rB, D);
-      if (DPHI) {
-        mass += pair * D.flux0; d0 += pair * D.d0;
-        dphi -= lcn * ((isx ? -pair : pair) * D.dn) + lct * (pair * D.dt);
-        if (!(L.h[rc] - (mass + swap_pair(mass)) < 0.)) dphi -= lc0 * d0;
-        if (isx) dphi += lcn * L.dsrc[0][q] + lct * L.dsrc[1][q];
+      FaceDk DA, DB;
+      FaceJac A = face_jac<TX, DPHI>(L, isx, isx, rc, rA, DA);
+      FaceJac B = face_jac<TX, DPHI>(L, isx, !isx, rc, rB, DB);
+      if constexpr (DPHI) {
+        // lambda^{s+1}_c . d U^{s+1}_c / d phi_bed at frozen dt (no reference
+        // counterpart): the flux differences of this thread's direction, plus
+        // face minus minus face (mass and tangential: mirrored, so their sum);
+        // an outflow face copies the opposite face, so the pair's difference
+        // vanishes; h clamped at 0 does not vary
+        double fA, fB, dA, dB;
+        face_mass_dk<TX>(L, isx, isx, rc, rA, fA, dA);
+        face_mass_dk<TX>(L, isx, !isx, rc, rB, fB, dB);
+        const bool pair = hasA && hasB;
+        const double f0 = dtd * (pair ? fA + fB : 0.);
+        const double m0 = dtd * (pair ? dA + dB : 0.), mt = dtd * (pair ? DA.dt + DB.dt : 0.);
+        const double mn = dts * (pair ? DA.dn - DB.dn : 0.);
+        // out = -x - y: the x thread adds them up (its n = 1, t = 2)
+        const double y0 = swap_pair(m0), y2 = swap_pair(mn), y1 = swap_pair(mt);
+        const double fy = swap_pair(f0);
+        double o0 = -m0 - y0, o1 = -mn - y1, o2 = -mt - y2;
+        if (hraw - f0 - fy < 0.) o0 = 0.;
+        o1 += L.dsrc[0][q];
+        o2 += L.dsrc[1][q];
+        dphi = lc0 * o0 + lcn * o1 + lct * o2;
       }
       if (full) {
         // an outflow face copies the opposite face (boundary_flux): its
@@ -1243,14 +1516,18 @@ __device__ __forceinline__ void adjoint_tile(const AdjArgs& a, const TileRef& t,
     const int cnt = __syncthreads_count(act && isx);
     if (tid == 0) atomicAdd(a.active, (unsigned long long)cnt);
   }
+  // the cell's term where its self terms were (only this pair reads them)
+  if (DPHI && isx) L.self[0][q] = dphi;
   const bool all = a.mk_out || DPHI ? __syncthreads_and(zero_out) : false;
-  if (DPHI) {
-    dphi = wave_sum(dphi);
-    if (tid % 64 == 0) L.sp[tid / 64] = dphi;
+  if (DPHI) {  // the tile's sum: 64 cells to a wave, then the waves in order
+    if (tid < BLOCK) {
+      dphi = wave_sum(L.self[0][tid]);
+      if (tid % 64 == 0) L.sp[tid / 64] = dphi;
+    }
     __syncthreads();
     if (tid == 0) {
-      for (int k = 1; k < ADJ_THREADS / 64; k++) dphi += L.sp[k];
-      unsafeAtomicAdd(a.dphi_part + t.tile, dphi);  // the tile's only writer: nothing waits for it
+      for (int k = 1; k < BLOCK / 64; k++) dphi += L.sp[k];
+      unsafeAtomicAdd(a.dphi_part + t.tile, dphi);  // its only writer: nothing waits for it
     }
   }
   if (a.mk_out) mark_store<TX>(a.mk_out, t, all);
@@ -1266,6 +1543,16 @@ __global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint(AdjArgs a) {
   }
 }
 
+// Reverse step on small meshes, one workgroup per tile, nothing listed.
+template <int TX, bool DPHI>
+__global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint_tile(AdjArgs a) {
+  __shared__ DualLds<TX, DPHI> L;
+  const int tile = tile_of(a);
+  const TileDev t = a.tiles[tile];
+  if (a.mk_out && adjoint_skip(a.mk_U, DPHI ? a.mk_lnext : nullptr, a.mk_out, t.mw)) return;
+  adjoint_tile<TX, DPHI, true>(a, ref_of(t, tile), L);
+}
+
 }  // namespace
 
 // one instantiation per built tile width; a.shape selects it
@@ -1279,29 +1566,49 @@ __global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint(AdjArgs a) {
   } while (0)
 
 void launch_coef(const StepArgs& a, bool reduce, hipStream_t s) {
-  TG_LAUNCH_TX(a.shape, k_coef, dim3(a.nblocks), s, a, reduce ? 1 : 0);
+  if (a.by_tile) TG_LAUNCH_TX(a.shape, k_coef_tile, dim3(a.ntiles), s, a, reduce ? 1 : 0);
+  else TG_LAUNCH_TX(a.shape, k_coef, dim3(a.nblocks), s, a, reduce ? 1 : 0);
 }
 void launch_dt(const StepArgs& a, int ninst, hipStream_t s) {
   hipLaunchKernelGGL(k_dt, dim3((ninst + 63) / 64), dim3(64), 0, s, a, ninst);
 }
 // classify every tile (skipped by the marks, short path written, or
-// listed), then a fixed grid walks the list with the full path
+// listed), then a fixed grid walks the list with the full path; the
+// coefficient pass emptied the list
 void launch_update(const StepArgs& a, hipStream_t s) {
-  if (!a.dt_clears_count) launch_zero(a.tile_count, sizeof(int), s);
-  TG_LAUNCH_TX(a.shape, k_update_classify, dim3(a.nblocks), s, a);
-  TG_LAUNCH_TX(a.shape, k_update, dim3(a.ntiles < LIST_GRID ? a.ntiles : LIST_GRID), s, a);
+  const int g = a.by_tile || a.ntiles < LIST_GRID ? a.ntiles : LIST_GRID;
+#define TG_UPD(TX)                                                                             \
+  if (a.by_tile)                                                                               \
+    hipLaunchKernelGGL(k_update_tile<TX>, dim3(g), dim3(face_threads<TX>()), 0, s, a);         \
+  else {                                                                                       \
+    hipLaunchKernelGGL(k_update_classify<TX>, dim3(a.nblocks), dim3(BLOCK), 0, s, a);          \
+    hipLaunchKernelGGL(k_update<TX>, dim3(g), dim3(record_threads<TX>()), 0, s, a);            \
+  }
+  switch (SHAPE_TX[a.shape]) {
+    case 64: TG_UPD(64); break;
+    case 32: TG_UPD(32); break;
+    default: TG_UPD(16); break;
+  }
+#undef TG_UPD
 }
 void launch_adjoint(const AdjArgs& a, hipStream_t s) {
-  launch_zero(a.tile_count, sizeof(int), s);
-  TG_LAUNCH_TX(a.shape, k_adjoint_classify, dim3(a.nblocks), s, a);
-  const dim3 g(a.ntiles < ADJ_GRID ? a.ntiles : ADJ_GRID);
-#define TG_ADJ(TX)                                                                        \
-  if (a.dphi_part) hipLaunchKernelGGL((k_adjoint<TX, true>), g, dim3(ADJ_THREADS), 0, s, a); \
-  else hipLaunchKernelGGL((k_adjoint<TX, false>), g, dim3(ADJ_THREADS), 0, s, a)
-  switch (SHAPE_TX[a.shape]) {
-    case 64: TG_ADJ(64); break;
-    case 32: TG_ADJ(32); break;
-    default: TG_ADJ(16); break;
+  if (!a.by_tile) {
+    launch_zero(a.tile_count, sizeof(int), s);
+    TG_LAUNCH_TX(a.shape, k_adjoint_classify, dim3(a.nblocks), s, a);
+  }
+  const dim3 g(a.by_tile || a.ntiles < ADJ_GRID ? a.ntiles : ADJ_GRID), b(ADJ_THREADS);
+#define TG_ADJ(TX, DPHI)                                                            \
+  if (a.by_tile) hipLaunchKernelGGL((k_adjoint_tile<TX, DPHI>), g, b, 0, s, a);     \
+  else hipLaunchKernelGGL((k_adjoint<TX, DPHI>), g, b, 0, s, a)
+  const int tx = SHAPE_TX[a.shape];
+  if (a.dphi_part) {
+    if (tx == 64) { TG_ADJ(64, true); }
+    else if (tx == 32) { TG_ADJ(32, true); }
+    else { TG_ADJ(16, true); }
+  } else {
+    if (tx == 64) { TG_ADJ(64, false); }
+    else if (tx == 32) { TG_ADJ(32, false); }
+    else { TG_ADJ(16, false); }
   }
 #undef TG_ADJ
 }
@@ -1337,8 +1644,10 @@ void launch_member_fill(const void* src, void* dst, int es, long long ncell, lon
   hipLaunchKernelGGL(k_member_fill, dim3(grid_for(n)), dim3(256), 0, s, (const uint32_t*)src,
                      (uint32_t*)dst, ncell * w, off * w, count * w, mk, mw0, nmw);
 }
-void launch_reset_red(RedDev* red, int ninst, hipStream_t s) {
-  hipLaunchKernelGGL(k_reset_red, dim3((ninst + 63) / 64), dim3(64), 0, s, red, ninst);
+void launch_reset_red(RedDev* red, int ninst, const double* time, double* clock, long long stride,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(k_reset_red, dim3((ninst + 63) / 64), dim3(64), 0, s, red, ninst, time,
+                     clock, stride);
 }
 void launch_stats(const InstDev* inst, const TileDev* tiles, int ntiles, Fields U,
                   const uint32_t* mk, double* part_mass, double* part_hmax, double tiny,

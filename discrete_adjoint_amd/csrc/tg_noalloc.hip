@@ -33,7 +33,7 @@ constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 // byte offsets into the scratch array
 constexpr size_t OFF_INST = 0;
 constexpr size_t OFF_RED = OFF_INST + align256(sizeof(InstDev));
-constexpr size_t OFF_MISC = OFF_RED + align256(sizeof(RedDev));  // dt, time, err, count
+constexpr size_t OFF_MISC = OFF_RED + align256(2 * sizeof(RedDev));  // dt, time, err, count
 constexpr size_t OFF_TILES = OFF_MISC + 256;
 constexpr size_t OFF_BLOCKS = OFF_TILES + align256(sizeof(TileDev) * NA_MAX_TILES);
 constexpr size_t OFF_LIST = OFF_BLOCKS + align256(sizeof(BlockDev) * NA_MAX_BLOCKS);
@@ -50,7 +50,7 @@ InstDev g_inst;
 TileDev g_tiles[NA_MAX_TILES];
 BlockDev g_blocks[NA_MAX_BLOCKS];
 struct Misc {
-  double dt_rec, time;
+  double dt_rec, time, clock[2];
   int err, tile_count;
 };
 
@@ -156,7 +156,7 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   g_inst.eps = prm->epsilon; g_inst.gscale = prm->gravity_scale;
   g_inst.maxtime = prm->maxtime; g_inst.nextoutput = prm->nextoutput;
   g_inst.nextsave = prm->nextsave;
-  const Misc misc{0.0, time, 0, 0};
+  const Misc misc{0.0, time, {time, 0.0}, 0, 0};
 
   NA_CHK(hipMemcpyAsync(base + OFF_INST, &g_inst, sizeof(InstDev), hipMemcpyHostToDevice, s));
   NA_CHK(hipMemcpyAsync(base + OFF_MISC, &misc, sizeof(Misc), hipMemcpyHostToDevice, s));
@@ -179,7 +179,11 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.kact = (double*)(base + OFF_KACT);
   a.red = (RedDev*)(base + OFF_RED);
   a.dt_rec = &md->dt_rec;
+  a.red_next = a.red + 1;
   a.time = &md->time;
+  a.clock = md->clock;
+  a.fold = 1;
+  a.by_tile = ntiles <= TILE_LAUNCH_MAX ? 1 : 0;
   a.max_steps = 1;
   a.step = 0;
   a.ft = (step < cfg->frict_tiny_switch) ? cfg->frict_tiny_early : cfg->frict_tiny_late;
@@ -190,14 +194,12 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.active = nullptr;
   a.tile_list = (TileRef*)(base + OFF_LIST);
   a.tile_count = &md->tile_count;
-  a.dt_clears_count = 1;
   a.mk_in = nullptr;   // no zero marks: every tile is classified from its cells
   a.mk_out = nullptr;
   a.short_cells = nullptr;
 
-  launch_reset_red(a.red, 1, s);
+  launch_reset_red(a.red, 1, nullptr, nullptr, 0, s);
   launch_coef(a, true, s);
-  launch_dt(a, 1, s);
   launch_update(a, s);
   NA_CHK(hipGetLastError());
   Misc back{};
