@@ -28,6 +28,8 @@ struct SweepGraph {
   bool valid = false;
 };
 
+constexpr int NCOUNT = 6;
+
 struct tg_ctx {
   tg_config cfg{};
   hipStream_t stream = nullptr;
@@ -115,6 +117,8 @@ struct tg_ctx {
   // tiles taking the full path of the update / adjoint (compacted by their
   // classifying pass) and the list length
   TileRef* act_list = nullptr;  // (the FP32 adjoint lists bare tile indices in it)
+  // [NCOUNT] list lengths: two pairs of the forward steps, two of the reverse
+  // steps (launches alternate; [0] also the FP32 adjoint's)
   int* act_count = nullptr;
 
   // adaptive mesh (TG_MESH_LEAVES): leaf tables and reverse-step buffers
@@ -413,6 +417,10 @@ void use_tiles(const tg_ctx* ctx, int kernel, A& a) {
   a.shape = v;
 }
 
+// The kernel whose tile variant the FP64 first pass takes: where it lists the
+// update's tiles, the update's.
+int first_variant_of(const tg_ctx* ctx) { return tile_launch(ctx, 0) == 0 ? 1 : 0; }
+
 // Zero marks of a buffer given by its field pointers (h first), or null
 // when the kernels keep none.
 uint32_t* marks_of(const tg_ctx* ctx, void* const f[3]) {
@@ -594,7 +602,9 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
     a.h_out = (double*)out[0]; a.hu_out = (double*)out[1]; a.hv_out = (double*)out[2];
     a.err = ctx->err_d;
     a.tile_list = ctx->act_list;
-    a.tile_count = ctx->act_count;
+    a.tile_count = ctx->act_count + 2 * (s & 1);
+    a.count_next = ctx->act_count + 2 * ((s + 1) & 1);
+    a.ninst = ctx->ninst;
     a.mk_in = marks_of(ctx, in);
     a.mk_out = marks_of(ctx, out);
     a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[1]] == ctx->mk_tx[0];
@@ -617,8 +627,9 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
     a.fold = compute_dt;
     a.red = ctx->red + (s & 1) * ctx->ninst;
     a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst;
-    use_tiles(ctx, 0, a);
-    a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[0]] == ctx->mk_tx[0];
+    const int first = first_variant_of(ctx);
+    use_tiles(ctx, first, a);
+    a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[first]] == ctx->mk_tx[0];
     a.active = inst_counter(ctx, 0, true);
     a.short_cells = inst_short(ctx, 0, true);
     inst_mark(ctx, 0, true);
@@ -659,7 +670,8 @@ void enqueue_adjoint(tg_ctx* ctx, void* const U[3], void* const lnext[3], void* 
     a.lam_h = (double*)lout[0]; a.lam_hu = (double*)lout[1]; a.lam_hv = (double*)lout[2];
     a.dphi_part = dphi ? ctx->dphi_part : nullptr;
     a.tile_list = ctx->act_list;
-    a.tile_count = ctx->act_count;
+    a.tile_count = ctx->act_count + 4 + (s & 1);
+    a.count_next = ctx->act_count + 4 + ((s + 1) & 1);
     a.mk_U = marks_of(ctx, U);
     a.mk_lnext = marks_of(ctx, lnext);
     a.mk_out = marks_of(ctx, lout);
@@ -908,8 +920,15 @@ int stored_steps(const tg_ctx* ctx, int nsteps) {
   return (int)(m < nsteps ? (m < 0 ? 0 : m) : nsteps);
 }
 
-// The reduction cells cleared and every member's clock set for step s.
+// Every sequence of consecutive steps, forward or reverse, starts from empty
+// tile lists (each step then empties the next one's).
+void empty_lists(tg_ctx* ctx) {
+  if (!ctx->leaves && tile_launch(ctx, 0) == 0)
+    launch_zero(ctx->act_count, sizeof(int) * NCOUNT, ctx->stream);
+}
+// ... and the reduction cells cleared and every member's clock set for step s.
 void start_clock(tg_ctx* ctx, int s) {
+  empty_lists(ctx);
   launch_reset_red(ctx->red, ctx->ninst, ctx->time_d, ctx->clock_d + s,
                    (long long)ctx->cfg.max_steps + 1, ctx->stream);
 }
@@ -1110,6 +1129,7 @@ int adjoint_loop(tg_ctx* ctx, const tg_params* prm, const double* w, const int* 
     return b < S ? b : S;
   };
   auto stored = [&](int& cur) {
+    empty_lists(ctx);
     for (int s = S - 1; s >= s0; s--) {
       void* Us[3];
       void* Un[3];
@@ -1130,6 +1150,7 @@ int adjoint_loop(tg_ctx* ctx, const tg_params* prm, const double* w, const int* 
   };
   auto recompute = [&](int sg) {
     const int a = sg * k, b = seg_end(a);
+    empty_lists(ctx);
     for (int s = a; s + 1 < b; s++) {
       void* in[3];
       void* out[3];
@@ -1524,7 +1545,7 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
     rc = dalloc(ctx, (void**)&ctx->thin_list, sizeof(int2) * (size_t)n);
   if (!rc && ctx->mode != TG_FP64) rc = dalloc(ctx, (void**)&ctx->thin_count, sizeof(int));
   if (!rc) rc = dalloc(ctx, (void**)&ctx->act_list, sizeof(TileRef) * (size_t)ctx->ntiles);
-  if (!rc) rc = dalloc(ctx, (void**)&ctx->act_count, sizeof(int));
+  if (!rc) rc = dalloc(ctx, (void**)&ctx->act_count, sizeof(int) * NCOUNT);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->inst_d, sizeof(InstDev) * nm);
   for (int v = 0; v < NSHAPE && !rc; v++)
     rc = dalloc(ctx, (void**)&ctx->tiles_d[v], sizeof(TileDev) * ctx->nt[v]);
@@ -2067,6 +2088,7 @@ int tg_forward_step(tg_ctx* ctx, const tg_params* prm, tg_stats* stats) {
   if (rc) return rc;
   if (ctx->rec_steps == 0) zero_box_record(ctx);
   if (ctx->rec_steps == 0 || ctx->clock_at != ctx->rec_steps) start_clock(ctx, ctx->rec_steps);
+  else empty_lists(ctx);
   ctx->clock_at = -1;  // until this step has been taken
   enqueue_step(ctx, ctx->U, ctx->Ut, ctx->rec_steps, true);
   enqueue_box_max(ctx, ctx->Ut, ctx->rec_steps);
@@ -2124,6 +2146,7 @@ int tg_get_trajectory_state(tg_ctx* ctx, int s, double* h, double* hu, double* h
     void* base[3];
     split(ctx, ctx->ckpt[s / k], base);
     copy_state(ctx, ctx->seg[0], base);
+    empty_lists(ctx);
     for (int t = a; t < s; t++) {
       void* in[3];
       void* out[3];
@@ -2314,6 +2337,7 @@ int adjoint_step_impl(tg_ctx* ctx, const tg_params* prm, int s, double dt,
   clear_marks(ctx, ctx->lam[0][0]);
   const bool dphi = dphi_member != nullptr;
   if (dphi) launch_zero(ctx->dphi_part, sizeof(double) * ctx->ntiles, ctx->stream);
+  empty_lists(ctx);
   enqueue_adjoint(ctx, ctx->U, ctx->lam[0], ctx->lam[1], s, dphi);
   HIPCHK(ctx, hipGetLastError());
   for (int c = 0; c < 3; c++) {
@@ -2367,12 +2391,13 @@ int time_kernel_variant(tg_ctx* ctx, int which, int v, int reps, double* avg_ms)
   // here and cleared by the next tg_adjoint_run)
   auto one = [&](int w) {
     if (w == 2) {
+      empty_lists(ctx);
       enqueue_adjoint(ctx, ctx->U, ctx->lam[0], ctx->lam[1], 0, true);
     } else if (fwd64(ctx)) {
       StepArgs a{};
       const long long n = ctx->ncell;
       a.inst = ctx->inst_d;
-      use_tiles(ctx, w, a);
+      use_tiles(ctx, w == 0 ? first_variant_of(ctx) : w, a);
       a.U = Fields{(double*)ctx->U[0], (double*)ctx->U[1], (double*)ctx->U[2]};
       a.S = Statics{at<double>(ctx->statics, 0, n), at<double>(ctx->statics, 1, n),
                     at<double>(ctx->statics, 2, n), at<double>(ctx->statics, 3, n),
@@ -2384,6 +2409,9 @@ int time_kernel_variant(tg_ctx* ctx, int which, int v, int reps, double* avg_ms)
       a.err = ctx->err_d;
       a.tile_list = ctx->act_list;
       a.tile_count = ctx->act_count;
+      a.count_next = ctx->act_count + 2;
+      a.ninst = ctx->ninst;
+      if (w == 0) empty_lists(ctx);  // (the update walks the list of the launch before)
       a.mk_in = marks_of(ctx, ctx->U);
       a.mk_out = marks_of(ctx, ctx->Ut);
       a.zbytes = 0;  // (timing: see bytes_off)
@@ -2396,7 +2424,6 @@ int time_kernel_variant(tg_ctx* ctx, int which, int v, int reps, double* avg_ms)
       } else if (w == 0) {
         launch_coef(a, false, ctx->stream);
       } else {
-        if (!a.by_tile) launch_zero(ctx->act_count, sizeof(int), ctx->stream);
         launch_update(a, ctx->stream);
       }
       inst_mark(ctx, w, false);

@@ -95,22 +95,16 @@ __device__ __forceinline__ void mark_store(uint32_t* mk, const T& t, bool all) {
 }
 
 // Skips decided from the marks alone, for a whole mark block.
-// Coefficient pass: the block of U is +0.0 -- h = +0.0 < tiny: no kact
-// written, nothing added to the CFL reduction.
-__device__ __forceinline__ bool coef_skip(const uint32_t* mk, int mw) {
-  return mk[mw] == MARK_FULL;
-}
 // Update: the block and the four side blocks of U are +0.0 -- every cell
 // and side neighbour has h < tiny, so the fluxes are zero and there are no
 // sources, and U^{s+1} = U^s - dtdx*(0 - 0) - dtdy*(0 - 0) = +0.0 for a
 // finite dt -- and the block of the output already holds +0.0.
 template <class Blk>
 __device__ __forceinline__ bool update_skip(const uint32_t* in, const uint32_t* out,
-                                            const Blk& B, double dt) {
+                                            const Blk& B) {
   return in[B.mw] == MARK_FULL && out[B.mw] == MARK_FULL &&
          (B.mwW < 0 || in[B.mwW] == MARK_FULL) && (B.mwE < 0 || in[B.mwE] == MARK_FULL) &&
-         (B.mwS < 0 || in[B.mwS] == MARK_FULL) && (B.mwN < 0 || in[B.mwN] == MARK_FULL) &&
-         isfinite(dt);
+         (B.mwS < 0 || in[B.mwS] == MARK_FULL) && (B.mwN < 0 || in[B.mwN] == MARK_FULL);
 }
 // Adjoint: the block of U^s is +0.0 (void cells: lambda^s = +0.0), that of
 // lambda^{s+1} too when the gradient is wanted (no bed-friction terms), and
@@ -226,35 +220,61 @@ __device__ __forceinline__ void coef_reduce(RedDev* red, double minev, double hm
   }
 }
 
-// Coefficient pass on large meshes, one workgroup per mark block: forward
-// slopes -> kact (getcoef.f) and the per-instance CFL min / hmax reduction
-// (get_coef_and_eigen.C:29-180).  The block's wet cells are listed in LDS and
-// worked off 256 at a time, so a block that a front crosses takes as many
-// rounds as it has wet cells, not one for each of its four tiles (64 members,
-// 5.8 M cells: 15.5 us, a round per tile 23 us).
+// First pass on large meshes, one workgroup per mark block.
+//
+// Coefficients: forward slopes -> kact (getcoef.f) and the per-instance CFL
+// min / hmax reduction (get_coef_and_eigen.C:29-180).  The block's wet cells
+// are listed in LDS and worked off 256 at a time, so a block that a front
+// crosses takes as many rounds as it has wet cells, not one for each of its
+// four tiles.
+//
+// Tiles for the update: a tile whose cells and side neighbours all hold h <
+// tiny has every face flux zero (the physical flux is zero below tiny and
+// riemannflux of two such sides is zero) and no source terms (update_states
+// adds them only above tiny); it goes on the dry list, unless the marks show
+// that input and output hold +0.0 already.  Every other tile goes on the full
+// list.  (No dt is needed for that: see k_update for one that is not finite.)
+// Both jobs read h of the same blocks; in two passes they took 12.4 + 12.4 us
+// of a 2048 x 2048 step and 15.5 + 20 us on 64 members of 5.8 M cells, in one
+// 18 and 24 us.
 template <int TX>
 __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *a.tile_count = 0;  // the update's list starts empty
+  constexpr int TY = BLOCK / TX;
   // (the block table is indexed by mark word)
-  if (a.mk_in && coef_skip(a.mk_in, (int)blockIdx.x)) return;
   const BlockDev B = a.blocks[blockIdx.x];
+  if (a.mk_in && update_skip(a.mk_in, a.mk_out, B)) return;
   __shared__ int s_n;
+  __shared__ unsigned s_wet;
   __shared__ unsigned short s_cell[4 * BLOCK];
   __shared__ double s_h[4 * BLOCK];
-  if (threadIdx.x == 0) s_n = 0;
+  if (threadIdx.x == 0) { s_n = 0; s_wet = 0u; }
   Cell q[4];
   block_cells<TX>(B, q);
-  // a tile the marks show to hold +0.0 has h < tiny everywhere: nothing to
-  // read or write
-  const uint32_t zin = (a.mk_in && a.zbytes) ? a.mk_in[blockIdx.x] : 0u;
+  // tiles of the block holding +0.0 in the input / output state (mark bytes):
+  // their h is not read
+  const uint32_t zin = (a.mk_in && a.zbytes) ? a.mk_in[B.mw] : 0u;
+  const uint32_t zout = (a.mk_out && a.zbytes) ? a.mk_out[B.mw] : 0u;
+  const long long nx = B.nx;
+  const int tx = (int)(threadIdx.x % TX), ty = (int)(threadIdx.x / TX);
+  double h[4];
+  unsigned flows = 0u;  // tiles with a cell or side neighbour not below tiny
 #pragma unroll
   for (int b = 0; b < 4; b++)
-    if ((zin >> (8 * b)) & 1u) q[b].act = false;
-  double h[4];
+    h[b] = q[b].act && !((zin >> (8 * b)) & 1u) ? a.U.h[q[b].c] : 0.;
 #pragma unroll
-  for (int b = 0; b < 4; b++) h[b] = q[b].act ? a.U.h[q[b].c] : 0.;
+  for (int b = 0; b < 4; b++) {
+    if (!q[b].act) continue;
+    const long long c = q[b].c;
+    bool w = !(h[b] < a.tiny);
+    if (tx == 0 && q[b].hasW) w = w || !(a.U.h[c - 1] < a.tiny);
+    if (tx == TX - 1 && q[b].hasE) w = w || !(a.U.h[c + 1] < a.tiny);
+    if (ty == 0 && q[b].hasS) w = w || !(a.U.h[c - nx] < a.tiny);
+    if (ty == TY - 1 && q[b].hasN) w = w || !(a.U.h[c + nx] < a.tiny);
+    if (w) flows |= 1u << b;
+  }
   const InstDev I = a.inst[B.inst];
-  __syncthreads();  // s_n set
+  __syncthreads();  // s_n, s_wet set
+  if (flows) atomicOr(&s_wet, flows);
   int nwet = 0, nshort = 0;
   const int lane = threadIdx.x % 64;
 #pragma unroll
@@ -271,7 +291,7 @@ __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
         s_h[k] = h[b];
       }
     }
-    if (!q[b].act) continue;
+    if (!q[b].act || ((zin >> (8 * b)) & 1u)) continue;
     if (wet) {
       nwet++;
     } else {
@@ -290,7 +310,35 @@ __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
     const int cnt = (int)wave_sum((double)nshort);
     if (threadIdx.x % 64 == 0 && cnt) atomicAdd(a.short_cells, (unsigned long long)cnt);
   }
-  __syncthreads();  // the list is complete
+  __syncthreads();  // the wet cells and tiles are complete
+  if (a.copy_dry) {
+    // dry_cell for a dt known to be zero or positive: the state, h clamped
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      if (!q[b].act || ((s_wet >> b) & 1u)) continue;
+      const long long c = q[b].c;
+      const double hu = a.U.hu[c], hv = a.U.hv[c];
+      if (!isfinite(h[b]) || !isfinite(hu) || !isfinite(hv)) atomicOr(a.err, 1);
+      a.h_out[c] = (h[b] < 0.) ? 0. : h[b];
+      a.hu_out[c] = hu;
+      a.hv_out[c] = hv;
+    }
+  }
+  if (threadIdx.x == 0) {
+    unsigned full = s_wet, dry = 0u;
+#pragma unroll
+    for (int b = 0; b < 4 && !a.copy_dry; b++)
+      if (B.tile[b] >= 0 && !((full >> b) & 1u) && !(((zin & zout) >> (8 * b)) & 1u)) dry |= 1u << b;
+    int kf = full ? atomicAdd(a.tile_count, __popc(full)) : 0;
+    int kd = dry ? atomicAdd(a.tile_count + 1, __popc(dry)) : 0;
+    // the full list grows from the front of the array, the dry one from its
+    // end: a tile is on at most one of them
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      if ((full >> b) & 1u) a.tile_list[kf++] = tile_ref<TX>(B, b);
+      if ((dry >> b) & 1u) a.tile_list[a.ntiles - 1 - kd++] = tile_ref<TX>(B, b);
+    }
+  }
   const int n = s_n;
   double minev = HUGE_VAL, hmax = 0.;
   for (int k = (int)threadIdx.x; k < n; k += BLOCK)
@@ -527,110 +575,18 @@ __device__ __forceinline__ void face_flux(const FaceLds<TX>& L, int dir, int l, 
   }
 }
 
-// Update pass 1 (one workgroup per mark block, one cell of each of its four
-// tiles per thread): a tile whose cells and side neighbours all hold
-// h < tiny has every face flux zero (the physical flux is zero below tiny
-// and riemannflux of two such sides is zero) and no source terms
-// (update_states adds them only above tiny); its cells get update_states'
-// own arithmetic with zero fluxes, bit for bit, here.  Every other tile is
-// appended to the list pass 2 walks.  A tile the input marks show to hold
-// +0.0 is not read (its cells are +0.0); when it is dry, its output tile
-// already holds +0.0 and dt is finite, the formula gives +0.0 again and
-// nothing is written.
-template <int TX>
-__global__ __launch_bounds__(BLOCK) void k_update_classify(StepArgs a) {
-  constexpr int TY = BLOCK / TX;
-  const BlockDev B = a.blocks[blockIdx.x];
-  const double dt = step_dt(a, B.inst, B.x0 == 0 && B.y0 == 0);
-  if (a.mk_in && update_skip(a.mk_in, a.mk_out, B, dt)) return;
-  const InstDev I = a.inst[B.inst];
-  // tiles of the block holding +0.0 in the input / output state (mark bytes)
-  const uint32_t zin = (a.mk_in && a.zbytes) ? a.mk_in[B.mw] : 0u;
-  const uint32_t zout = (a.mk_out && a.zbytes && isfinite(dt)) ? a.mk_out[B.mw] : 0u;
-  __shared__ unsigned s_wet, s_nz;
-  if (threadIdx.x == 0) { s_wet = 0u; s_nz = 0u; }
-  Cell q[4];
-  block_cells<TX>(B, q);
-  const long long nx = I.nx;
-  const int tx = (int)(threadIdx.x % TX), ty = (int)(threadIdx.x / TX);
-  unsigned wet = 0u;
-  // h of every cell not known to be +0.0 (the wet test); the momenta only
-  // once the tile is known to be dry
-  double out[4][3];
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    if (!q[b].act) continue;
-    const long long c = q[b].c;
-    out[b][0] = out[b][1] = out[b][2] = 0.;
-    if (!((zin >> (8 * b)) & 1u)) out[b][0] = a.U.h[c];
-    bool w = !(out[b][0] < a.tiny);
-    if (tx == 0 && q[b].hasW) w = w || !(a.U.h[c - 1] < a.tiny);
-    if (tx == TX - 1 && q[b].hasE) w = w || !(a.U.h[c + 1] < a.tiny);
-    if (ty == 0 && q[b].hasS) w = w || !(a.U.h[c - nx] < a.tiny);
-    if (ty == TY - 1 && q[b].hasN) w = w || !(a.U.h[c + nx] < a.tiny);
-    if (w) wet |= 1u << b;
-  }
-  __syncthreads();  // s_wet, s_nz set
-  if (wet) atomicOr(&s_wet, wet);
-  __syncthreads();
-  const unsigned W = s_wet;
-  if (threadIdx.x == 0 && W) {
-    int k = atomicAdd(a.tile_count, __popc(W));
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-      if ((W >> b) & 1u) a.tile_list[k++] = tile_ref<TX>(B, b);
-  }
-  // the momenta of the dry tiles that hold something (a wet tile's cells are
-  // read again by the full path)
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    if (!q[b].act || ((W >> b) & 1u) || ((zin >> (8 * b)) & 1u)) continue;
-    out[b][1] = a.U.hu[q[b].c];
-    out[b][2] = a.U.hv[q[b].c];
-  }
+// The dry tile's cells: update_states' own arithmetic with zero fluxes, bit for
+// bit (U - dtdx (0 - 0) - dtdy (0 - 0), h clamped at 0; inf and NaN included).
+// Returns whether the new state is +0.0.
+__device__ __forceinline__ bool dry_cell(const StepArgs& a, const InstDev& I, double dt,
+                                         double h, double hu, double hv, double out[3]) {
   const double dtdx = dt / I.dx, dtdy = dt / I.dy, zero = 0.;
-  unsigned nz = 0u;
-  int nshort = 0;
+  out[0] = h; out[1] = hu; out[2] = hv;
 #pragma unroll
-  for (int b = 0; b < 4; b++) {
-    if (!q[b].act || ((W >> b) & 1u)) continue;
-    nshort++;
-#pragma unroll
-    for (int v = 0; v < 3; v++)
-      out[b][v] = out[b][v] - dtdx * (zero - zero) - dtdy * (zero - zero);
-    if (out[b][0] < 0.) out[b][0] = 0;
-    if (!isfinite(out[b][0]) || !isfinite(out[b][1]) || !isfinite(out[b][2])) atomicOr(a.err, 1);
-    if (!bitzero3(out[b][0], out[b][1], out[b][2])) nz |= 1u << b;
-  }
-  if (a.short_cells) {
-    const int cnt = (int)wave_sum((double)nshort);
-    if (threadIdx.x % 64 == 0 && cnt) atomicAdd(a.short_cells, (unsigned long long)cnt);
-  }
-  // the marks' reduction before the stores: no barrier waits on them
-  if (a.mk_out) {
-    if (nz) atomicOr(&s_nz, nz);
-    __syncthreads();
-  }
-  // a dry tile of +0.0 whose output already holds +0.0 (finite dt): the
-  // formula gives +0.0 again, nothing to write
-  unsigned keep = 0u;
-#pragma unroll
-  for (int b = 0; b < 4; b++)
-    if (((zin & zout) >> (8 * b)) & 1u) keep |= 1u << b;
-#pragma unroll
-  for (int b = 0; b < 4; b++) {
-    if (!q[b].act || (((W | keep) >> b) & 1u)) continue;
-    a.h_out[q[b].c] = out[b][0];
-    a.hu_out[q[b].c] = out[b][1];
-    a.hv_out[q[b].c] = out[b][2];
-  }
-  if (a.mk_out && threadIdx.x == 0) {
-    const unsigned NZ = s_nz;
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-      if (B.tile[b] >= 0 && !(((W | keep) >> b) & 1u))
-        mark_byte_store(a.mk_out, B.mw, b, !((NZ >> b) & 1u));
-  }
+  for (int v = 0; v < 3; v++) out[v] = out[v] - dtdx * (zero - zero) - dtdy * (zero - zero);
+  if (out[0] < 0.) out[0] = 0;
+  if (!isfinite(out[0]) || !isfinite(out[1]) || !isfinite(out[2])) atomicOr(a.err, 1);
+  return bitzero3(out[0], out[1], out[2]);
 }
 
 // What the corrector reads of a tile's own cell besides the faces.
@@ -745,14 +701,8 @@ __device__ __forceinline__ void update_tile(const StepArgs& a, const TileRef& t,
                         (a.mk_out[t.mw] >> (8 * mark_byte<TX>(t))) & 1u;
       bool z = true;
       if (q.act) {
-        const double dtdx = dt / I.dx, dtdy = dt / I.dy, zero = 0.;
-        double out[3] = {u.h, u.hu, u.hv};
-#pragma unroll
-        for (int v = 0; v < 3; v++)
-          out[v] = out[v] - dtdx * (zero - zero) - dtdy * (zero - zero);
-        if (out[0] < 0.) out[0] = 0;
-        if (!isfinite(out[0]) || !isfinite(out[1]) || !isfinite(out[2])) atomicOr(a.err, 1);
-        z = bitzero3(out[0], out[1], out[2]);
+        double out[3];
+        z = dry_cell(a, I, dt, u.h, u.hu, u.hv, out);
         if (!keep) {
           a.h_out[q.c] = out[0];
           a.hu_out[q.c] = out[1];
@@ -803,14 +753,47 @@ __device__ __forceinline__ void update_tile(const StepArgs& a, const TileRef& t,
   if (a.mk_out) mark_store<TX>(a.mk_out, t, __syncthreads_and(z));
 }
 
+// A listed dry tile.
+template <int TX, int NT>
+__device__ __forceinline__ void update_dry_tile(const StepArgs& a, const TileRef& t, double dt) {
+  const InstDev I = a.inst[t.inst];
+  const Cell q = cell_of<TX>(t);
+  const bool act = q.act && threadIdx.x < BLOCK;
+  bool z = true;
+  if (act) {
+    double out[3];
+    z = dry_cell(a, I, dt, a.U.h[q.c], a.U.hu[q.c], a.U.hv[q.c], out);
+    a.h_out[q.c] = out[0];
+    a.hu_out[q.c] = out[1];
+    a.hv_out[q.c] = out[2];
+  }
+  if (a.short_cells) {
+    const int cnt = __syncthreads_count(act);
+    if (threadIdx.x == 0) atomicAdd(a.short_cells, (unsigned long long)cnt);
+  }
+  if (a.mk_out) mark_store<TX>(a.mk_out, t, __syncthreads_and(z));
+}
+
+// Second pass on large meshes: a fixed grid walks the full list, then the dry
+// one.  The first workgroups also keep the members' records (step_dt); a dt
+// that is not finite makes every cell so, the unlisted ones too, so it is
+// reported here as the state it would give is.
 template <int TX>
 __global__ __launch_bounds__(record_threads<TX>(), 5) void k_update(StepArgs a) {
   __shared__ FaceLds<TX> L;
-  const int n = *a.tile_count;
+  const int n = a.tile_count[0], nd = a.tile_count[1];
+  if (blockIdx.x == 0 && threadIdx.x < 2) a.count_next[threadIdx.x] = 0;
+  for (int b = (int)blockIdx.x; b < a.ninst; b += (int)gridDim.x)
+    if (!isfinite(step_dt(a, b, true)) && threadIdx.x == 0) atomicOr(a.err, 1);
   for (int i = (int)blockIdx.x; i < n; i += (int)gridDim.x) {
     const TileRef t = a.tile_list[list_band(i, n)];
-    update_tile<TX, record_threads<TX>(), false>(a, t, a.dt_rec[(long long)t.inst * a.max_steps + a.step], L);
+    update_tile<TX, record_threads<TX>(), false>(a, t, step_dt(a, t.inst, false), L);
     __syncthreads();  // LDS reused by the next tile
+  }
+  // (from the grid's end: its last workgroups have the fewest full tiles)
+  for (int i = (int)(gridDim.x - 1 - blockIdx.x); i < nd; i += (int)gridDim.x) {
+    const TileRef t = a.tile_list[a.ntiles - 1 - i];
+    update_dry_tile<TX, record_threads<TX>()>(a, t, step_dt(a, t.inst, false));
   }
 }
 
@@ -825,7 +808,7 @@ __global__ __launch_bounds__(face_threads<TX>()) void k_update_tile(StepArgs a) 
   const int tile = tile_of(a);
   const TileDev t = a.tiles[tile];
   const double dt = step_dt(a, t.inst, t.x0 == 0 && t.y0 == 0);
-  if (a.mk_in && update_skip(a.mk_in, a.mk_out, t, dt)) return;
+  if (a.mk_in && isfinite(dt) && update_skip(a.mk_in, a.mk_out, t)) return;
   update_tile<TX, face_threads<TX>(), true>(a, ref_of(t, tile), dt, L);
 }
 
@@ -1537,6 +1520,7 @@ template <int TX, bool DPHI>
 __global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint(AdjArgs a) {
   __shared__ DualLds<TX, DPHI> L;
   const int n = *a.tile_count;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.count_next = 0;
   for (int i = (int)blockIdx.x; i < n; i += (int)gridDim.x) {
     adjoint_tile<TX, DPHI, false>(a, a.tile_list[list_band(i, n)], L);
     __syncthreads();  // LDS reused by the next tile
@@ -1572,18 +1556,13 @@ void launch_coef(const StepArgs& a, bool reduce, hipStream_t s) {
 void launch_dt(const StepArgs& a, int ninst, hipStream_t s) {
   hipLaunchKernelGGL(k_dt, dim3((ninst + 63) / 64), dim3(64), 0, s, a, ninst);
 }
-// classify every tile (skipped by the marks, short path written, or
-// listed), then a fixed grid walks the list with the full path; the
-// coefficient pass emptied the list
 void launch_update(const StepArgs& a, hipStream_t s) {
   const int g = a.by_tile || a.ntiles < LIST_GRID ? a.ntiles : LIST_GRID;
 #define TG_UPD(TX)                                                                             \
   if (a.by_tile)                                                                               \
     hipLaunchKernelGGL(k_update_tile<TX>, dim3(g), dim3(face_threads<TX>()), 0, s, a);         \
-  else {                                                                                       \
-    hipLaunchKernelGGL(k_update_classify<TX>, dim3(a.nblocks), dim3(BLOCK), 0, s, a);          \
-    hipLaunchKernelGGL(k_update<TX>, dim3(g), dim3(record_threads<TX>()), 0, s, a);            \
-  }
+  else                                                                                         \
+    hipLaunchKernelGGL(k_update<TX>, dim3(g), dim3(record_threads<TX>()), 0, s, a)
   switch (SHAPE_TX[a.shape]) {
     case 64: TG_UPD(64); break;
     case 32: TG_UPD(32); break;
@@ -1592,10 +1571,7 @@ void launch_update(const StepArgs& a, hipStream_t s) {
 #undef TG_UPD
 }
 void launch_adjoint(const AdjArgs& a, hipStream_t s) {
-  if (!a.by_tile) {
-    launch_zero(a.tile_count, sizeof(int), s);
-    TG_LAUNCH_TX(a.shape, k_adjoint_classify, dim3(a.nblocks), s, a);
-  }
+  if (!a.by_tile) TG_LAUNCH_TX(a.shape, k_adjoint_classify, dim3(a.nblocks), s, a);
   const dim3 g(a.by_tile || a.ntiles < ADJ_GRID ? a.ntiles : ADJ_GRID), b(ADJ_THREADS);
 #define TG_ADJ(TX, DPHI)                                                            \
   if (a.by_tile) hipLaunchKernelGGL((k_adjoint_tile<TX, DPHI>), g, b, 0, s, a);     \

@@ -51,7 +51,7 @@ TileDev g_tiles[NA_MAX_TILES];
 BlockDev g_blocks[NA_MAX_BLOCKS];
 struct Misc {
   double dt_rec, time, clock[2];
-  int err, tile_count;
+  int err, tile_count[2], count_next[2];
 };
 
 int device_scratch(int device, unsigned char** out) {
@@ -156,7 +156,7 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   g_inst.eps = prm->epsilon; g_inst.gscale = prm->gravity_scale;
   g_inst.maxtime = prm->maxtime; g_inst.nextoutput = prm->nextoutput;
   g_inst.nextsave = prm->nextsave;
-  const Misc misc{0.0, time, {time, 0.0}, 0, 0};
+  const Misc misc{0.0, time, {time, 0.0}, 0, {0, 0}, {0, 0}};
 
   NA_CHK(hipMemcpyAsync(base + OFF_INST, &g_inst, sizeof(InstDev), hipMemcpyHostToDevice, s));
   NA_CHK(hipMemcpyAsync(base + OFF_MISC, &misc, sizeof(Misc), hipMemcpyHostToDevice, s));
@@ -184,6 +184,7 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.clock = md->clock;
   a.fold = 1;
   a.by_tile = ntiles <= TILE_LAUNCH_MAX ? 1 : 0;
+  a.copy_dry = time <= prm->maxtime && time <= prm->nextoutput && time <= prm->nextsave;
   a.max_steps = 1;
   a.step = 0;
   a.ft = (step < cfg->frict_tiny_switch) ? cfg->frict_tiny_early : cfg->frict_tiny_late;
@@ -193,7 +194,9 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.err = &md->err;
   a.active = nullptr;
   a.tile_list = (TileRef*)(base + OFF_LIST);
-  a.tile_count = &md->tile_count;
+  a.tile_count = md->tile_count;
+  a.count_next = md->count_next;
+  a.ninst = 1;
   a.mk_in = nullptr;   // no zero marks: every tile is classified from its cells
   a.mk_out = nullptr;
   a.short_cells = nullptr;
