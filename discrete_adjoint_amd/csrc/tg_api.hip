@@ -608,6 +608,9 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
     a.mk_in = marks_of(ctx, in);
     a.mk_out = marks_of(ctx, out);
     a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[1]] == ctx->mk_tx[0];
+    a.fold = compute_dt;
+    a.red = ctx->red + (s & 1) * ctx->ninst;
+    a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst;
     if (ctx->leaves) {
       a.mat = ctx->mat_d;
       a.mtab = ctx->mtab_d;
@@ -616,7 +619,6 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
       inst_mark(ctx, 0, true);
       launch_leaf_coef(a, ctx->leaf, compute_dt, ctx->stream);
       inst_mark(ctx, 0, false);
-      if (compute_dt) launch_dt(a, 1, ctx->stream);
       a.active = inst_counter(ctx, 1, true);
       a.short_cells = inst_short(ctx, 1, true);
       inst_mark(ctx, 1, true);
@@ -624,9 +626,6 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
       inst_mark(ctx, 1, false);
       return;
     }
-    a.fold = compute_dt;
-    a.red = ctx->red + (s & 1) * ctx->ninst;
-    a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst;
     const int first = first_variant_of(ctx);
     use_tiles(ctx, first, a);
     a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[first]] == ctx->mk_tx[0];

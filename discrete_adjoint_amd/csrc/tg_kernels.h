@@ -215,6 +215,45 @@ struct StepArgs {
   int zbytes;
 };
 
+// dt = 0.5 * min(0.5 * min(dx / ev), 0.9 * sqrt(hmax eps Gs / 9.8)) clamped as
+// TimeProps::incrtime does (properties.h:397-410)
+__device__ __forceinline__ double cfl_dt(const StepArgs& a, const InstDev& I, const RedDev& R,
+                                         double time) {
+  const double min_ev = __longlong_as_double((long long)R.min_ev), hmax = __longlong_as_double((long long)R.hmax);
+  const double dt0 = a.cfl_inner * min_ev;
+  const double dt1 = -0.9 * sqrt(hmax * I.eps * I.gscale / 9.8);
+  const double m = (dt0 > -dt1) ? -dt1 : dt0;
+  double dt = a.cfl_outer * m;
+  if (dt == 0.0) dt = 0.5 * HUGE_VAL;
+  if (time + dt > I.nextoutput) dt = I.nextoutput - time;
+  if (time + dt > I.nextsave) dt = I.nextsave - time;
+  if (time + dt > I.maxtime) dt = I.maxtime - time;
+  return dt;
+}
+
+// The dt of member b at this step.  a.fold: it is made here, by every workgroup
+// alike, from the reduction cells the coefficient pass filled (k_dt's
+// arithmetic), instead of in a launch of its own; one workgroup of the member
+// (`own`) also records it, moves the member's clock on and clears the
+// reduction cells of the next step, which nothing else touches meanwhile
+// (steps alternate between two sets, and the clock has a slot per step).
+// Otherwise it was prescribed or recorded before.
+__device__ __forceinline__ double step_dt(const StepArgs& a, int b, bool own) {
+  double* rec = a.dt_rec + (long long)b * a.max_steps + a.step;
+  if (!a.fold) return *rec;
+  const InstDev& I = a.inst[b];
+  const RedDev R = a.red[b];
+  double* clock = a.clock + (long long)b * (a.max_steps + 1) + a.step;
+  const double dt = cfl_dt(a, I, R, *clock);
+  if (own && threadIdx.x == 0) {
+    *rec = dt;
+    clock[1] = a.time[b] = *clock + dt;
+    a.red_next[b].min_ev = (unsigned long long)__double_as_longlong(10000000.);
+    a.red_next[b].hmax = 0ull;
+  }
+  return dt;
+}
+
 struct AdjArgs {
   const InstDev* inst;
   const TileDev* tiles;

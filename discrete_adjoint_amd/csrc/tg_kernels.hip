@@ -452,22 +452,6 @@ __global__ void k_member_fill(const uint32_t* __restrict__ src, uint32_t* __rest
     for (long long i = t0; i < nmw; i += stride) mk[mw0 + i] = 0u;
 }
 
-// dt = 0.5 * min(0.5 * min(dx / ev), 0.9 * sqrt(hmax eps Gs / 9.8)) clamped as
-// TimeProps::incrtime does (properties.h:397-410)
-__device__ __forceinline__ double cfl_dt(const StepArgs& a, const InstDev& I, const RedDev& R,
-                                         double time) {
-  const double min_ev = bitsd(R.min_ev), hmax = bitsd(R.hmax);
-  const double dt0 = a.cfl_inner * min_ev;
-  const double dt1 = -0.9 * sqrt(hmax * I.eps * I.gscale / 9.8);
-  const double m = (dt0 > -dt1) ? -dt1 : dt0;
-  double dt = a.cfl_outer * m;
-  if (dt == 0.0) dt = 0.5 * HUGE_VAL;
-  if (time + dt > I.nextoutput) dt = I.nextoutput - time;
-  if (time + dt > I.nextsave) dt = I.nextsave - time;
-  if (time + dt > I.maxtime) dt = I.maxtime - time;
-  return dt;
-}
-
 __global__ void k_dt(StepArgs a, int ninst) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= ninst) return;
@@ -477,29 +461,6 @@ __global__ void k_dt(StepArgs a, int ninst) {
   a.dt_rec[(long long)b * a.max_steps + a.step] = dt;
   a.red[b].min_ev = dbits(10000000.);
   a.red[b].hmax = dbits(0.);
-}
-
-// The dt of member b at this step.  a.fold: it is made here, by every workgroup
-// alike, from the reduction cells the coefficient pass filled (k_dt's
-// arithmetic), instead of in a launch of its own; one workgroup of the member
-// (`own`) also records it, moves the member's clock on and clears the
-// reduction cells of the next step, which nothing else touches meanwhile
-// (steps alternate between two sets, and the clock has a slot per step).
-// Otherwise it was prescribed or recorded before.
-__device__ __forceinline__ double step_dt(const StepArgs& a, int b, bool own) {
-  double* rec = a.dt_rec + (long long)b * a.max_steps + a.step;
-  if (!a.fold) return *rec;
-  const InstDev& I = a.inst[b];
-  const RedDev R = a.red[b];
-  double* clock = a.clock + (long long)b * (a.max_steps + 1) + a.step;
-  const double dt = cfl_dt(a, I, R, *clock);
-  if (own && threadIdx.x == 0) {
-    *rec = dt;
-    clock[1] = a.time[b] = *clock + dt;
-    a.red_next[b].min_ev = dbits(10000000.);
-    a.red_next[b].hmax = dbits(0.);
-  }
-  return dt;
 }
 
 // Face records of one tile: every face flux and every one-sided difference
@@ -1246,15 +1207,25 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_classify(AdjArgs a) {
   }
   Cell q[4];
   block_cells<TX>(B, q);
+  // every load in flight at once (a test between them would make each wait for
+  // the one before)
+  double u[4], l[4][3];
+#pragma unroll
+  for (int b = 0; b < 4; b++) {
+    u[b] = l[b][0] = l[b][1] = l[b][2] = 0.;
+    if (!q[b].act || ((zvoid >> (8 * b)) & 1u)) continue;
+    const long long c = q[b].c;
+    u[b] = a.U.h[c];
+    if (a.dphi_part) {
+      l[b][0] = a.lam_next.h[c]; l[b][1] = a.lam_next.hu[c]; l[b][2] = a.lam_next.hv[c];
+    }
+  }
   unsigned busy = 0u;
 #pragma unroll
   for (int b = 0; b < 4; b++) {
-    if (!q[b].act || ((zvoid >> (8 * b)) & 1u)) continue;
-    const long long c = q[b].c;
-    bool u = a.U.h[c] != 0.;
-    if (a.dphi_part)
-      u = u || !(a.lam_next.h[c] == 0. && a.lam_next.hu[c] == 0. && a.lam_next.hv[c] == 0.);
-    if (u) busy |= 1u << b;
+    // (bitwise on purpose: no branch between the operands)
+    const bool nz = (u[b] != 0.) | !((l[b][0] == 0.) & (l[b][1] == 0.) & (l[b][2] == 0.));
+    if (nz) busy |= 1u << b;
   }
   __syncthreads();  // s_busy set
   if (busy) atomicOr(&s_busy, busy);

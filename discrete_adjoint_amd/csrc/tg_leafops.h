@@ -109,6 +109,35 @@ __device__ __forceinline__ Hfv leaf_hfv(const Fields& U, const double* k, const 
   return hfv_fwd(dir, U.h[c], U.hu[c], U.hv[c], k[c], gz[c], tiny);
 }
 
+// Brings what the passes read of leaf c's neighbours -- the state, two more
+// fields (null: none) and the centres -- towards the CU in two round trips,
+// the neighbour indexes and then everything at once; side by side the passes
+// would wait for each of up to eight neighbours in turn.  The values themselves
+// are read again where they are used (no registers are held).
+__device__ __forceinline__ void touch(double v) { asm volatile("" ::"v"(v)); }
+__device__ __forceinline__ void touch_neighbours(const LeafDev& L, const Fields& U,
+                                                 const double* f, const double* g, int c,
+                                                 uint32_t meta) {
+  int nb[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) nb[k] = slot_present(meta, k) ? L.nbr[k * L.n + c] : c;
+  double v[8][5], x[4];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    v[k][0] = U.h[nb[k]]; v[k][1] = U.hu[nb[k]]; v[k][2] = U.hv[nb[k]];
+    v[k][3] = f ? f[nb[k]] : 0.;
+    v[k][4] = g ? g[nb[k]] : 0.;
+  }
+#pragma unroll
+  for (int s = 0; s < 4; s++) x[s] = L.xc[(size_t)((s & 1) ? 0 : 1) * L.n + nb[s]];
+#pragma unroll
+  for (int k = 0; k < 8; k++)
+#pragma unroll
+    for (int i = 0; i < 5; i++) touch(v[k][i]);
+#pragma unroll
+  for (int s = 0; s < 4; s++) touch(x[s]);
+}
+
 // Flux of side s of leaf c (not a boundary side): HLL with the minus-side
 // leaf on the left; half the sum of both small faces on a side with two
 // finer neighbours.

@@ -82,6 +82,7 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_coef(StepArgs a, LeafDev L, int 
       const uint32_t meta = L.meta[c];
       const double hu = a.U.hu[c], hv = a.U.hv[c];
       double hx = 0., hux = 0., hy = 0., hvy = 0.;
+      touch_neighbours(L, a.U, nullptr, nullptr, c, meta);
       if (!touches_boundary(meta)) {
         const DirNb qx = dir_nb(L, c, meta, 0), qy = dir_nb(L, c, meta, 1);
         hx = lslope_fwd(a.U.h, c, qx, a.gamma, a.tiny);
@@ -137,19 +138,24 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_coef(StepArgs a, LeafDev L, int 
 // fluxes and no sources: update_states' own arithmetic with zero fluxes.
 __device__ __forceinline__ bool leaf_dry(const StepArgs& a, const LeafDev& L, int c,
                                         uint32_t meta) {
-  if (!(a.U.h[c] < a.tiny)) return false;
+  // all indexes, then all depths (an early exit would make each neighbour wait
+  // for the one before)
+  int nb[8];
 #pragma unroll
-  for (int k = 0; k < 8; k++)
-    if (slot_present(meta, k) && !(a.U.h[L.nbr[k * L.n + c]] < a.tiny)) return false;
-  return true;
+  for (int k = 0; k < 8; k++) nb[k] = slot_present(meta, k) ? L.nbr[k * L.n + c] : c;
+  bool dry = a.U.h[c] < a.tiny;
+#pragma unroll
+  for (int k = 0; k < 8; k++) dry = dry & (a.U.h[nb[k]] < a.tiny);
+  return dry;
 }
 
 // One leaf of the update: update_states with its face fluxes.
 __device__ __forceinline__ void leaf_update_full(const StepArgs& a, const LeafDev& L, int c,
-                                                 uint32_t meta, double out[3]) {
+                                                 uint32_t meta, double dt, double out[3]) {
   const InstDev I = a.inst[0];
   const double h = a.U.h[c], hu = a.U.hu[c], hv = a.U.hv[c];
   double hx = 0., hvx = 0., hy = 0., huy = 0.;
+  touch_neighbours(L, a.U, a.kact, a.S.gz, c, meta);
   if (!touches_boundary(meta)) {
     const DirNb qx = dir_nb(L, c, meta, 0), qy = dir_nb(L, c, meta, 1);
     hx = lslope_fwd(a.U.h, c, qx, a.gamma, a.tiny);
@@ -170,7 +176,6 @@ __device__ __forceinline__ void leaf_update_full(const StepArgs& a, const LeafDe
     if (kind_of(meta, s) == LEAF_BOUNDARY)
 #pragma unroll
       for (int v = 0; v < 3; v++) F[s][v] = F[(s + 2) & 3][v];
-  const double dt = a.dt_rec[a.step];
   const double dtdx = dt / L.cdx[c], dtdy = dt / L.cdx[L.n + c];
   const double prev[3] = {h, hu, hv};
   SrcInfo si;
@@ -184,7 +189,7 @@ __device__ __forceinline__ void leaf_update_full(const StepArgs& a, const LeafDe
 // U^s - dtdx*(0 - 0) - dtdy*(0 - 0) = +0.0 (finite dt): skipped when its
 // output chunk already holds +0.0.
 __global__ __launch_bounds__(BLOCK) void k_leaf_update(StepArgs a, LeafDev L) {
-  const double dt = a.dt_rec[a.step];
+  const double dt = step_dt(a, 0, blockIdx.x == 0);
   if (a.mk_in && a.mk_out[blockIdx.x] == MARK_FULL && isfinite(dt) &&
       chunk_nbhd_zero(a.mk_in, L, (int)blockIdx.x))
     return;
@@ -209,7 +214,7 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_update(StepArgs a, LeafDev L) {
     for (int v = 0; v < 3; v++) out[v] = out[v] - dtdx * (z - z) - dtdy * (z - z);
     if (out[0] < 0.) out[0] = 0;
   } else if (c < L.n) {
-    leaf_update_full(a, L, c, meta, out);
+    leaf_update_full(a, L, c, meta, dt, out);
   }
   if (c < L.n) {
     if (!isfinite(out[0]) || !isfinite(out[1]) || !isfinite(out[2])) atomicOr(a.err, 1);
@@ -252,6 +257,7 @@ __device__ __forceinline__ void leaf_dualk_wet(const AdjArgs& a, const LeafDev& 
   const uint32_t meta = L.meta[c];
   const double hu = a.U.hu[c], hv = a.U.hv[c];
   double hx = 0., hux = 0., hy = 0., hvy = 0.;
+  touch_neighbours(L, a.U, nullptr, nullptr, c, meta);
   if (!touches_boundary(meta)) {
     const DirNb qx = dir_nb(L, c, meta, 0), qy = dir_nb(L, c, meta, 1);
     hx = lslope_dual(a.U.h, c, qx, a.gamma, a.tiny, false).d;
@@ -495,10 +501,11 @@ __device__ __forceinline__ M3 side_pass(const AdjArgs& a, const LeafDev& L, cons
 // where this leaf sits in slot which_neighbor + 1: each block is multiplied
 // by this leaf's lambda^{s+1} here and its nine products are stored in that
 // reader's record slot, so the gather reads its own records in slot order.
-__global__ __launch_bounds__(BLOCK) void k_leaf_jac(AdjArgs a, LeafDev L, LeafBufs B) {
+__device__ __forceinline__ void leaf_jac_chunk(const AdjArgs& a, const LeafDev& L,
+                                               const LeafBufs& B, int chunk) {
   // void leaves among void neighbours only: no block to store
-  if (a.mk_U && chunk_nbhd_zero(a.mk_U, L, (int)blockIdx.x)) return;
-  const int c = blockIdx.x * BLOCK + threadIdx.x;
+  if (a.mk_U && chunk_nbhd_zero(a.mk_U, L, chunk)) return;
+  const int c = chunk * BLOCK + threadIdx.x;
   if (c >= L.n) return;
   const InstDev I = a.inst[0];
   JacCtx q;
@@ -509,12 +516,15 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_jac(AdjArgs a, LeafDev L, LeafBu
   // A void leaf among void neighbours stores no block (every block it would
   // store lands in the record of a leaf with h == 0).
   if (h == 0.) {
+    int nb[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) nb[k] = slot_present(q.meta, k) ? L.nbr[k * L.n + c] : c;
     bool any = false;
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-      if (slot_present(q.meta, k) && a.U.h[L.nbr[k * L.n + c]] != 0.) any = true;
+    for (int k = 0; k < 8; k++) any = any | (a.U.h[nb[k]] != 0.);
     if (!any) return;
   }
+  touch_neighbours(L, a.U, B.kd, a.S.gz, c, q.meta);
   const double hu = a.U.hu[c], hv = a.U.hv[c];
   q.h = h;
   q.lam[0] = a.lam_next.h[c];
@@ -599,12 +609,13 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_jac(AdjArgs a, LeafDev L, LeafBu
 // independent -- and lane 0 gathers the four and adds the source terms, so
 // each lane carries a quarter of the face work of the leaf's chain.
 constexpr int DPHI_LANES = 4;
-__global__ __launch_bounds__(BLOCK) void k_leaf_dphi(AdjArgs a, LeafDev L, LeafBufs B) {
+__device__ __forceinline__ void leaf_dphi_quarter(const AdjArgs& a, const LeafDev& L,
+                                                  const LeafBufs& B, int quarter) {
   constexpr int LPW = BLOCK / DPHI_LANES;  // leaves per workgroup
-  const int chunk = (int)blockIdx.x / DPHI_LANES;
+  const int chunk = quarter / DPHI_LANES;
   // lambda^{s+1} = +0.0 on the whole chunk: zero terms
   if (a.mk_lnext && a.mk_lnext[chunk] == MARK_FULL) return;
-  const int c = (int)blockIdx.x * LPW + (int)threadIdx.x / DPHI_LANES;
+  const int c = quarter * LPW + (int)threadIdx.x / DPHI_LANES;
   const int side = (int)threadIdx.x % DPHI_LANES;
   // lambda^{s+1}_c == 0 contributes a zero term
   const bool act = c < L.n && (a.lam_next.h[c] != 0. || a.lam_next.hu[c] != 0. ||
@@ -643,6 +654,19 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_dphi(AdjArgs a, LeafDev L, LeafB
     for (int k = 1; k < BLOCK / 64; k++) dphi += sp[k];
     atomicAdd(&a.dphi_part[chunk], dphi);  // the chunk's DPHI_LANES workgroups
   }
+}
+
+__global__ __launch_bounds__(BLOCK) void k_leaf_jac(AdjArgs a, LeafDev L, LeafBufs B) {
+  leaf_jac_chunk(a, L, B, (int)blockIdx.x);
+}
+// The Jacobian pass and the gradient term of the same step in one launch: they
+// read the same state and write different buffers, and each alone leaves most
+// of the chip waiting for one chain of loads (187 k leaves: 17 + 11 us apart).
+// The longer chains, the Jacobian's, are dispatched first.
+__global__ __launch_bounds__(BLOCK) void k_leaf_jac_dphi(AdjArgs a, LeafDev L, LeafBufs B,
+                                                         int nchunk) {
+  if ((int)blockIdx.x < nchunk) leaf_jac_chunk(a, L, B, (int)blockIdx.x);
+  else leaf_dphi_quarter(a, L, B, (int)blockIdx.x - nchunk);
 }
 
 // calc_adjoint_elem (calc_adjoint.C:76-157): the terms of slots 0..8 in
@@ -730,9 +754,10 @@ void launch_leaf_adjoint(const AdjArgs& a, const AdjArgs* next, bool dualk,
   const dim3 g(leaf_grid(L.n)), b(BLOCK);
   const int want_dk = a.dphi_part ? 1 : 0;
   if (dualk) hipLaunchKernelGGL(k_leaf_dualk, g, b, 0, s, a, L, B, want_dk);
-  hipLaunchKernelGGL(k_leaf_jac, g, b, 0, s, a, L, B);
+  const int nchunk = (int)leaf_grid(L.n);
   if (a.dphi_part)
-    hipLaunchKernelGGL(k_leaf_dphi, dim3(leaf_grid(L.n) * DPHI_LANES), b, 0, s, a, L, B);
+    hipLaunchKernelGGL(k_leaf_jac_dphi, dim3(nchunk * (1 + DPHI_LANES)), b, 0, s, a, L, B, nchunk);
+  else hipLaunchKernelGGL(k_leaf_jac, g, b, 0, s, a, L, B);
   if (next) hipLaunchKernelGGL(k_leaf_gather_dualk, g, b, 0, s, a, *next, L, B, want_dk);
   else hipLaunchKernelGGL(k_leaf_gather, g, b, 0, s, a, L, B);
 }
