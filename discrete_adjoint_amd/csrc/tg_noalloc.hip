@@ -13,7 +13,6 @@
 // mutex serialises the host side).
 #include <hip/hip_runtime.h>
 
-#include <cstring>
 #include <mutex>
 
 #include "../../include/tg.h"
@@ -45,10 +44,6 @@ __device__ __align__(256) unsigned char scratch[NA_BYTES];
 std::mutex g_mu;
 unsigned char* g_ptr[NA_MAX_DEVICES] = {};  // scratch's address on each device
 
-// host staging of the tables (static storage: nothing allocated per call)
-InstDev g_inst;
-TileDev g_tiles[NA_MAX_TILES];
-BlockDev g_blocks[NA_MAX_BLOCKS];
 struct Misc {
   double dt_rec, time, clock[2];
   int err, tile_count[2], count_next[2];
@@ -65,33 +60,41 @@ int device_scratch(int device, unsigned char** out) {
   return TG_OK;
 }
 
-// The tile / block tables of the 64x4 row-major variant for one nx x ny
-// member (as tg_set_mesh builds them for variant 0).
-void build_tables(int nx, int ny, int* ntiles, int* nblocks) {
-  const int TX = SHAPE_TX[0], TY = BLOCK / TX;
-  const int nsx = (nx + MARK_W - 1) / MARK_W, nsy = (ny + MARK_H - 1) / MARK_H;
-  int nt = 0;
-  for (int ty = 0; ty < ny; ty += TY)
-    for (int tx = 0; tx < nx; tx += TX) {
-      const int bx = tx / MARK_W, by = ty / MARK_H, mw = by * nsx + bx;
-      g_tiles[nt++] = TileDev{0, tx, ty, mw, bx > 0 ? mw - 1 : -1, bx + 1 < nsx ? mw + 1 : -1,
-                              by > 0 ? mw - nsx : -1, by + 1 < nsy ? mw + nsx : -1, nx, ny, 0};
+// The member's record, the step's words, the reduction cells and the tile and
+// block tables of the 64x4 row-major variant for one nx x ny member (as
+// tg_set_mesh builds them for variant 0), written by one launch whose arguments
+// carry what the host knows: the call copies nothing to the device (four copies
+// and a host loop over the tables took 40 us of a 64 x 64 call's 76 us).
+__global__ __launch_bounds__(256) void k_noalloc_setup(InstDev I, Misc m, InstDev* inst,
+                                                       Misc* misc, RedDev* red, TileDev* tiles,
+                                                       BlockDev* blocks, int ntx, int ntiles,
+                                                       int nblocks) {
+  constexpr int TX = SHAPE_TX[0], TY = BLOCK / TX, ROWS = MARK_H / TY;
+  static_assert(TX == MARK_W, "a mark block is a column of tiles");
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i == 0) {
+    *inst = I;
+    *misc = m;
+    for (int k = 0; k < 2; k++) {
+      red[k].min_ev = (unsigned long long)__double_as_longlong(10000000.);  // get_coef_and_eigen.C:35
+      red[k].hmax = 0ull;
     }
-  const int nb = nsx * nsy;
-  for (int by = 0; by < nsy; by++)
-    for (int bx = 0; bx < nsx; bx++) {
-      const int mw = by * nsx + bx;
-      g_blocks[mw] = BlockDev{0, mw, bx > 0 ? mw - 1 : -1, bx + 1 < nsx ? mw + 1 : -1,
-                              by > 0 ? mw - nsx : -1, by + 1 < nsy ? mw + nsx : -1,
-                              {-1, -1, -1, -1}, bx * MARK_W, by * MARK_H, nx, ny, 0};
-    }
-  for (int i = 0; i < nt; i++) {
-    const TileDev& t = g_tiles[i];
-    const int byte = ((t.y0 % MARK_H) / TY) * (MARK_W / TX) + (t.x0 % MARK_W) / TX;
-    g_blocks[t.mw].tile[byte] = i;
   }
-  *ntiles = nt;
-  *nblocks = nb;
+  const int nsx = I.nsx;
+  if (i < ntiles) {
+    const int bx = i % ntx, ty = i / ntx, by = ty / ROWS, mw = by * nsx + bx;
+    tiles[i] = TileDev{0, bx * TX, ty * TY, mw, bx > 0 ? mw - 1 : -1, bx + 1 < nsx ? mw + 1 : -1,
+                       by > 0 ? mw - nsx : -1, by + 1 < I.nsy ? mw + nsx : -1, I.nx, I.ny, 0};
+  }
+  if (i < nblocks) {
+    const int bx = i % nsx, by = i / nsx;
+    BlockDev B{0, i, bx > 0 ? i - 1 : -1, bx + 1 < nsx ? i + 1 : -1, by > 0 ? i - nsx : -1,
+               by + 1 < I.nsy ? i + nsx : -1, {-1, -1, -1, -1}, bx * MARK_W, by * MARK_H, I.nx,
+               I.ny, 0};
+    for (int k = 0; k < ROWS; k++)
+      if ((by * ROWS + k) * TY < I.ny) B.tile[k] = (by * ROWS + k) * ntx + bx;
+    blocks[i] = B;
+  }
 }
 
 int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_params* prm,
@@ -141,30 +144,28 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   int rc = device_scratch(cfg->device, &base);
   if (rc) return rc;
 
-  int ntiles = 0, nblocks = 0;
-  build_tables(blk->nx, blk->ny, &ntiles, &nblocks);
-  std::memset(&g_inst, 0, sizeof(g_inst));
-  g_inst.nx = blk->nx; g_inst.ny = blk->ny; g_inst.off = 0;
-  g_inst.nsx = (blk->nx + MARK_W - 1) / MARK_W;
-  g_inst.nsy = (blk->ny + MARK_H - 1) / MARK_H;
-  g_inst.soff = 0;
-  g_inst.dx = blk->dx; g_inst.dy = blk->dy;
-  g_inst.inv_dx = 1 / blk->dx; g_inst.inv_sx = 1 / (blk->dx + blk->dx);
-  g_inst.inv_dy = 1 / blk->dy; g_inst.inv_sy = 1 / (blk->dy + blk->dy);
-  g_inst.sin_int = prm->sin_int; g_inst.tan_bed = prm->tan_bed;
-  g_inst.kc1 = prm->kact_c1; g_inst.kroot = prm->kact_root; g_inst.dkroot = prm->dkroot_dphi;
-  g_inst.eps = prm->epsilon; g_inst.gscale = prm->gravity_scale;
-  g_inst.maxtime = prm->maxtime; g_inst.nextoutput = prm->nextoutput;
-  g_inst.nextsave = prm->nextsave;
+  constexpr int TX = SHAPE_TX[0], TY = BLOCK / TX;
+  InstDev I{};
+  I.nx = blk->nx; I.ny = blk->ny; I.off = 0;
+  I.nsx = (blk->nx + MARK_W - 1) / MARK_W;
+  I.nsy = (blk->ny + MARK_H - 1) / MARK_H;
+  I.soff = 0;
+  I.dx = blk->dx; I.dy = blk->dy;
+  I.inv_dx = 1 / blk->dx; I.inv_sx = 1 / (blk->dx + blk->dx);
+  I.inv_dy = 1 / blk->dy; I.inv_sy = 1 / (blk->dy + blk->dy);
+  I.sin_int = prm->sin_int; I.tan_bed = prm->tan_bed;
+  I.kc1 = prm->kact_c1; I.kroot = prm->kact_root; I.dkroot = prm->dkroot_dphi;
+  I.eps = prm->epsilon; I.gscale = prm->gravity_scale;
+  I.maxtime = prm->maxtime; I.nextoutput = prm->nextoutput;
+  I.nextsave = prm->nextsave;
   const Misc misc{0.0, time, {time, 0.0}, 0, {0, 0}, {0, 0}};
-
-  NA_CHK(hipMemcpyAsync(base + OFF_INST, &g_inst, sizeof(InstDev), hipMemcpyHostToDevice, s));
-  NA_CHK(hipMemcpyAsync(base + OFF_MISC, &misc, sizeof(Misc), hipMemcpyHostToDevice, s));
-  NA_CHK(hipMemcpyAsync(base + OFF_TILES, g_tiles, sizeof(TileDev) * ntiles,
-                        hipMemcpyHostToDevice, s));
-  NA_CHK(hipMemcpyAsync(base + OFF_BLOCKS, g_blocks, sizeof(BlockDev) * nblocks,
-                        hipMemcpyHostToDevice, s));
+  const int ntx = (blk->nx + TX - 1) / TX, ntiles = ntx * ((blk->ny + TY - 1) / TY);
+  const int nblocks = I.nsx * I.nsy;
   Misc* md = (Misc*)(base + OFF_MISC);
+  hipLaunchKernelGGL(k_noalloc_setup, dim3((ntiles + 255) / 256), dim3(256), 0, s, I, misc,
+                     (InstDev*)(base + OFF_INST), md, (RedDev*)(base + OFF_RED),
+                     (TileDev*)(base + OFF_TILES), (BlockDev*)(base + OFF_BLOCKS), ntx, ntiles,
+                     nblocks);
 
   StepArgs a{};
   a.inst = (const InstDev*)(base + OFF_INST);
@@ -201,7 +202,6 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.mk_out = nullptr;
   a.short_cells = nullptr;
 
-  launch_reset_red(a.red, 1, nullptr, nullptr, 0, s);
   launch_coef(a, true, s);
   launch_update(a, s);
   NA_CHK(hipGetLastError());
