@@ -28,7 +28,7 @@ struct SweepGraph {
   bool valid = false;
 };
 
-constexpr int NCOUNT = 6;
+constexpr int NCOUNT = 8;
 
 struct tg_ctx {
   tg_config cfg{};
@@ -89,11 +89,11 @@ struct tg_ctx {
   bool box_on = false;  // a region is set (it may hold no cell)
   long long box_version = 0;  // changes with every tg_set_maxh_region
   double* box_rec = nullptr;
-  RedDev* red = nullptr;     // 2 * ninst: the FP64 uniform steps alternate
+  RedDev* red = nullptr;     // 2 * ninst: steps alternate
   double* dt_rec = nullptr;  // ninst * max_steps
   double* time_d = nullptr;  // ninst
   // ninst * (max_steps + 1): each member's time before each recorded step of
-  // the FP64 uniform path; clock_at: the step whose slot is current (-1: none)
+  // a uniform mesh; clock_at: the step whose slot is current (-1: none)
   double* clock_d = nullptr;
   int clock_at = -1;
   int* err_d = nullptr;
@@ -113,12 +113,11 @@ struct tg_ctx {
   bool kd_dk = false;
   double* dphi_part = nullptr;
   int2* thin_list = nullptr;  // FP32 adjoint modes: cells gathered in FP64
-  int* thin_count = nullptr;
   // tiles taking the full path of the update / adjoint (compacted by their
   // classifying pass) and the list length
   TileRef* act_list = nullptr;  // (the FP32 adjoint lists bare tile indices in it)
   // [NCOUNT] list lengths: two pairs of the forward steps, two of the reverse
-  // steps (launches alternate; [0] also the FP32 adjoint's)
+  // steps, two of the FP32 reverse steps' thin cells (steps alternate)
   int* act_count = nullptr;
 
   // adaptive mesh (TG_MESH_LEAVES): leaf tables and reverse-step buffers
@@ -298,7 +297,6 @@ void free_fields(tg_ctx* ctx) {
   ctx->red_host = nullptr;
   dfree(ctx->dphi_part);
   dfree(ctx->thin_list);
-  dfree(ctx->thin_count);
   dfree(ctx->act_list);
   dfree(ctx->act_count);
   free_error_grid(ctx);
@@ -400,8 +398,10 @@ int tile_launch(const tg_ctx* ctx, int v) {
 }
 void set_by_tile(const tg_ctx* ctx, int v, StepArgs& a) { a.by_tile = tile_launch(ctx, v); }
 void set_by_tile(const tg_ctx* ctx, int v, AdjArgs& a) { a.by_tile = tile_launch(ctx, v); }
-template <class A>
-void set_by_tile(const tg_ctx*, int, A&) {}
+template <class S>
+void set_by_tile(const tg_ctx* ctx, int v, AdjArgsM<S>& a) { a.by_tile = tile_launch(ctx, v); }
+template <class S>
+void set_by_tile(const tg_ctx*, int, StepArgsM<S>&) {}
 
 // points a kernel's arguments at the tile table of its selected variant
 template <class A>
@@ -516,7 +516,11 @@ StepArgsM<S> step_args_m(tg_ctx* ctx, void* const in[3], void* const out[3], int
   a.inst = ctx->inst_d;
   a.U = FieldsT<S>{(S*)in[0], (S*)in[1], (S*)in[2]};
   a.S32 = statics32(ctx);
-  a.kact = (float*)ctx->kact; a.red = ctx->red; a.dt_rec = ctx->dt_rec; a.time = ctx->time_d;
+  a.kact = (float*)ctx->kact; a.dt_rec = ctx->dt_rec; a.time = ctx->time_d;
+  a.red = ctx->red + (s & 1) * ctx->ninst;
+  a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst;
+  a.clock = ctx->clock_d;
+  a.cfl_inner = ctx->cfg.cfl_inner; a.cfl_outer = ctx->cfg.cfl_outer;
   a.max_steps = ctx->cfg.max_steps; a.step = s; a.ft = frict_tiny(ctx, s);
   a.tiny = ctx->cfg.tiny; a.gamma = ctx->cfg.gamma;
   a.h_out = (S*)out[0]; a.hu_out = (S*)out[1]; a.hv_out = (S*)out[2];
@@ -529,6 +533,7 @@ StepArgsM<S> step_args_m(tg_ctx* ctx, void* const in[3], void* const out[3], int
 template <class S>
 void enqueue_step_m(tg_ctx* ctx, void* const in[3], void* const out[3], int s, bool compute_dt) {
   StepArgsM<S> a = step_args_m<S>(ctx, in, out, s);
+  a.fold = compute_dt;
   use_tiles(ctx, 0, a);
   inst_counter(ctx, 0, false);
   inst_counter(ctx, 1, false);
@@ -538,13 +543,6 @@ void enqueue_step_m(tg_ctx* ctx, void* const in[3], void* const out[3], int s, b
   a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[0]] == ctx->mk_tx[0];
   launch_coef_m<S>(a, compute_dt, ctx->stream);
   inst_mark(ctx, 0, false);
-  if (compute_dt) {
-    StepArgs d{};
-    d.inst = ctx->inst_d; d.red = ctx->red; d.dt_rec = ctx->dt_rec; d.time = ctx->time_d;
-    d.max_steps = ctx->cfg.max_steps; d.step = s;
-    d.cfl_inner = ctx->cfg.cfl_inner; d.cfl_outer = ctx->cfg.cfl_outer;
-    launch_dt(d, ctx->ninst, ctx->stream);
-  }
   use_tiles(ctx, 1, a);
   inst_mark(ctx, 1, true);
   a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[1]] == ctx->mk_tx[0];
@@ -567,11 +565,12 @@ void enqueue_adjoint_m(tg_ctx* ctx, void* const U[3], void* const lnext[3], void
   a.lam_h = (S*)lout[0]; a.lam_hu = (S*)lout[1]; a.lam_hv = (S*)lout[2];
   a.dphi_part = dphi ? ctx->dphi_part : nullptr;
   a.thin_list = ctx->thin_list;
-  a.thin_count = ctx->thin_count;
+  a.thin_count = ctx->act_count + 6 + (s & 1);
+  a.thin_next = ctx->act_count + 6 + ((s + 1) & 1);
   a.s64 = (ctx->ses == 8) ? (const double*)ctx->statics : nullptr;
   a.ncell = ctx->ncell;
   a.tile_list = (int*)ctx->act_list;
-  a.tile_count = ctx->act_count;
+  a.tile_count = ctx->act_count + 4;
   a.mk_U = marks_of(ctx, U);
   a.mk_lnext = marks_of(ctx, lnext);
   a.mk_out = marks_of(ctx, lout);
@@ -920,9 +919,9 @@ int stored_steps(const tg_ctx* ctx, int nsteps) {
 }
 
 // Every sequence of consecutive steps, forward or reverse, starts from empty
-// tile lists (each step then empties the next one's).
+// lists of tiles and thin cells (each step then empties the next one's).
 void empty_lists(tg_ctx* ctx) {
-  if (!ctx->leaves && tile_launch(ctx, 0) == 0)
+  if (!ctx->leaves && (ctx->mode != TG_FP64 || tile_launch(ctx, 0) == 0))
     launch_zero(ctx->act_count, sizeof(int) * NCOUNT, ctx->stream);
 }
 // ... and the reduction cells cleared and every member's clock set for step s.
@@ -1542,7 +1541,6 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
   if (!rc) rc = dalloc(ctx, (void**)&ctx->dphi_part, sizeof(double) * ctx->ntiles);
   if (!rc && ctx->mode != TG_FP64)
     rc = dalloc(ctx, (void**)&ctx->thin_list, sizeof(int2) * (size_t)n);
-  if (!rc && ctx->mode != TG_FP64) rc = dalloc(ctx, (void**)&ctx->thin_count, sizeof(int));
   if (!rc) rc = dalloc(ctx, (void**)&ctx->act_list, sizeof(TileRef) * (size_t)ctx->ntiles);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->act_count, sizeof(int) * NCOUNT);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->inst_d, sizeof(InstDev) * nm);

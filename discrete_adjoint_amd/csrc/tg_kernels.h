@@ -217,7 +217,8 @@ struct StepArgs {
 
 // dt = 0.5 * min(0.5 * min(dx / ev), 0.9 * sqrt(hmax eps Gs / 9.8)) clamped as
 // TimeProps::incrtime does (properties.h:397-410)
-__device__ __forceinline__ double cfl_dt(const StepArgs& a, const InstDev& I, const RedDev& R,
+template <class A>
+__device__ __forceinline__ double cfl_dt(const A& a, const InstDev& I, const RedDev& R,
                                          double time) {
   const double min_ev = __longlong_as_double((long long)R.min_ev), hmax = __longlong_as_double((long long)R.hmax);
   const double dt0 = a.cfl_inner * min_ev;
@@ -232,13 +233,14 @@ __device__ __forceinline__ double cfl_dt(const StepArgs& a, const InstDev& I, co
 }
 
 // The dt of member b at this step.  a.fold: it is made here, by every workgroup
-// alike, from the reduction cells the coefficient pass filled (k_dt's
-// arithmetic), instead of in a launch of its own; one workgroup of the member
+// alike, from the reduction cells the coefficient pass filled, instead of in a
+// launch of its own (4.4 us of every step); one workgroup of the member
 // (`own`) also records it, moves the member's clock on and clears the
 // reduction cells of the next step, which nothing else touches meanwhile
 // (steps alternate between two sets, and the clock has a slot per step).
 // Otherwise it was prescribed or recorded before.
-__device__ __forceinline__ double step_dt(const StepArgs& a, int b, bool own) {
+template <class A>
+__device__ __forceinline__ double step_dt(const A& a, int b, bool own) {
   double* rec = a.dt_rec + (long long)b * a.max_steps + a.step;
   if (!a.fold) return *rec;
   const InstDev& I = a.inst[b];
@@ -320,13 +322,17 @@ struct StepArgsM {
   FieldsT<S> U;
   Statics32 S32;
   float* kact;
-  RedDev* red;
+  RedDev* red;           // as in StepArgs, down to fold
+  RedDev* red_next;
   double* dt_rec;
   double* time;
+  double* clock;
+  int fold;
   int max_steps;
   int step;
   double ft;
   double tiny, gamma;  // thresholds kept in FP64: the switches compare in W
+  double cfl_inner, cfl_outer;
   S* h_out;
   S* hu_out;
   S* hv_out;
@@ -360,8 +366,13 @@ struct AdjArgsM {
   S* lam_hu;
   S* lam_hv;
   double* dphi_part;
-  int2* thin_list;       // [ncell] (tile, thread) of cells gathered in FP64
+  // [ncell] (tile, thread) of the cells gathered in FP64, and their count;
+  // thin_next: the next reverse step's count, emptied by this step's last
+  // pass (steps alternate between two), and so is tile_count
+  int2* thin_list;
   int* thin_count;
+  int* thin_next;
+  int by_tile;           // as in StepArgs
   const double* s64;     // FP64 static coefficients [7 * ncell] or null
   long long ncell;
   unsigned long long* active;  // null, or counter of cells in non-void tiles
@@ -375,8 +386,9 @@ struct AdjArgsM {
   uint32_t* mk_out;
   int u_bytes, l_bytes;
 };
-// workgroups of the FP64 thin-layer adjoint pass (strides over its list)
-constexpr int THIN_GRID = 1024;
+// most workgroups of the FP64 thin-layer adjoint pass (strides over its list):
+// as many as the chip holds of them at once
+constexpr int THIN_GRID = 512;
 // workgroups of the update / adjoint passes that stride over the compacted
 // list of tiles taking the full path (a fixed grid, for graph capture):
 // 16 per CU, so that the workgroups left without a tile exit early while
@@ -477,7 +489,6 @@ void launch_leaf_stats(const LeafDev& L, Fields U, double* part_mass, double* pa
                        double tiny, hipStream_t s);
 
 void launch_coef(const StepArgs& a, bool reduce, hipStream_t s);
-void launch_dt(const StepArgs& a, int ninst, hipStream_t s);
 void launch_update(const StepArgs& a, hipStream_t s);
 void launch_adjoint(const AdjArgs& a, hipStream_t s);
 // clears both sets of reduction cells (red [2 * ninst]); clock (or null):

@@ -452,17 +452,6 @@ __global__ void k_member_fill(const uint32_t* __restrict__ src, uint32_t* __rest
     for (long long i = t0; i < nmw; i += stride) mk[mw0 + i] = 0u;
 }
 
-__global__ void k_dt(StepArgs a, int ninst) {
-  int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= ninst) return;
-  const double time = a.time[b];
-  const double dt = cfl_dt(a, a.inst[b], a.red[b], time);
-  a.time[b] = time + dt;
-  a.dt_rec[(long long)b * a.max_steps + a.step] = dt;
-  a.red[b].min_ev = dbits(10000000.);
-  a.red[b].hmax = dbits(0.);
-}
-
 // Face records of one tile: every face flux and every one-sided difference
 // the tile's cells use is computed once (a face is shared by two cells) and
 // staged in LDS.  x-face fi of row fj lies between tile columns fi-1 and fi.
@@ -1523,9 +1512,6 @@ __global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint_tile(AdjArgs a) {
 void launch_coef(const StepArgs& a, bool reduce, hipStream_t s) {
   if (a.by_tile) TG_LAUNCH_TX(a.shape, k_coef_tile, dim3(a.ntiles), s, a, reduce ? 1 : 0);
   else TG_LAUNCH_TX(a.shape, k_coef, dim3(a.nblocks), s, a, reduce ? 1 : 0);
-}
-void launch_dt(const StepArgs& a, int ninst, hipStream_t s) {
-  hipLaunchKernelGGL(k_dt, dim3((ninst + 63) / 64), dim3(64), 0, s, a, ninst);
 }
 void launch_update(const StepArgs& a, hipStream_t s) {
   const int g = a.by_tile || a.ntiles < LIST_GRID ? a.ntiles : LIST_GRID;

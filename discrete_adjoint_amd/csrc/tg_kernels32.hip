@@ -198,7 +198,8 @@ __device__ __forceinline__ Hfv rec_hfv32(const Lds32<W, TX>& L, int dir, int r) 
              L.g[r], L.wet[r] != 0);
 }
 
-// One workgroup per tile.  A tile whose cells and frame are all below tiny
+// One workgroup per tile, which also makes dt (step_dt): a pass of its own
+// cost 4.4 us beside this one's 8.4 (389 x 301 cells).  A tile whose cells and frame are all below tiny
 // has every face flux zero and no sources: its cells take the update's own
 // arithmetic with zero fluxes, without the flux and slope work.
 template <class S, int TX>
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(BLOCK) void k32_update(StepArgsM<S> a) {
   __shared__ L32 L;
   const TileDev t = a.tiles[blockIdx.x];
   const InstDev I = a.inst[t.inst];
-  const double dt = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
+  const double dt = step_dt(a, t.inst, t.x0 == 0 && t.y0 == 0);
   // the tile and its four side tiles of U marked +0.0: zero fluxes, no
   // sources (h < tiny), so U^{s+1} = +0.0 + (-dtdx * 0 - dtdy * 0) = +0.0 for
   // a finite dt; nothing to do when the output tile is marked +0.0 already
@@ -665,31 +666,29 @@ __device__ __forceinline__ void face_dk(int side, const DualInfoT<F>& L, const D
   driemann(hl, hr, dFl, dWl, dFr, dWr, dflux);
 }
 
-// lambda^{s+1} . dF/d phi_bed of one cell at frozen dt
+// lambda^{s+1} . dF/d phi_bed of one cell at frozen dt, from the fluxes of its
+// faces (slot 1 E, 2 N, 3 W, 4 S) and their derivatives along phi_bed
+template <class F>
+struct FaceDk {
+  F f[3], d[3];
+};
 template <class S, class F>
 __device__ __forceinline__ F dphi_term(const AdjArgsM<S>& a, const InstDev& I, long long c,
-                       const DualInfoT<F>& C, const DualInfoT<F>& E, const DualInfoT<F>& N,
-                       const DualInfoT<F>& Wc, const DualInfoT<F>& Sc, const bool has[5], F dt,
-                       const F lam[3]) {
-  F fE[3] = {0, 0, 0}, fN[3] = {0, 0, 0}, fW[3] = {0, 0, 0}, fS[3] = {0, 0, 0};
-  F dE[3] = {0, 0, 0}, dN[3] = {0, 0, 0}, dW[3] = {0, 0, 0}, dS[3] = {0, 0, 0};
-  if (has[1]) face_dk(0, C, E, fE, dE);
-  if (has[3]) face_dk(0, Wc, C, fW, dW);
-  if (has[2]) face_dk(1, C, N, fN, dN);
-  if (has[4]) face_dk(1, Sc, C, fS, dS);
+                                       const DualInfoT<F>& C, FaceDk<F> E, FaceDk<F> N,
+                                       FaceDk<F> W, FaceDk<F> B, const bool has[5], F dt) {
   // boundary faces copy the opposite face
 #pragma unroll
   for (int v = 0; v < 3; v++) {
-    if (!has[1]) { fE[v] = fW[v]; dE[v] = dW[v]; }
-    if (!has[3]) { fW[v] = fE[v]; dW[v] = dE[v]; }
-    if (!has[2]) { fN[v] = fS[v]; dN[v] = dS[v]; }
-    if (!has[4]) { fS[v] = fN[v]; dS[v] = dN[v]; }
+    if (!has[1]) { E.f[v] = W.f[v]; E.d[v] = W.d[v]; }
+    if (!has[3]) { W.f[v] = E.f[v]; W.d[v] = E.d[v]; }
+    if (!has[2]) { N.f[v] = B.f[v]; N.d[v] = B.d[v]; }
+    if (!has[4]) { B.f[v] = N.f[v]; B.d[v] = N.d[v]; }
   }
   const F dtdx = (F)(dt * I.inv_dx), dtdy = (F)(dt * I.inv_dy);
   F out[3];
 #pragma unroll
-  for (int v = 0; v < 3; v++) out[v] = -dtdx * (dE[v] - dW[v]) - dtdy * (dN[v] - dS[v]);
-  if (C.h - dtdx * (fE[0] - fW[0]) - dtdy * (fN[0] - fS[0]) < F(0)) out[0] = F(0);
+  for (int v = 0; v < 3; v++) out[v] = -dtdx * (E.d[v] - W.d[v]) - dtdy * (N.d[v] - B.d[v]);
+  if (C.h - dtdx * (E.f[0] - W.f[0]) - dtdy * (N.f[0] - B.f[0]) < F(0)) out[0] = F(0);
   if (C.thick) {
     const double tbc = mat_of(I, a.mat, a.mtab, c).tan_bed;
     const F sec2 = (F)(1. + tbc * tbc), sint = (F)I.sin_int;
@@ -701,138 +700,150 @@ __device__ __forceinline__ F dphi_term(const AdjArgsM<S>& a, const InstDev& I, l
     out[1] -= dt * (ds2x + ds3x);
     out[2] -= dt * (ds2y + ds3y);
   }
-  return lam[0] * out[0] + lam[1] * out[1] + lam[2] * out[2];
+  return C.lam[0] * out[0] + C.lam[1] * out[1] + C.lam[2] * out[2];
 }
 
-// The gather of one cell in arithmetic type F: adj = sum of the transposed
-// Jacobian blocks (the self block without its identity) applied to
-// lambda^{s+1}; nbr(s) returns the record of neighbour slot s (1 E, 2 N,
-// 3 W, 4 S).  Returns the cell's dJ/dphi_bed term (0 unless want_dphi).
-template <class S, class F, class NBR>
+// The own block of one cell without its identity (applied in the storage type
+// by the caller), from the Jacobians of its face fluxes, applied to
+// lambda^{s+1}; boundary faces copy the opposite face.
+template <class S, class F>
+__device__ __forceinline__ void self_part(const AdjArgsM<S>& a, const InstDev& I, long long c,
+                                          const DualInfoT<F>& self, const bool has[5],
+                                          const M3T<F>& JE, const M3T<F>& JN, const M3T<F>& JW,
+                                          const M3T<F>& JS, F dt, F dtdx, F dtdy, F adj[3]) {
+  M3T<F> J;
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const F pE = has[1] ? JE.a[i][j] : JW.a[i][j];
+      const F nW = has[3] ? JW.a[i][j] : JE.a[i][j];
+      const F pN = has[2] ? JN.a[i][j] : JS.a[i][j];
+      const F nS = has[4] ? JS.a[i][j] : JN.a[i][j];
+      J.a[i][j] = dtdx * (pE - nW) + dtdy * (pN - nS);
+    }
+  if (self.thick) {
+    const F sint = (F)I.sin_int, tb = (F)mat_of(I, a.mat, a.mtab, c).tan_bed;
+    const F alpha = sint * self.sgn[0] * self.k, betta = sint * self.sgn[1] * self.k;
+    const F u = self.u, v = self.v;
+    const F g2 = self.g2, k0 = stat<F>(a, 5, c), k1 = stat<F>(a, 6, c);
+    J.a[1][0] -= dt * (stat<F>(a, 0, c) -
+                       alpha * self.h * (F(2) * stat<F>(a, 4, c) + g2 * self.hsy[0]) -
+                       alpha * g2 * self.hy);
+    if (self.sgn[2] != F(0) && !self.stop[0]) {
+      J.a[1][0] += dt * self.sgn[2] * tb * (g2 - u * u * k0);
+      J.a[1][1] += dt * self.sgn[2] * tb * (F(2) * u * k0);
+    }
+    J.a[2][0] -= dt * (stat<F>(a, 1, c) -
+                       betta * self.h * (F(2) * stat<F>(a, 3, c) + g2 * self.hsx[0]) -
+                       betta * g2 * self.hx);
+    if (self.sgn[3] != F(0) && !self.stop[1]) {
+      J.a[2][0] += dt * self.sgn[3] * tb * (g2 - v * v * k1);
+      J.a[2][2] += dt * self.sgn[3] * tb * (F(2) * v * k1);
+    }
+  }
+  accum_T(adj, J, self.lam);
+}
+
+// The block of neighbour slot s (record N): the Jacobian jf of the face
+// between, where the neighbour is no cell of the member's edge, and its slope
+// sensitivity.
+template <class F>
+__device__ __forceinline__ M3T<F> nbr_part(const InstDev& I, const Cell& q, int s,
+                                           const M3T<F>& jf, const DualInfoT<F>& N, F dt, F dtdx,
+                                           F dtdy) {
+  const F sint = (F)I.sin_int;
+  M3T<F> J = zero3<F>();
+  if (s == 1) {
+    if (q.i + 2 < I.nx)
+      for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = -dtdx * jf.a[i][j];
+    nbr_block(J, N, sint, dt, N.hsx[1], F(0));
+  } else if (s == 3) {
+    if (q.i - 2 >= 0)
+      for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = dtdx * jf.a[i][j];
+    nbr_block(J, N, sint, dt, N.hsx[2], F(0));
+  } else if (s == 2) {
+    if (q.j + 2 < I.ny)
+      for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = -dtdy * jf.a[i][j];
+    nbr_block(J, N, sint, dt, F(0), N.hsy[1]);
+  } else {
+    if (q.j - 2 >= 0)
+      for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = dtdy * jf.a[i][j];
+    nbr_block(J, N, sint, dt, F(0), N.hsy[2]);
+  }
+  return J;
+}
+
+// The gather of one cell in FP32: adj = sum of the transposed Jacobian blocks
+// (the self block without its identity) applied to lambda^{s+1}; nbr(s)
+// returns the record of neighbour slot s (1 E, 2 N, 3 W, 4 S).  Returns the
+// cell's dJ/dphi_bed term (0 unless want_dphi).
+template <class S, class NBR>
 __device__ __forceinline__ double gather(const AdjArgsM<S>& a, const InstDev& I, const Cell& q,
-                                         const DualInfoT<F>& self, NBR&& nbr, double dtd,
-                                         F adj[3], bool want_dphi) {
-  const long long c = q.c, nx = I.nx;
+                                         const DualInfoT<float>& self, NBR&& nbr, double dtd,
+                                         float adj[3], bool want_dphi) {
+  using F = float;
+  const long long c = q.c;
   const F dt = (F)dtd, dtdx = (F)(dtd * I.inv_dx), dtdy = (F)(dtd * I.inv_dy);
   const bool has[5] = {true, q.hasE, q.hasN, q.hasW, q.hasS};
   adj[0] = adj[1] = adj[2] = F(0);
   if (self.nz) {
-    M3T<F> JE = zero3<F>(), JN = zero3<F>(), JW = zero3<F>(), JS = zero3<F>();
+    M3T<F> JF[5];  // of the face fluxes, by slot
+#pragma unroll
+    for (int s = 1; s < 5; s++) JF[s] = zero3<F>();
     {
       const DualHfvT<F> cx = dual_hfv(0, self);
-      if (has[1]) JE = dual_riemann_side(cx, dual_hfv(0, nbr(1)), true);
-      if (has[3]) JW = dual_riemann_side(dual_hfv(0, nbr(3)), cx, false);
+      if (has[1]) JF[1] = dual_riemann_side(cx, dual_hfv(0, nbr(1)), true);
+      if (has[3]) JF[3] = dual_riemann_side(dual_hfv(0, nbr(3)), cx, false);
     }
     {
       const DualHfvT<F> cy = dual_hfv(1, self);
-      if (has[2]) JN = dual_riemann_side(cy, dual_hfv(1, nbr(2)), true);
-      if (has[4]) JS = dual_riemann_side(dual_hfv(1, nbr(4)), cy, false);
+      if (has[2]) JF[2] = dual_riemann_side(cy, dual_hfv(1, nbr(2)), true);
+      if (has[4]) JF[4] = dual_riemann_side(dual_hfv(1, nbr(4)), cy, false);
     }
     asm volatile("" ::: "memory");
-    // self block without its identity (applied in the storage type by the
-    // caller); boundary faces copy the opposite face
-    {
-      M3T<F> J;
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-          const F pE = has[1] ? JE.a[i][j] : JW.a[i][j];
-          const F nW = has[3] ? JW.a[i][j] : JE.a[i][j];
-          const F pN = has[2] ? JN.a[i][j] : JS.a[i][j];
-          const F nS = has[4] ? JS.a[i][j] : JN.a[i][j];
-          J.a[i][j] = dtdx * (pE - nW) + dtdy * (pN - nS);
-        }
-      if (self.thick) {
-        const F sint = (F)I.sin_int, tb = (F)mat_of(I, a.mat, a.mtab, c).tan_bed;
-        const F alpha = sint * self.sgn[0] * self.k, betta = sint * self.sgn[1] * self.k;
-        const F u = self.u, v = self.v;
-        const F g2 = self.g2, k0 = stat<F>(a, 5, c), k1 = stat<F>(a, 6, c);
-        J.a[1][0] -= dt * (stat<F>(a, 0, c) -
-                           alpha * self.h * (F(2) * stat<F>(a, 4, c) + g2 * self.hsy[0]) -
-                           alpha * g2 * self.hy);
-        if (self.sgn[2] != F(0) && !self.stop[0]) {
-          J.a[1][0] += dt * self.sgn[2] * tb * (g2 - u * u * k0);
-          J.a[1][1] += dt * self.sgn[2] * tb * (F(2) * u * k0);
-        }
-        J.a[2][0] -= dt * (stat<F>(a, 1, c) -
-                           betta * self.h * (F(2) * stat<F>(a, 3, c) + g2 * self.hsx[0]) -
-                           betta * g2 * self.hx);
-        if (self.sgn[3] != F(0) && !self.stop[1]) {
-          J.a[2][0] += dt * self.sgn[3] * tb * (g2 - v * v * k1);
-          J.a[2][2] += dt * self.sgn[3] * tb * (F(2) * v * k1);
-        }
-      }
-      accum_T(adj, J, self.lam);
-    }
-    const int order[4] = {4, 1, 2, 3};  // S, E, N, W (reference visiting order)
-    const F sint = (F)I.sin_int;
+    self_part<S, F>(a, I, c, self, has, JF[1], JF[2], JF[3], JF[4], dt, dtdx, dtdy, adj);
 #pragma unroll
     for (int o = 0; o < 4; o++) {
-      const int s = order[o];
+      const int s = o == 0 ? 4 : o;  // S, E, N, W (reference visiting order)
       if (!has[s]) continue;
       const DualInfoT<F> N = nbr(s);
-      M3T<F> J = zero3<F>();
-      if (s == 1) {
-        if (q.i + 2 < I.nx)
-          for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = -dtdx * JE.a[i][j];
-        nbr_block(J, N, sint, dt, N.hsx[1], F(0));
-      } else if (s == 3) {
-        if (q.i - 2 >= 0)
-          for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = dtdx * JW.a[i][j];
-        nbr_block(J, N, sint, dt, N.hsx[2], F(0));
-      } else if (s == 2) {
-        if (q.j + 2 < I.ny)
-          for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = -dtdy * JN.a[i][j];
-        nbr_block(J, N, sint, dt, F(0), N.hsy[1]);
-      } else {
-        if (q.j - 2 >= 0)
-          for (int i = 0; i < 3; i++) for (int j = 0; j < 3; j++) J.a[i][j] = dtdy * JS.a[i][j];
-        nbr_block(J, N, sint, dt, F(0), N.hsy[2]);
-      }
-      accum_T(adj, J, N.lam);
+      accum_T(adj, nbr_part(I, q, s, JF[s], N, dt, dtdx, dtdy), N.lam);
     }
   }
   if (!want_dphi) return 0.;
   asm volatile("" ::: "memory");
-  return (double)dphi_term<S, F>(a, I, c, self, nbr(1), nbr(2), nbr(3), nbr(4), has, dt,
-                                 self.lam);
+  FaceDk<F> K[5] = {};
+  if (has[1]) face_dk(0, self, nbr(1), K[1].f, K[1].d);
+  if (has[3]) face_dk(0, nbr(3), self, K[3].f, K[3].d);
+  if (has[2]) face_dk(1, self, nbr(2), K[2].f, K[2].d);
+  if (has[4]) face_dk(1, nbr(4), self, K[4].f, K[4].d);
+  return (double)dphi_term<S, F>(a, I, c, self, K[1], K[2], K[3], K[4], has, dt);
 }
 
-// Adjoint pass 1 (one workgroup per tile): a tile of void cells (h == 0)
-// gets lambda^s = 0 -- every block that multiplies a void cell's state is
+// A tile of void cells (h == 0) gets lambda^s = 0 -- every block that multiplies a void cell's state is
 // zero (calc_jacobain.C:117-122), as in pass 2 -- and, with lambda^{s+1} == 0
-// on the tile, zero bed-friction terms; it is written here.  Every other
-// tile is appended to the list pass 2 walks.  With marks, a tile whose U^s
+// on the tile, zero bed-friction terms; it is written here (true).  Every
+// other tile takes the gather; on large meshes pass 1 (one workgroup per tile)
+// appends it to the list pass 2 walks.  With marks, a tile whose U^s
 // (and lambda^{s+1}, when the gradient is wanted) is marked +0.0 is void
 // without reading the fields, and its lambda^s is not rewritten when that
 // is marked +0.0 already.
 template <class S, int TX>
-__global__ __launch_bounds__(BLOCK) void k32_adjoint_classify(AdjArgsM<S> a) {
-  const TileDev t = a.tiles[blockIdx.x];
-  const InstDev I = a.inst[t.inst];
-  const Cell q = cell_of<TX>(t, I);
+__device__ __forceinline__ bool adjoint32_void(const AdjArgsM<S>& a, const TileDev& t,
+                                               const Cell& q) {
   if (a.mk_out && tile_marked_zero<TX>(a.mk_U, t, a.u_bytes) &&
       (!a.dphi_part || tile_marked_zero<TX>(a.mk_lnext, t, a.l_bytes))) {
-    if (tile_marked_zero<TX>(a.mk_out, t, a.l_bytes)) return;
+    if (tile_marked_zero<TX>(a.mk_out, t, a.l_bytes)) return true;
+  } else {
+    bool busy = false;
     if (q.act) {
-      a.lam_h[q.c] = (S)0;
-      a.lam_hu[q.c] = (S)0;
-      a.lam_hv[q.c] = (S)0;
+      busy = a.U.h[q.c] != (S)0;
+      if (a.dphi_part)
+        busy = busy || !(a.lam_next.h[q.c] == (S)0 && a.lam_next.hu[q.c] == (S)0 &&
+                         a.lam_next.hv[q.c] == (S)0);
     }
-    tile_mark_store<TX>(a.mk_out, t, true);
-    return;
-  }
-  bool busy = false;
-  if (q.act) {
-    busy = a.U.h[q.c] != (S)0;
-    if (a.dphi_part)
-      busy = busy || !(a.lam_next.h[q.c] == (S)0 && a.lam_next.hu[q.c] == (S)0 &&
-                       a.lam_next.hv[q.c] == (S)0);
-  }
-  if (__syncthreads_or(busy)) {
-    if (threadIdx.x == 0) a.tile_list[atomicAdd(a.tile_count, 1)] = (int)blockIdx.x;
-    return;
+    if (__syncthreads_or(busy)) return false;
   }
   if (q.act) {
     a.lam_h[q.c] = (S)0;
@@ -840,18 +851,26 @@ __global__ __launch_bounds__(BLOCK) void k32_adjoint_classify(AdjArgsM<S> a) {
     a.lam_hv[q.c] = (S)0;
   }
   if (a.mk_out) tile_mark_store<TX>(a.mk_out, t, true);
+  return true;
 }
 
-// Adjoint pass 2, one listed tile.
 template <class S, int TX>
-__device__ __forceinline__ void adjoint32_tile(const AdjArgsM<S>& a, int tile, DualLds& L,
-                                               double* sp) {
-  const TileDev t = a.tiles[tile];
-  const InstDev I = a.inst[t.inst];
-  const Cell q = cell_of<TX>(t, I);
+__global__ __launch_bounds__(BLOCK) void k32_adjoint_classify(AdjArgsM<S> a) {
+  const TileDev t = a.tiles[blockIdx.x];
+  if (!adjoint32_void<S, TX>(a, t, cell_of<TX>(t, a.inst[t.inst])) && threadIdx.x == 0)
+    a.tile_list[atomicAdd(a.tile_count, 1)] = (int)blockIdx.x;
+}
+
+// The gather of one tile by THREADS threads: the first 256 take a cell each;
+// those after them, where there are any, the halo records, else the first do.
+template <class S, int TX, int THREADS>
+__device__ __forceinline__ void adjoint32_tile(const AdjArgsM<S>& a, const TileDev& t,
+                                               const InstDev& I, const Cell& q, int tile,
+                                               DualLds& L, double* sp) {
   const bool want_dphi = a.dphi_part != nullptr;
   // the halo is the four side strips: the 5-point stencil reads no corner
   constexpr int TY = BLOCK / TX, RX = TX + 2, RY = TY + 2, NHALO = 2 * TX + 2 * TY;
+  constexpr int HALO0 = THREADS > BLOCK ? BLOCK : 0;  // the halo's first thread
   static_assert(RX * RY <= RN && NHALO <= BLOCK, "tile does not fit the LDS records");
   if (a.active) {
     const int cnt = __syncthreads_count(q.act);
@@ -864,8 +883,8 @@ __device__ __forceinline__ void adjoint32_tile(const AdjArgsM<S>& a, int tile, D
     self = dual_info<S, float>(a, I, q.i, q.j, want_dphi);
     lds_put(L, rself, self);
   }
-  if ((int)threadIdx.x < NHALO) {
-    const int h = (int)threadIdx.x;
+  const int h = (int)threadIdx.x - HALO0;
+  if (h >= 0 && h < NHALO) {
     int rx, ry;
     if (h < TX) { rx = h + 1; ry = 0; }
     else if (h < 2 * TX) { rx = h - TX + 1; ry = RY - 1; }
@@ -900,7 +919,7 @@ __device__ __forceinline__ void adjoint32_tile(const AdjArgsM<S>& a, int tile, D
     } else {
       const S lc[3] = {a.lam_next.h[c], a.lam_next.hu[c], a.lam_next.hv[c]};
       float adj[3];
-      dphi = gather<S, float>(a, I, q, self, [&](int s) { return lds_get(L, rn(s)); }, dtd, adj,
+      dphi = gather<S>(a, I, q, self, [&](int s) { return lds_get(L, rn(s)); }, dtd, adj,
                               want_dphi);
       // lambda^s = -(K_self - I)^T lambda_c - sum K_n^T lambda_n = lambda_c - adj;
       // flush |lambda| < 1e-16 (calc_adjoint.C:150-152)
@@ -928,9 +947,10 @@ __device__ __forceinline__ void adjoint32_tile(const AdjArgsM<S>& a, int tile, D
 }
 
 
-// Five waves per SIMD: the register cap costs a few spills to scratch, but
-// the gather is latency-bound and the extra wave in flight hides more of it
-// (about 6% faster than the unconstrained 4-wave allocation, measured).
+// Pass 2 on large meshes: a fixed grid walks the listed tiles.  Five waves per
+// SIMD: the register cap costs a few spills to scratch, but the gather is
+// latency-bound and the extra wave in flight hides more of it (about 6% faster
+// than the unconstrained 4-wave allocation, measured).
 template <class S, int TX>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
 void k32_adjoint(AdjArgsM<S> a) {
@@ -938,20 +958,70 @@ void k32_adjoint(AdjArgsM<S> a) {
   __shared__ double sp[BLOCK / 64];
   const int n = *a.tile_count;
   for (int i = (int)blockIdx.x; i < n; i += (int)gridDim.x) {
-    adjoint32_tile<S, TX>(a, a.tile_list[list_band(i, n)], L, sp);
+    const int tile = a.tile_list[list_band(i, n)];
+    const TileDev t = a.tiles[tile];
+    const InstDev I = a.inst[t.inst];
+    adjoint32_tile<S, TX, BLOCK>(a, t, I, cell_of<TX>(t, I), tile, L, sp);
     __syncthreads();  // LDS reused by the next tile
   }
 }
 
-// The cells k32_adjoint listed (a thin layer in their stencil), gathered in
-// FP64 from global memory.  A fixed grid strides over the list, so the
-// launch does not depend on the count (graph capture).
+// Both passes on small meshes, one workgroup per tile, nothing listed: a step
+// there lasts as long as one tile's chain of loads and arithmetic, so every
+// record has a thread of its own and nothing is spilled (389 x 301 cells, 457
+// tiles, mixed: 16 us against 5.3 for the classifying pass, 22 for the gather
+// and 4.4 for emptying the list).  The line to the two passes is the FP64
+// kernels' (TILE_LAUNCH_MAX): past it the LDS of empty tiles queues.
+template <int TX>
+constexpr int adj32_threads() {
+  return BLOCK + (2 * TX + 2 * (BLOCK / TX) + 63) / 64 * 64;
+}
+template <class S, int TX>
+__global__ __launch_bounds__(adj32_threads<TX>()) void k32_adjoint_tile(AdjArgsM<S> a) {
+  __shared__ DualLds L;
+  __shared__ double sp[adj32_threads<TX>() / 64];
+  const int tile = a.by_tile == 2 ? unbanded((int)blockIdx.x, a.ntiles) : (int)blockIdx.x;
+  const TileDev t = a.tiles[tile];
+  const InstDev I = a.inst[t.inst];
+  Cell q = cell_of<TX>(t, I);
+  if (threadIdx.x >= BLOCK) q.act = false;
+  if (adjoint32_void<S, TX>(a, t, q)) return;
+  adjoint32_tile<S, TX, adj32_threads<TX>()>(a, t, I, q, tile, L, sp);
+}
+
+// The cells the gather listed (a thin layer in their stencil), gathered in
+// FP64 from global memory: lane 0 of eight takes the cell's record, lanes 1-4
+// its E, N, W and S neighbours', each then the block and the face derivative
+// of its side, and lane 0 adds them in the gather's order.  Some thousand
+// cells at a front leave the chip idle, so the time is one cell's chain of
+// loads and FP64 arithmetic: a thread per cell evaluates the neighbours'
+// records one after another, three times over (389 x 301 cells: 34.5 us
+// against 19.6).  A fixed grid strides over the list, so the launch does not depend on the
+// count (graph capture).
+constexpr int THIN_LANES = 8, THIN_CELLS = BLOCK / THIN_LANES;
+struct ThinLds {
+  DualInfoT<double> self[THIN_CELLS];
+  M3T<double> face[5][THIN_CELLS], block[5][THIN_CELLS];  // by slot
+  double lam[5][THIN_CELLS][3];
+  FaceDk<double> dk[5][THIN_CELLS];
+};
 template <class S, int TX>
 __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
+  using F = double;
+  __shared__ ThinLds L;
   const bool want_dphi = a.dphi_part != nullptr;
+  const int g = (int)threadIdx.x / THIN_LANES, s = (int)threadIdx.x % THIN_LANES;
+  const int e1 = (int)blockIdx.x * THIN_CELLS + g;
+  // (beside the count's load: entries at or past the count are not used)
+  const int2 first = a.thin_list[e1 < a.ncell ? e1 : 0];
   const int n = *a.thin_count;
-  for (int e = blockIdx.x * BLOCK + threadIdx.x; e < n; e += gridDim.x * BLOCK) {
-    const int2 item = a.thin_list[e];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.tile_count = *a.thin_next = 0;
+#pragma unroll 1
+  for (int e0 = e1 - g; e0 < n; e0 += (int)gridDim.x * THIN_CELLS) {
+    const int e = e0 + g;
+    const bool in = e < n && s < 5;
+    int2 item = e0 == e1 - g ? first : a.thin_list[e < n ? e : e0];
+    if (e >= n) item = make_int2(0, 0);
     const TileDev t = a.tiles[item.x];
     const InstDev I = a.inst[t.inst];
     Cell q;
@@ -963,31 +1033,68 @@ __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
     q.hasW = q.i > 0;
     q.hasN = q.j + 1 < I.ny;
     q.hasS = q.j > 0;
-    const long long c = q.c;
-    const double dtd = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
-    const DualInfoT<double> self = dual_info<S, double>(a, I, q.i, q.j, want_dphi);
-    double adj[3];
-    // neighbour s (1 E, 2 N, 3 W, 4 S); an absent neighbour (domain edge)
-    // is never read by the gather -- return the cell's own record instead of
-    // touching memory outside the block
-    auto nbr = [&](int s) {
-      const bool present = s == 1 ? q.hasE : (s == 2 ? q.hasN : (s == 3 ? q.hasW : q.hasS));
-      if (!present) return self;
-      const int i = q.i + (s == 1 ? 1 : (s == 3 ? -1 : 0));
-      const int j = q.j + (s == 2 ? 1 : (s == 4 ? -1 : 0));
-      return dual_info<S, double>(a, I, i, j, want_dphi);
-    };
-    const double dphi = gather<S, double>(a, I, q, self, nbr, dtd, adj, want_dphi);
-    const S lc[3] = {a.lam_next.h[c], a.lam_next.hu[c], a.lam_next.hv[c]};
-    S out[3];
-    for (int j = 0; j < 3; j++) {
-      out[j] = self.nz ? (S)((double)lc[j] - adj[j]) : (S)0;
-      if (fabs((double)out[j]) < 1e-16) out[j] = (S)0;
+    const double dt = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
+    const double dtdx = dt * I.inv_dx, dtdy = dt * I.inv_dy;
+    const bool has[5] = {true, q.hasE, q.hasN, q.hasW, q.hasS};
+    const bool mine =
+        in && (s == 0 || (s == 1 ? q.hasE : s == 2 ? q.hasN : s == 3 ? q.hasW : q.hasS));
+    const int dir = (s & 1) ? 0 : 1;
+    DualInfoT<F> R;
+    if (mine) {
+      R = dual_info<S, F>(a, I, q.i + (s == 1) - (s == 3), q.j + (s == 2) - (s == 4), want_dphi);
+      if (s == 0) L.self[g] = R;
     }
-    a.lam_h[c] = out[0];
-    a.lam_hu[c] = out[1];
-    a.lam_hv[c] = out[2];
-    if (want_dphi) atomicAdd(&a.dphi_part[item.x], dphi);
+    __syncthreads();
+    if (mine && s) {
+      const DualInfoT<F> C = L.self[g];
+      const bool left = s <= 2;  // the cell is the face's left side
+      if (C.nz) {
+        const DualHfvT<F> hc = dual_hfv(dir, C), hn = dual_hfv(dir, R);
+        const M3T<F> jf = left ? dual_riemann_side(hc, hn, true) : dual_riemann_side(hn, hc, false);
+        L.face[s][g] = jf;
+        L.block[s][g] = nbr_part(I, q, s, jf, R, dt, dtdx, dtdy);
+        for (int v = 0; v < 3; v++) L.lam[s][g][v] = R.lam[v];
+      }
+      if (want_dphi) {
+        FaceDk<F> k;
+        if (left) face_dk(dir, C, R, k.f, k.d);
+        else face_dk(dir, R, C, k.f, k.d);
+        L.dk[s][g] = k;
+      }
+    }
+    __syncthreads();
+    if (mine && s == 0) {
+      const long long c = q.c;
+      F adj[3] = {0., 0., 0.};
+      if (R.nz) {
+        M3T<F> JF[5];
+#pragma unroll
+        for (int o = 1; o < 5; o++) JF[o] = has[o] ? L.face[o][g] : zero3<F>();
+        self_part<S, F>(a, I, c, R, has, JF[1], JF[2], JF[3], JF[4], dt, dtdx, dtdy, adj);
+#pragma unroll
+        for (int o = 0; o < 4; o++) {
+          const int k = o == 0 ? 4 : o;  // S, E, N, W (reference visiting order)
+          if (has[k]) accum_T(adj, L.block[k][g], L.lam[k][g]);
+        }
+      }
+      S out[3];
+      for (int j = 0; j < 3; j++) {
+        out[j] = R.nz ? (S)(R.lam[j] - adj[j]) : (S)0;
+        if (fabs((double)out[j]) < 1e-16) out[j] = (S)0;
+      }
+      a.lam_h[c] = out[0];
+      a.lam_hu[c] = out[1];
+      a.lam_hv[c] = out[2];
+      if (want_dphi) {
+        FaceDk<F> K[5] = {};
+#pragma unroll
+        for (int o = 1; o < 5; o++)
+          if (has[o]) K[o] = L.dk[o][g];
+        atomicAdd(&a.dphi_part[item.x],
+                  dphi_term<S, F>(a, I, c, R, K[1], K[2], K[3], K[4], has, dt));
+      }
+    }
+    __syncthreads();  // LDS reused by the next cells
   }
 }
 
@@ -1012,12 +1119,21 @@ void launch_update_m(const StepArgsM<S>& a, hipStream_t s) {
 }
 template <class S>
 void launch_adjoint_m(const AdjArgsM<S>& a, hipStream_t s) {
-  launch_zero(a.thin_count, sizeof(int), s);
-  launch_zero(a.tile_count, sizeof(int), s);
-  TG_LAUNCH_TX(a.shape, k32_adjoint_classify, S, dim3(a.ntiles), s, a);
-  TG_LAUNCH_TX(a.shape, k32_adjoint, S, dim3(a.ntiles < LIST_GRID ? a.ntiles : LIST_GRID), s,
-               a);
-  const int g = a.ntiles < THIN_GRID ? a.ntiles : THIN_GRID;
+  const int tx = SHAPE_TX[a.shape];
+  if (a.by_tile) {
+#define TG_ADJ32(TX) \
+  hipLaunchKernelGGL((k32_adjoint_tile<S, TX>), dim3(a.ntiles), dim3(adj32_threads<TX>()), 0, s, a)
+    if (tx == 64) TG_ADJ32(64);
+    else if (tx == 32) TG_ADJ32(32);
+    else TG_ADJ32(16);
+#undef TG_ADJ32
+  } else {
+    TG_LAUNCH_TX(a.shape, k32_adjoint_classify, S, dim3(a.ntiles), s, a);
+    TG_LAUNCH_TX(a.shape, k32_adjoint, S, dim3(a.ntiles < LIST_GRID ? a.ntiles : LIST_GRID), s,
+                 a);
+  }
+  // (a tile's 256 cells are eight rounds of a workgroup; most tiles have none)
+  const int g = 4LL * a.ntiles < THIN_GRID ? 4 * a.ntiles : THIN_GRID;
   TG_LAUNCH_TX(a.shape, k32_adjoint_thin, S, dim3(g), s, a);
 }
 template void launch_coef_m<float>(const StepArgsM<float>&, bool, hipStream_t);

@@ -1,4 +1,4 @@
-"""GPU: the FP64 steps at the sizes where their tiles end -- members of one
+"""GPU: the steps at the sizes where their tiles end -- members of one
 tile less, equal and more than each tile shape, the thinnest ones, whole rows
 of boundary cells -- and on both sides of the line between a workgroup per
 tile (1024 tiles) and the tile list, against the oracle.  Bar: states, dt and
@@ -10,6 +10,7 @@ import sys
 import numpy as np
 import pytest
 
+from discrete_adjoint_amd import _lib
 from discrete_adjoint_amd.solver import Simulation
 from helpers import analytic_problem, paraboloid
 
@@ -106,3 +107,33 @@ def test_reverse_sweep_on_both_launches(oracle_lib):
                 assert np.array_equal(sim.dt_record(), dts)
                 lam, _ = sim.dual_solver(w, want_dphi=True)
                 assert np.array_equal(lam, lam_ref), (nx, graph)
+
+
+@pytest.mark.parametrize("tile", [(64, 4), (32, 8), (16, 16)])
+@pytest.mark.parametrize("nx,ny", SIZES + [(513, 512)])
+def test_fp32_reverse_step_at_tile_edges(oracle_lib, nx, ny, tile):
+    """The FP32 gather and the FP64 pass over the cells next to a thin layer
+    (eight lanes each), on both launches, over void, thin and boundary cells.
+    Bar: 1e-4 in norm, the one the sweeps of this mode are held to -- some
+    hundred FP32 roundings of terms of the result's own size, with the cells
+    whose 1/h is largest gathered in FP64.  A second step in a row reads the
+    counts the first emptied."""
+    _say(f"case fp32 reverse step {nx}x{ny} tile {tile}")
+    pb = _problem(nx, ny, 11 * nx + ny)
+    if nx * ny > 100000:
+        j, i = np.divmod(np.arange(pb.n), nx)
+        away = np.hypot(i - nx // 2, j - ny // 2) > 60
+        pb.h[away] = pb.hu[away] = pb.hv[away] = 0.0
+    orc = oracle_lib.Oracle.from_problem(pb)
+    rng = np.random.default_rng(nx + ny)
+    lam = rng.normal(size=(3, pb.n)) * np.where(rng.uniform(size=pb.n) < 0.2, 0.0, 1.0)
+    with Simulation(pb, max_steps=64, tile_x=tile[0], tile_y=tile[1],
+                    precision=_lib.TG_FWD64_ADJ32) as sim:
+        for s, dt in ((3, 0.03), (60, 0.05)):
+            ref, dphi = orc.adjoint_step([pb.h, pb.hu, pb.hv], s, dt, lam, want_dphi=True)
+            ref = np.asarray(ref).reshape(3, -1)
+            got, g = sim.adjoint_step_grad(s, dt, lam)
+            assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref), s
+            assert np.array_equal(sim.adjoint_step(s, dt, lam), got), s
+            scale = np.abs(lam).sum() * max(np.abs(pb.hu).max(), np.abs(pb.hv).max(), 1.0) * dt
+            assert abs(g - dphi) <= 1e-4 * max(abs(dphi), scale), s
