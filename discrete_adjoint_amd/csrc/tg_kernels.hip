@@ -1,15 +1,18 @@
 // FP64 kernels of the forward step and the per-step discrete adjoint on
-// uniform blocks of cells.  One workgroup = one 64x4 tile of one instance
-// (tile table), so an ensemble of uneven blocks runs in one launch.
+// uniform blocks of cells.  Tiles of 256 cells (tile table), of one member
+// each, so an ensemble of uneven blocks runs in one launch.
 //
 // Forward step s (replaces step.C:38-232, order 1):
 //   k_coef   : forward slopes -> kact (getcoef.f) + per-instance CFL min /
 //              hmax reduction (get_coef_and_eigen.C:29-180)
-//   k_dt     : dt = 0.5*min(0.5*min(dx/ev), 0.9*sqrt(hmax eps Gs/9.8)), incrtime
-//   k_update : slopes, HLL edge fluxes with outflow copies, update_states
+//   k_update : dt = 0.5*min(0.5*min(dx/ev), 0.9*sqrt(hmax eps Gs/9.8)) and
+//              incrtime; slopes, HLL edge fluxes with outflow copies,
+//              update_states
 // Reverse step s (replaces calc_jacobian + calc_adjoint, dual_solver.C:200-206):
 //   k_adjoint: gathers lambda^s_c = g_c - sum_j J_j[slot->c]^T lambda^{s+1}_j,
 //              recomputing every Jacobian block from U^s in registers.
+// Small meshes launch a workgroup per tile of each (..._tile); on large ones
+// the first pass of a step lists the tiles that have work for the second.
 #include "tg_kernels.h"
 #include "tg_math.h"
 

@@ -10,12 +10,12 @@
 //     FluxJac entries are (J1 + J2) * .5 for the leaf itself and
 //     (J_k + 0) * .5 for each finer neighbour (FluxJac::set, matrix.h:228-234);
 //   * a domain-boundary side copies the opposite side (outflow).
-// Forward step: k_leaf_coef (slopes, kact, CFL reduction), k_dt,
-// k_leaf_update (slopes, face fluxes, update_states).  Reverse step:
-// k_leaf_dualk (kact of the dual slopes), k_leaf_jac (the nine Jacobian
-// blocks of calc_jacobian, each times lambda^{s+1} of its leaf, stored where
-// the leaf that gathers it reads), k_leaf_dphi (bed-friction gradient term,
-// when asked for), k_leaf_gather (calc_adjoint's sum, in slot order).
+// Forward step: k_leaf_coef (slopes, kact, CFL reduction), k_leaf_update (dt,
+// slopes, face fluxes, update_states).  Reverse step: k_leaf_dualk (kact of
+// the dual slopes), k_leaf_jac (the nine Jacobian blocks of calc_jacobian,
+// each times lambda^{s+1} of its leaf, stored where the leaf that gathers it
+// reads), k_leaf_jac_dphi (the same with the bed-friction gradient's term
+// beside it), k_leaf_gather (calc_adjoint's sum, in slot order).
 #include "tg_kernels.h"
 #include "tg_leafops.h"
 #include "tg_math.h"
