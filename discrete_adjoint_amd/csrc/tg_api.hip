@@ -45,6 +45,7 @@ struct tg_ctx {
   // used by kernel k (0 coef, 1 update, 2 adjoint); ntiles = largest table
   std::vector<TileDev> tiles_h[NSHAPE];
   InstDev* inst_d = nullptr;
+  std::vector<InstDev> inst_up;  // what inst_d holds (empty: not known)
   TileDev* tiles_d[NSHAPE] = {};
   int nt[NSHAPE] = {};
   // mark blocks of each variant's tile table (uniform blocks)
@@ -101,11 +102,10 @@ struct tg_ctx {
   double* part_hmax = nullptr;
   // per-member reductions (k_member_reduce): each variant's tiles grouped by
   // member (member b: red_idx[v][red_off[v][b] .. red_off[v][b+1]), row-major
-  // within the member), the results on the device and in pinned host memory
+  // within the member), the results in pinned host memory
   int* red_off[NSHAPE] = {};
   int* red_idx[NSHAPE] = {};
-  double* red_out = nullptr;   // [4 * ninst]
-  double* red_host = nullptr;  // [4 * ninst], pinned
+  double* red_host = nullptr;  // [4 * ninst + 1], pinned; the last: the error word
   // leaf path: the step and state buffer whose dual kact the last reverse
   // launch made ahead (-1: none) and whether with its phi_bed derivative
   int kd_step = -1;
@@ -290,7 +290,6 @@ void free_fields(tg_ctx* ctx) {
   dfree(ctx->mat_d);
   dfree(ctx->mtab_d);
   dfree(ctx->part_hmax);
-  dfree(ctx->red_out);
   for (auto& t : ctx->red_off) dfree(t);
   for (auto& t : ctx->red_idx) dfree(t);
   if (ctx->red_host) (void)hipHostFree(ctx->red_host);
@@ -313,6 +312,7 @@ void free_fields(tg_ctx* ctx) {
   ctx->leaf = LeafDev{};
   ctx->leaves = false;
   dfree(ctx->inst_d);
+  ctx->inst_up.clear();
   for (auto& t : ctx->tiles_d) dfree(t);
   for (auto& t : ctx->blocks_d) dfree(t);
   dfree(ctx->red);
@@ -360,6 +360,12 @@ int upload_params(tg_ctx* ctx, const tg_params* p) {
   if (ctx->marks) marks_follow_selection(ctx);
   if (p)
     for (auto& I : ctx->inst_h) params_into(I, p);
+  // (a caller that steps hands the same values over with every call)
+  const bool same = ctx->inst_up.size() == ctx->inst_h.size() && !ctx->mat_d &&
+                    !std::memcmp(ctx->inst_up.data(), ctx->inst_h.data(),
+                                 sizeof(InstDev) * ctx->inst_h.size());
+  if (same) return TG_OK;
+  ctx->inst_up.clear();
   HIPCHK(ctx, hipMemcpyAsync(ctx->inst_d, ctx->inst_h.data(), sizeof(InstDev) * ctx->ninst,
                              hipMemcpyHostToDevice, ctx->stream));
   if (ctx->mat_d) {  // materials no tg_set_materials gave follow the member's parameters
@@ -372,6 +378,7 @@ int upload_params(tg_ctx* ctx, const tg_params* p) {
                                sizeof(MatDev) * ctx->mtab_h.size(), hipMemcpyHostToDevice,
                                ctx->stream));
   }
+  ctx->inst_up = ctx->inst_h;
   return TG_OK;
 }
 
@@ -703,16 +710,28 @@ void enqueue_adjoint(tg_ctx* ctx, void* const U[3], void* const lnext[3], void* 
   }
 }
 
-int check_err(tg_ctx* ctx) {
-  int e = 0;
-  HIPCHK(ctx, hipMemcpyAsync(&e, ctx->err_d, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+int err_code(tg_ctx* ctx, int e) {
   if (e & 1) return set_err(ctx, TG_ERR_NONFINITE, "non-finite state (residual.C:137-147)");
   if (e & 2) return set_err(ctx, TG_ERR_EIGEN, "eigenvalue > 1e9 (get_coef_and_eigen.C:144)");
   return TG_OK;
 }
 
-// FP64 host array of one field of one member <-> device storage
+int check_err(tg_ctx* ctx) {
+  int e = 0;
+  HIPCHK(ctx, hipMemcpyAsync(&e, ctx->err_d, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  return err_code(ctx, e);
+}
+
+// waits for what launch_member_reduce writes to red_host
+int wait_reduced(tg_ctx* ctx) {
+  HIPCHK(ctx, hipGetLastError());
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  return err_code(ctx, (int)ctx->red_host[4 * ctx->ninst]);
+}
+
+// FP64 host array of one field (or of the three, which lie one after another)
+// of one member <-> device storage
 int h2d_field(tg_ctx* ctx, void* dev_base, long long off, long long count, const double* src,
               int es = 0) {
   if ((es ? es : ctx->es) == 8)
@@ -744,8 +763,28 @@ int d2h_field(tg_ctx* ctx, const void* dev_base, long long off, long long count,
   return TG_OK;
 }
 
-int fill_stats(tg_ctx* ctx, tg_stats* st, int nst) {
-  if (!st) return TG_OK;
+// Three fields to host arrays of their own, one wait for all.
+int d2h_fields(tg_ctx* ctx, void* const f[3], long long off, long long count,
+               double* const dst[3]) {
+  if (ctx->es == 8) {
+    for (int c = 0; c < 3; c++)
+      HIPCHK(ctx, hipMemcpyAsync(dst[c], (const double*)f[c] + off, sizeof(double) * count,
+                                 hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    return TG_OK;
+  }
+  for (int c = 0; c < 3; c++) {
+    const int rc = d2h_field(ctx, f[c], off, count, dst[c]);
+    if (rc) return rc;
+  }
+  return TG_OK;
+}
+
+// The error check of what was enqueued, and the stats of the state after
+// `steps` recorded steps (st null: the check alone), with one wait.
+int finish_steps(tg_ctx* ctx, int steps, tg_stats* st, int nst) {
+  HIPCHK(ctx, hipGetLastError());
+  if (!st) return check_err(ctx);
   if (ctx->leaves)
     launch_leaf_stats(ctx->leaf,
                       Fields{(double*)ctx->U[0], (double*)ctx->U[1], (double*)ctx->U[2]},
@@ -759,37 +798,32 @@ int fill_stats(tg_ctx* ctx, tg_stats* st, int nst) {
     launch_stats32(ctx->inst_d, ctx->tiles_d[0], ctx->nt[0],
                    FieldsT<float>{(float*)ctx->U[0], (float*)ctx->U[1], (float*)ctx->U[2]},
                    ctx->part_mass, ctx->part_hmax, ctx->cfg.tiny, ctx->stream);
-  // mass, hmax, time and last dt of every member in one launch and one copy
+  // mass, hmax, time and last dt of every member in one launch
   const int nm = ctx->ninst;
-  const bool dt = ctx->rec_steps > 0;
+  const bool dt = steps > 0;
   launch_member_reduce(ctx->part_mass, ctx->part_hmax, ctx->red_off[0], ctx->red_idx[0], nm,
-                       ctx->time_d, dt ? ctx->dt_rec : nullptr, ctx->cfg.max_steps,
-                       ctx->rec_steps - 1, ctx->red_out, ctx->stream);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->red_host, ctx->red_out, sizeof(double) * 4 * nm,
-                             hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+                       ctx->time_d, dt ? ctx->dt_rec : nullptr, ctx->cfg.max_steps, steps - 1,
+                       ctx->err_d, ctx->red_host, ctx->stream);
+  const int rc = wait_reduced(ctx);
+  if (rc) return rc;
   const double* r = ctx->red_host;
   for (int b = 0; b < nst && b < nm; b++) {
     st[b].dt = dt ? r[3 * nm + b] : 0.;
     st[b].time = r[2 * nm + b];
     st[b].mass = r[b];
     st[b].hmax = r[nm + b];
-    st[b].step = ctx->rec_steps;
+    st[b].step = steps;
   }
   return TG_OK;
 }
 
 // Each member's dJ/dphi_bed from the adjoint's per-tile partials (tiles of
-// the adjoint's variant), reduced on the device.
-int member_dphi(tg_ctx* ctx, double* out) {
-  const int nm = ctx->ninst, v = ctx->sel[2];
-  launch_member_reduce(ctx->dphi_part, nullptr, ctx->red_off[v], ctx->red_idx[v], nm, nullptr,
-                       nullptr, 0, 0, ctx->red_out, ctx->stream);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->red_host, ctx->red_out, sizeof(double) * nm,
-                             hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  for (int b = 0; b < nm; b++) out[b] = ctx->red_host[b];
-  return TG_OK;
+// the adjoint's variant), reduced on the device: enqueued, then read after
+// wait_reduced.
+void enqueue_member_dphi(tg_ctx* ctx) {
+  const int v = ctx->sel[2];
+  launch_member_reduce(ctx->dphi_part, nullptr, ctx->red_off[v], ctx->red_idx[v], ctx->ninst,
+                       nullptr, nullptr, 0, 0, ctx->err_d, ctx->red_host, ctx->stream);
 }
 
 int ensure_store(tg_ctx* ctx, std::vector<void*>& v, size_t count) {
@@ -1004,8 +1038,8 @@ int forward_loop(tg_ctx* ctx, const tg_params* prm, int nsteps, const double* dt
   }
   if (endU == B)
     for (int c = 0; c < 3; c++) std::swap(ctx->U[c], ctx->Ut[c]);
-  HIPCHK(ctx, hipGetLastError());
-  rc = check_err(ctx);
+  // (a prescribed sequence moves the clocks below, before the stats read them)
+  rc = finish_steps(ctx, nsteps, dt_seq ? nullptr : stats, nstats);
   if (rc) return rc;
   float ms = 0;
   HIPCHK(ctx, hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
@@ -1021,8 +1055,9 @@ int forward_loop(tg_ctx* ctx, const tg_params* prm, int nsteps, const double* dt
       for (int s = 0; s < nsteps; s++) v += dt_seq[s];
     HIPCHK(ctx, hipMemcpy(ctx->time_d, t.data(), sizeof(double) * ctx->ninst,
                           hipMemcpyHostToDevice));
+    if (stats) return finish_steps(ctx, nsteps, stats, nstats);
   }
-  return fill_stats(ctx, stats, nstats);
+  return TG_OK;
 }
 
 // FNV-1a over 64-bit words (graph keys of staged functionals)
@@ -1084,10 +1119,8 @@ int adjoint_loop(tg_ctx* ctx, const tg_params* prm, const double* w, const int* 
     copy_state(ctx, ctx->lam[0][0], f);
     src = ctx->wsrc;
   } else if (w) {
-    for (int c = 0; c < 3; c++) {
-      rc = h2d_field(ctx, ctx->lam[0][c], 0, n, w + c * n);
-      if (rc) return rc;
-    }
+    rc = h2d_field(ctx, ctx->lam[0][0], 0, 3 * n, w);
+    if (rc) return rc;
     clear_marks(ctx, ctx->lam[0][0]);
   } else {
     src = ctx->fw;
@@ -1235,8 +1268,13 @@ int adjoint_loop(tg_ctx* ctx, const tg_params* prm, const double* w, const int* 
   }
   if (graph) cur = S % 2;
   HIPCHK(ctx, hipEventRecord(ctx->ev[3], ctx->stream));
-  HIPCHK(ctx, hipGetLastError());
-  rc = check_err(ctx);
+  if (dphi) {
+    enqueue_member_dphi(ctx);
+    rc = wait_reduced(ctx);
+  } else {
+    HIPCHK(ctx, hipGetLastError());
+    rc = check_err(ctx);
+  }
   if (rc) return rc;
   HIPCHK(ctx, hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[3]));
   ctx->adj_ms = ms;
@@ -1248,15 +1286,13 @@ int adjoint_loop(tg_ctx* ctx, const tg_params* prm, const double* w, const int* 
   HIPCHK(ctx, hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[6]));
   ctx->stored_ms = ms;
   ctx->stored_steps = nstored;
-  if (lambda0)
-    for (int c = 0; c < 3; c++) {
-      rc = d2h_field(ctx, ctx->lam[cur][c], 0, n, lambda0 + c * n);
-      if (rc) return rc;
-    }
+  if (lambda0) {
+    rc = d2h_field(ctx, ctx->lam[cur][0], 0, 3 * n, lambda0);
+    if (rc) return rc;
+  }
   ctx->member_dphi.assign(ctx->ninst, 0.);
   if (dphi) {
-    rc = member_dphi(ctx, ctx->member_dphi.data());
-    if (rc) return rc;
+    ctx->member_dphi.assign(ctx->red_host, ctx->red_host + ctx->ninst);
     double acc = 0;
     for (double v : ctx->member_dphi) acc += v;
     *dJ = acc;
@@ -1530,12 +1566,11 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
   if (!rc) rc = dalloc(ctx, &ctx->kact, sb);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->part_mass, sizeof(double) * ctx->ntiles);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->part_hmax, sizeof(double) * ctx->ntiles);
-  if (!rc) rc = dalloc(ctx, (void**)&ctx->red_out, sizeof(double) * 4 * nm);
   for (int v = 0; v < NSHAPE && !rc; v++) {
     rc = dalloc(ctx, (void**)&ctx->red_off[v], sizeof(int) * (nm + 1));
     if (!rc) rc = dalloc(ctx, (void**)&ctx->red_idx[v], sizeof(int) * (ctx->nt[v] + 1));
   }
-  if (!rc && hipHostMalloc((void**)&ctx->red_host, sizeof(double) * 4 * nm,
+  if (!rc && hipHostMalloc((void**)&ctx->red_host, sizeof(double) * (4 * nm + 1),
                            hipHostMallocDefault) != hipSuccess)
     rc = set_err(ctx, TG_ERR_NOMEM, "pinned host buffer of the per-member results");
   if (!rc) rc = dalloc(ctx, (void**)&ctx->dphi_part, sizeof(double) * ctx->ntiles);
@@ -1662,10 +1697,8 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
 
 int reset_time(tg_ctx* ctx) {
   ctx->clock_at = -1;
-  std::vector<double> z(ctx->ninst, 0.);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->time_d, z.data(), sizeof(double) * ctx->ninst,
-                             hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(ctx, hipMemsetAsync(ctx->err_d, 0, sizeof(int), ctx->stream));
+  launch_set_time(ctx->time_d, ctx->ninst, 0., ctx->err_d, ctx->stream);
+  HIPCHK(ctx, hipGetLastError());
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   return TG_OK;
 }
@@ -2029,10 +2062,8 @@ int tg_set_clock(tg_ctx* ctx, int step0, double time) {
   if (!ctx->have_state) return set_err(ctx, TG_ERR_STATE, "no state");
   ctx->step0 = step0;
   ctx->clock_at = -1;
-  std::vector<double> t(ctx->ninst, time);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->time_d, t.data(), sizeof(double) * ctx->ninst,
-                             hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  launch_set_time(ctx->time_d, ctx->ninst, time, nullptr, ctx->stream);
+  HIPCHK(ctx, hipGetLastError());
   return TG_OK;
 }
 
@@ -2058,11 +2089,7 @@ int tg_get_state(tg_ctx* ctx, double* h, double* hu, double* hv) {
   if (!ctx || !h || !hu || !hv) return TG_ERR_ARG;
   if (!ctx->have_state) return set_err(ctx, TG_ERR_STATE, "no state");
   double* dst[3] = {h, hu, hv};
-  for (int k = 0; k < 3; k++) {
-    int rc = d2h_field(ctx, ctx->U[k], 0, ctx->ncell, dst[k]);
-    if (rc) return rc;
-  }
-  return TG_OK;
+  return d2h_fields(ctx, ctx->U, 0, ctx->ncell, dst);
 }
 
 int tg_get_member_state(tg_ctx* ctx, int member, double* h, double* hu, double* hv) {
@@ -2070,11 +2097,7 @@ int tg_get_member_state(tg_ctx* ctx, int member, double* h, double* hu, double* 
   if (!ctx->have_state) return set_err(ctx, TG_ERR_STATE, "no state");
   const InstDev& I = ctx->inst_h[member];
   double* dst[3] = {h, hu, hv};
-  for (int k = 0; k < 3; k++) {
-    int rc = d2h_field(ctx, ctx->U[k], I.off, (long long)I.nx * I.ny, dst[k]);
-    if (rc) return rc;
-  }
-  return TG_OK;
+  return d2h_fields(ctx, ctx->U, I.off, (long long)I.nx * I.ny, dst);
 }
 
 int tg_forward_step(tg_ctx* ctx, const tg_params* prm, tg_stats* stats) {
@@ -2090,12 +2113,11 @@ int tg_forward_step(tg_ctx* ctx, const tg_params* prm, tg_stats* stats) {
   enqueue_step(ctx, ctx->U, ctx->Ut, ctx->rec_steps, true);
   enqueue_box_max(ctx, ctx->Ut, ctx->rec_steps);
   for (int c = 0; c < 3; c++) std::swap(ctx->U[c], ctx->Ut[c]);
-  HIPCHK(ctx, hipGetLastError());
-  rc = check_err(ctx);
+  rc = finish_steps(ctx, ctx->rec_steps + 1, stats, 1);
   if (rc) return rc;
   ctx->clock_at = ++ctx->rec_steps;
   ctx->run_steps = 0;  // single steps keep no checkpoints
-  return fill_stats(ctx, stats, 1);
+  return TG_OK;
 }
 
 int tg_forward_run(tg_ctx* ctx, const tg_params* prm, int nsteps, tg_stats* stats) {
@@ -2157,10 +2179,8 @@ int tg_get_trajectory_state(tg_ctx* ctx, int s, double* h, double* hu, double* h
   int rc = check_err(ctx);
   if (rc) return rc;
   double* dst[3] = {h, hu, hv};
-  for (int c = 0; c < 3; c++) {
-    rc = d2h_field(ctx, f[c], 0, ctx->ncell, dst[c]);
-    if (rc) return rc;
-  }
+  rc = d2h_fields(ctx, f, 0, ctx->ncell, dst);
+  if (rc) return rc;
   return TG_OK;
 }
 
@@ -2324,27 +2344,21 @@ int adjoint_step_impl(tg_ctx* ctx, const tg_params* prm, int s, double dt,
   if (rc) return rc;
   ctx->kd_step = -1;
   const long long n = ctx->ncell;
-  for (int b = 0; b < ctx->ninst; b++)  // the step's dt goes where the kernel reads it
-    HIPCHK(ctx, hipMemcpyAsync(ctx->dt_rec + (long long)b * ctx->cfg.max_steps + s, &dt,
-                               sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-  for (int c = 0; c < 3; c++) {
-    rc = h2d_field(ctx, ctx->lam[0][c], 0, n, lambda_next + c * n);
-    if (rc) return rc;
-  }
-  clear_marks(ctx, ctx->lam[0][0]);
+  rc = h2d_field(ctx, ctx->lam[0][0], 0, 3 * n, lambda_next);
+  if (rc) return rc;
+  // the step's dt goes where the kernel reads it; nothing known of lambda_next;
+  // no gradient yet
   const bool dphi = dphi_member != nullptr;
-  if (dphi) launch_zero(ctx->dphi_part, sizeof(double) * ctx->ntiles, ctx->stream);
+  launch_reverse_setup(ctx->dt_rec + s, ctx->cfg.max_steps, ctx->ninst, dt,
+                       (uint32_t*)((char*)ctx->lam[0][0] + ctx->mk_off), ctx->nsuper,
+                       (uint32_t*)ctx->dphi_part, dphi ? 2LL * ctx->ntiles : 0, ctx->stream);
   empty_lists(ctx);
   enqueue_adjoint(ctx, ctx->U, ctx->lam[0], ctx->lam[1], s, dphi);
+  if (dphi) enqueue_member_dphi(ctx);
   HIPCHK(ctx, hipGetLastError());
-  for (int c = 0; c < 3; c++) {
-    rc = d2h_field(ctx, ctx->lam[1][c], 0, n, lambda_out + c * n);
-    if (rc) return rc;
-  }
-  if (dphi) {
-    rc = member_dphi(ctx, dphi_member);
-    if (rc) return rc;
-  }
+  rc = d2h_field(ctx, ctx->lam[1][0], 0, 3 * n, lambda_out);
+  if (rc) return rc;
+  if (dphi) std::copy(ctx->red_host, ctx->red_host + ctx->ninst, dphi_member);
   ctx->run_steps = 0;  // the dt record slot was overwritten
   return TG_OK;
 }

@@ -523,9 +523,16 @@ void launch_copy_marking(const BlockDev* blocks, int nblocks, int shape, int es,
                          uint32_t* mk_dst, hipStream_t s);
 // per-member reduction of per-tile partials (member b's tiles: idx[off[b] ..
 // off[b+1])): out[b] sums, out[n + b] maxima (max_part given), out[2n + b] =
-// time[b] (given), out[3n + b] = dt_rec[b * stride + col] (given)
+// time[b] (given), out[3n + b] = dt_rec[b * stride + col] (given), out[4n] =
+// *err; out may be pinned host memory
 void launch_member_reduce(const double* sum_part, const double* max_part, const int* off,
                           const int* idx, int n, const double* time, const double* dt_rec,
-                          long long stride, int col, double* out, hipStream_t s);
+                          long long stride, int col, const int* err, double* out, hipStream_t s);
+// time[b] = t of n members, and *err (given) cleared
+void launch_set_time(double* time, int n, double t, int* err, hipStream_t s);
+// What one reverse step of its own starts from, in one launch: dt_rec[b *
+// stride] = dt of n members, n0 words at z0 and n1 at z1 cleared
+void launch_reverse_setup(double* dt_rec, long long stride, int n, double dt, uint32_t* z0,
+                          long long n0, uint32_t* z1, long long n1, hipStream_t s);
 
 }  // namespace tg

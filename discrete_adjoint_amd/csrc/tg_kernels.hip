@@ -854,13 +854,17 @@ __global__ __launch_bounds__(BLOCK) void k_copy_marking(const BlockDev* blocks, 
 // order, the lanes combine by a fixed tree, so the result does not depend on
 // the launch), out[n + b] = the max of max_part over them (when given),
 // out[2n + b] = time[b] and out[3n + b] = dt_rec[b * stride + col] (when
-// given).  Replaces a copy of every tile's partial and a host loop over them.
+// given), out[4n] = *err.  out is pinned host memory, so that one wait for the
+// stream hands a step's results to the host; two copies to it, of the error
+// word and of the results, each with a wait of its own, and the parameters'
+// upload before it took longer than the step's kernels (128 x 128 cells, a
+// host's own loop: 61 us a step against 37).
 __global__ __launch_bounds__(BLOCK) void k_member_reduce(const double* sum_part,
                                                          const double* max_part,
                                                          const int* off, const int* idx, int n,
                                                          const double* time,
                                                          const double* dt_rec, long long stride,
-                                                         int col, double* out) {
+                                                         int col, const int* err, double* out) {
   const int b = blockIdx.x;
   double s = 0., m = 0.;
   for (int j = off[b] + (int)threadIdx.x; j < off[b + 1]; j += BLOCK) {
@@ -879,7 +883,26 @@ __global__ __launch_bounds__(BLOCK) void k_member_reduce(const double* sum_part,
     if (max_part) out[n + b] = m;
     if (time) out[2 * n + b] = time[b];
     if (dt_rec) out[3 * n + b] = dt_rec[(long long)b * stride + col];
+    if (b == 0) out[4 * n] = (double)*err;
   }
+}
+
+__global__ void k_set_time(double* time, int n, double t, int* err) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b < n) time[b] = t;
+  if (b == 0 && err) *err = 0;
+}
+
+// (one launch for a copy and two fills; with the three fields of lambda in one
+// copy each way and the gradient read with lambda's wait, a reverse step from
+// and to the host takes 200 us against 263 at 301 x 257 cells)
+__global__ void k_reverse_setup(double* dt_rec, long long stride, int n, double dt, uint32_t* z0,
+                                long long n0, uint32_t* z1, long long n1) {
+  const long long t0 = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  const long long all = (long long)gridDim.x * blockDim.x;
+  for (long long i = t0; i < n; i += all) dt_rec[i * stride] = dt;
+  for (long long i = t0; i < n0; i += all) z0[i] = 0u;
+  for (long long i = t0; i < n1; i += all) z1[i] = 0u;
 }
 
 // ---------------------------------------------------------------- adjoint --
@@ -1629,10 +1652,21 @@ void launch_copy_marking(const BlockDev* blocks, int nblocks, int shape, int es,
 
 void launch_member_reduce(const double* sum_part, const double* max_part, const int* off,
                           const int* idx, int n, const double* time, const double* dt_rec,
-                          long long stride, int col, double* out, hipStream_t s) {
+                          long long stride, int col, const int* err, double* out,
+                          hipStream_t s) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_member_reduce, dim3(n), dim3(BLOCK), 0, s, sum_part, max_part, off, idx,
-                     n, time, dt_rec, stride, col, out);
+                     n, time, dt_rec, stride, col, err, out);
+}
+void launch_set_time(double* time, int n, double t, int* err, hipStream_t s) {
+  hipLaunchKernelGGL(k_set_time, dim3((n + 63) / 64), dim3(64), 0, s, time, n, t, err);
+}
+void launch_reverse_setup(double* dt_rec, long long stride, int n, double dt, uint32_t* z0,
+                          long long n0, uint32_t* z1, long long n1, hipStream_t s) {
+  long long m = n0 > n1 ? n0 : n1;
+  if (n > m) m = n;
+  hipLaunchKernelGGL(k_reverse_setup, dim3(grid_for(m)), dim3(256), 0, s, dt_rec, stride, n, dt,
+                     z0, n0, z1, n1);
 }
 
 }  // namespace tg
