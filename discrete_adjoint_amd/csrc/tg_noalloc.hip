@@ -1,8 +1,7 @@
 // tg_step_noalloc: one order-1 forward step of a uniform block with every
 // intermediate kept in a fixed device array of this file (no device memory
 // is allocated or freed by the call).  It runs the kernels of
-// tg_forward_step -- coefficient / CFL pass, dt, classifying pass and
-// update -- on caller-owned device arrays, so its results are those of
+// tg_forward_step -- coefficient / CFL pass and update -- on caller-owned device arrays, so its results are those of
 // tg_forward_step on the same state, bit for bit.
 //
 // Scratch: the member record, the tile and mark-block tables of the 64x4
