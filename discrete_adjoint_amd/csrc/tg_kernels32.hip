@@ -210,16 +210,23 @@ __global__ __launch_bounds__(BLOCK) void k32_update(StepArgsM<S> a) {
   __shared__ L32 L;
   const TileDev t = a.tiles[blockIdx.x];
   const InstDev I = a.inst[t.inst];
-  const double dt = step_dt(a, t.inst, t.x0 == 0 && t.y0 == 0);
+  const bool own = t.x0 == 0 && t.y0 == 0;  // keeps the member's records
   // the tile and its four side tiles of U marked +0.0: zero fluxes, no
   // sources (h < tiny), so U^{s+1} = +0.0 + (-dtdx * 0 - dtdy * 0) = +0.0 for
-  // a finite dt; nothing to do when the output tile is marked +0.0 already
-  if (a.mk_in && a.mk_out && isfinite(dt) && tile_marked_zero<TX>(a.mk_out, t, a.zbytes) &&
+  // a finite dt; nothing to do when the output tile is marked +0.0 already.
+  // (Looked at before dt is made, which most workgroups of a large mesh then
+  // never do; a dt that is not finite makes every cell so and is reported by
+  // the one that keeps the records, as the state it would give is.)
+  const bool skip =
+      a.mk_in && a.mk_out && tile_marked_zero<TX>(a.mk_out, t, a.zbytes) &&
       tile_marked_zero<TX>(a.mk_in, t, a.zbytes) && side_tile_zero<TX>(a.mk_in, t, I, 0, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 1, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 2, a.zbytes) &&
-      side_tile_zero<TX>(a.mk_in, t, I, 3, a.zbytes))
-    return;
+      side_tile_zero<TX>(a.mk_in, t, I, 3, a.zbytes);
+  if (skip && !own) return;
+  const double dt = step_dt(a, t.inst, own);
+  if (own && threadIdx.x == 0 && !isfinite(dt)) atomicOr(a.err, 1);
+  if (skip && isfinite(dt)) return;
   const Cell q = cell_of<TX>(t, I);
   const long long nx = I.nx;
   const W tiny = (W)a.tiny, gamma = (W)a.gamma;
@@ -774,15 +781,14 @@ __device__ __forceinline__ M3T<F> nbr_part(const InstDev& I, const Cell& q, int 
   return J;
 }
 
-// The gather of one cell in FP32: adj = sum of the transposed Jacobian blocks
+// The gather of one cell in arithmetic type F: adj = sum of the transposed Jacobian blocks
 // (the self block without its identity) applied to lambda^{s+1}; nbr(s)
 // returns the record of neighbour slot s (1 E, 2 N, 3 W, 4 S).  Returns the
 // cell's dJ/dphi_bed term (0 unless want_dphi).
-template <class S, class NBR>
+template <class S, class F, class NBR>
 __device__ __forceinline__ double gather(const AdjArgsM<S>& a, const InstDev& I, const Cell& q,
-                                         const DualInfoT<float>& self, NBR&& nbr, double dtd,
-                                         float adj[3], bool want_dphi) {
-  using F = float;
+                                         const DualInfoT<F>& self, NBR&& nbr, double dtd,
+                                         F adj[3], bool want_dphi) {
   const long long c = q.c;
   const F dt = (F)dtd, dtdx = (F)(dtd * I.inv_dx), dtdy = (F)(dtd * I.inv_dy);
   const bool has[5] = {true, q.hasE, q.hasN, q.hasW, q.hasS};
@@ -919,7 +925,7 @@ __device__ __forceinline__ void adjoint32_tile(const AdjArgsM<S>& a, const TileD
     } else {
       const S lc[3] = {a.lam_next.h[c], a.lam_next.hu[c], a.lam_next.hv[c]};
       float adj[3];
-      dphi = gather<S>(a, I, q, self, [&](int s) { return lds_get(L, rn(s)); }, dtd, adj,
+      dphi = gather<S, float>(a, I, q, self, [&](int s) { return lds_get(L, rn(s)); }, dtd, adj,
                               want_dphi);
       // lambda^s = -(K_self - I)^T lambda_c - sum K_n^T lambda_n = lambda_c - adj;
       // flush |lambda| < 1e-16 (calc_adjoint.C:150-152)
@@ -990,14 +996,20 @@ __global__ __launch_bounds__(adj32_threads<TX>()) void k32_adjoint_tile(AdjArgsM
 }
 
 // The cells the gather listed (a thin layer in their stencil), gathered in
-// FP64 from global memory: lane 0 of eight takes the cell's record, lanes 1-4
-// its E, N, W and S neighbours', each then the block and the face derivative
-// of its side, and lane 0 adds them in the gather's order.  Some thousand
-// cells at a front leave the chip idle, so the time is one cell's chain of
-// loads and FP64 arithmetic: a thread per cell evaluates the neighbours'
-// records one after another, three times over (389 x 301 cells: 34.5 us
-// against 19.6).  A fixed grid strides over the list, so the launch does not depend on the
-// count (graph capture).
+// FP64 from global memory, in one of two ways.  A fixed grid strides over the
+// list and the count decides on the device, so the launch does not depend on
+// it (graph capture).
+//
+// What the grid holds at once at eight lanes a cell: lane 0 takes the cell's
+// record, lanes 1-4 its E, N, W and S neighbours', each then the block and the
+// face derivative of its side, and lane 0 adds them in the gather's order.
+// The time there is one cell's chain of loads and FP64 arithmetic, which a
+// thread per cell walks for the neighbours' records one after another, three
+// times over (a front of some thousand cells, 389 x 301: 34.5 us against 19.6).
+// More cells than that (16,384): a thread each.  The lanes' time goes up by a
+// round at a time, the threads' stays one chain until 131,072 (96 members of
+// 64 to 512 cells a side, 32,768 to 65,536 thin cells: 73 us by lanes alone,
+// 52 by threads).
 constexpr int THIN_LANES = 8, THIN_CELLS = BLOCK / THIN_LANES;
 struct ThinLds {
   DualInfoT<double> self[THIN_CELLS];
@@ -1005,6 +1017,60 @@ struct ThinLds {
   double lam[5][THIN_CELLS][3];
   FaceDk<double> dk[5][THIN_CELLS];
 };
+
+template <int TX>
+__device__ __forceinline__ Cell thin_cell(const TileDev& t, const InstDev& I, int thread) {
+  Cell q;
+  q.i = t.x0 + thread % TX;
+  q.j = t.y0 + thread / TX;
+  q.act = true;
+  q.c = I.off + (long long)q.j * I.nx + q.i;
+  q.hasE = q.i + 1 < I.nx;
+  q.hasW = q.i > 0;
+  q.hasN = q.j + 1 < I.ny;
+  q.hasS = q.j > 0;
+  return q;
+}
+template <class S>
+__device__ __forceinline__ void thin_store(const AdjArgsM<S>& a, long long c,
+                                           const DualInfoT<double>& self, const double adj[3]) {
+  S out[3];
+  for (int j = 0; j < 3; j++) {
+    out[j] = self.nz ? (S)(self.lam[j] - adj[j]) : (S)0;
+    if (fabs((double)out[j]) < 1e-16) out[j] = (S)0;
+  }
+  a.lam_h[c] = out[0];
+  a.lam_hu[c] = out[1];
+  a.lam_hv[c] = out[2];
+}
+
+template <class S, int TX>
+__device__ __forceinline__ void thin_by_thread(const AdjArgsM<S>& a, int n) {
+  const bool want_dphi = a.dphi_part != nullptr;
+  for (int e = blockIdx.x * BLOCK + threadIdx.x; e < n; e += gridDim.x * BLOCK) {
+    const int2 item = a.thin_list[e];
+    const TileDev t = a.tiles[item.x];
+    const InstDev I = a.inst[t.inst];
+    const Cell q = thin_cell<TX>(t, I, item.y);
+    const double dtd = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
+    const DualInfoT<double> self = dual_info<S, double>(a, I, q.i, q.j, want_dphi);
+    double adj[3];
+    // neighbour s (1 E, 2 N, 3 W, 4 S); an absent neighbour (domain edge)
+    // is never read by the gather -- return the cell's own record instead of
+    // touching memory outside the block
+    auto nbr = [&](int s) {
+      const bool present = s == 1 ? q.hasE : (s == 2 ? q.hasN : (s == 3 ? q.hasW : q.hasS));
+      if (!present) return self;
+      const int i = q.i + (s == 1 ? 1 : (s == 3 ? -1 : 0));
+      const int j = q.j + (s == 2 ? 1 : (s == 4 ? -1 : 0));
+      return dual_info<S, double>(a, I, i, j, want_dphi);
+    };
+    const double dphi = gather<S, double>(a, I, q, self, nbr, dtd, adj, want_dphi);
+    thin_store(a, q.c, self, adj);
+    if (want_dphi) atomicAdd(&a.dphi_part[item.x], dphi);
+  }
+}
+
 template <class S, int TX>
 __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
   using F = double;
@@ -1016,6 +1082,10 @@ __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
   const int2 first = a.thin_list[e1 < a.ncell ? e1 : 0];
   const int n = *a.thin_count;
   if (blockIdx.x == 0 && threadIdx.x == 0) *a.tile_count = *a.thin_next = 0;
+  if (n > THIN_CELLS * (int)gridDim.x) {
+    thin_by_thread<S, TX>(a, n);
+    return;
+  }
 #pragma unroll 1
   for (int e0 = e1 - g; e0 < n; e0 += (int)gridDim.x * THIN_CELLS) {
     const int e = e0 + g;
@@ -1024,15 +1094,7 @@ __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
     if (e >= n) item = make_int2(0, 0);
     const TileDev t = a.tiles[item.x];
     const InstDev I = a.inst[t.inst];
-    Cell q;
-    q.i = t.x0 + item.y % TX;
-    q.j = t.y0 + item.y / TX;
-    q.act = true;
-    q.c = I.off + (long long)q.j * I.nx + q.i;
-    q.hasE = q.i + 1 < I.nx;
-    q.hasW = q.i > 0;
-    q.hasN = q.j + 1 < I.ny;
-    q.hasS = q.j > 0;
+    const Cell q = thin_cell<TX>(t, I, item.y);
     const double dt = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
     const double dtdx = dt * I.inv_dx, dtdy = dt * I.inv_dy;
     const bool has[5] = {true, q.hasE, q.hasN, q.hasW, q.hasS};
@@ -1077,14 +1139,7 @@ __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
           if (has[k]) accum_T(adj, L.block[k][g], L.lam[k][g]);
         }
       }
-      S out[3];
-      for (int j = 0; j < 3; j++) {
-        out[j] = R.nz ? (S)(R.lam[j] - adj[j]) : (S)0;
-        if (fabs((double)out[j]) < 1e-16) out[j] = (S)0;
-      }
-      a.lam_h[c] = out[0];
-      a.lam_hu[c] = out[1];
-      a.lam_hv[c] = out[2];
+      thin_store(a, c, R, adj);
       if (want_dphi) {
         FaceDk<F> K[5] = {};
 #pragma unroll

@@ -109,17 +109,22 @@ def test_reverse_sweep_on_both_launches(oracle_lib):
                 assert np.array_equal(lam, lam_ref), (nx, graph)
 
 
+@pytest.mark.parametrize("thin", [0.1, 0.5])
 @pytest.mark.parametrize("tile", [(64, 4), (32, 8), (16, 16)])
 @pytest.mark.parametrize("nx,ny", SIZES + [(513, 512)])
-def test_fp32_reverse_step_at_tile_edges(oracle_lib, nx, ny, tile):
+def test_fp32_reverse_step_at_tile_edges(oracle_lib, nx, ny, tile, thin):
     """The FP32 gather and the FP64 pass over the cells next to a thin layer
-    (eight lanes each), on both launches, over void, thin and boundary cells.
+    (eight lanes each or, where most cells are such, a thread each), on both
+    launches, over void, thin and boundary cells.
     Bar: 1e-4 in norm, the one the sweeps of this mode are held to -- some
     hundred FP32 roundings of terms of the result's own size, with the cells
     whose 1/h is largest gathered in FP64.  A second step in a row reads the
     counts the first emptied."""
-    _say(f"case fp32 reverse step {nx}x{ny} tile {tile}")
+    _say(f"case fp32 reverse step {nx}x{ny} tile {tile} thin {thin}")
     pb = _problem(nx, ny, 11 * nx + ny)
+    if thin > 0.1:
+        more = np.random.default_rng(nx * ny).uniform(size=pb.n) < thin
+        pb.h[more], pb.hu[more], pb.hv[more] = 5e-4, 3e-3, -2e-3
     if nx * ny > 100000:
         j, i = np.divmod(np.arange(pb.n), nx)
         away = np.hypot(i - nx // 2, j - ny // 2) > 60
