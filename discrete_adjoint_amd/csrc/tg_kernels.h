@@ -402,9 +402,8 @@ constexpr int LIST_GRID = 4096;
 // tiles, held to three a CU by their LDS, queue: the block passes leave a
 // block after a few words and only listed tiles take that LDS.
 constexpr int TILE_LAUNCH_MAX = 1024;
-// workgroups of the FP64 adjoint's list walk, and its waves per SIMD
+// workgroups of the FP64 adjoint's list walk
 constexpr int ADJ_GRID = 2048;
-constexpr int ADJ_WAVES = 3;
 
 template <class S>
 void launch_coef_m(const StepArgsM<S>& a, bool reduce, hipStream_t s);

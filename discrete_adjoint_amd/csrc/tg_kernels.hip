@@ -23,9 +23,6 @@ namespace {
 __device__ __forceinline__ unsigned long long dbits(double v) {
   return (unsigned long long)__double_as_longlong(v);
 }
-__device__ __forceinline__ double bitsd(unsigned long long v) {
-  return __longlong_as_double((long long)v);
-}
 
 __device__ __forceinline__ double wave_min(double v) {
 #pragma unroll
