@@ -140,6 +140,18 @@ __device__ __forceinline__ int mark_byte(const T& t) {
   return ((t.y0 % MARK_H) / TY) * (MARK_W / TX) + (t.x0 % MARK_W) / TX;
 }
 
+// Whether the tile of this workgroup holds +0.0 in a buffer that the launch
+// writes, per its marks (every thread calls it and all get the same answer).
+// The word's other bytes are stored by other workgroups of the same launch, so
+// only the tile's own byte is looked at, which this workgroup alone stores, and
+// not before a barrier.  bytes 0 (timing: the bytes follow another shape): the
+// whole word, read once for all waves.
+template <int TX, class T>
+__device__ __forceinline__ bool out_marked_zero(const uint32_t* mk, const T& t, int bytes) {
+  if (bytes) return ((const unsigned char*)(mk + t.mw))[mark_byte<TX>(t)] == 1;
+  return __syncthreads_or(threadIdx.x == 0 && mk[t.mw] == MARK_FULL);
+}
+
 struct Fields {
   const double* h;
   const double* hu;

@@ -98,20 +98,18 @@ __device__ __forceinline__ void mark_store(uint32_t* mk, const T& t, bool all) {
 // Update: the block and the four side blocks of U are +0.0 -- every cell
 // and side neighbour has h < tiny, so the fluxes are zero and there are no
 // sources, and U^{s+1} = U^s - dtdx*(0 - 0) - dtdy*(0 - 0) = +0.0 for a
-// finite dt -- and the block of the output already holds +0.0.
+// finite dt -- so nothing is to do where the output already holds +0.0.
 template <class Blk>
-__device__ __forceinline__ bool update_skip(const uint32_t* in, const uint32_t* out,
-                                            const Blk& B) {
-  return in[B.mw] == MARK_FULL && out[B.mw] == MARK_FULL &&
+__device__ __forceinline__ bool update_skip(const uint32_t* in, const Blk& B) {
+  return in[B.mw] == MARK_FULL &&
          (B.mwW < 0 || in[B.mwW] == MARK_FULL) && (B.mwE < 0 || in[B.mwE] == MARK_FULL) &&
          (B.mwS < 0 || in[B.mwS] == MARK_FULL) && (B.mwN < 0 || in[B.mwN] == MARK_FULL);
 }
 // Adjoint: the block of U^s is +0.0 (void cells: lambda^s = +0.0), that of
-// lambda^{s+1} too when the gradient is wanted (no bed-friction terms), and
-// the block of lambda^s already holds +0.0.
-__device__ __forceinline__ bool adjoint_skip(const uint32_t* mu, const uint32_t* ml,
-                                             const uint32_t* out, int mw) {
-  return mu[mw] == MARK_FULL && out[mw] == MARK_FULL && (!ml || ml[mw] == MARK_FULL);
+// lambda^{s+1} too when the gradient is wanted (no bed-friction terms): nothing
+// is to do where lambda^s already holds +0.0.
+__device__ __forceinline__ bool adjoint_skip(const uint32_t* mu, const uint32_t* ml, int mw) {
+  return mu[mw] == MARK_FULL && (!ml || ml[mw] == MARK_FULL);
 }
 // the byte of block word mw that tile byte b owns
 __device__ __forceinline__ void mark_byte_store(uint32_t* mk, int mw, int b, bool zero) {
@@ -242,7 +240,7 @@ __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
   constexpr int TY = BLOCK / TX;
   // (the block table is indexed by mark word)
   const BlockDev B = a.blocks[blockIdx.x];
-  if (a.mk_in && update_skip(a.mk_in, a.mk_out, B)) return;
+  if (a.mk_in && a.mk_out[B.mw] == MARK_FULL && update_skip(a.mk_in, B)) return;
   __shared__ int s_n;
   __shared__ unsigned s_wet;
   __shared__ unsigned short s_cell[4 * BLOCK];
@@ -758,7 +756,9 @@ __global__ __launch_bounds__(face_threads<TX>()) void k_update_tile(StepArgs a) 
   const int tile = tile_of(a);
   const TileDev t = a.tiles[tile];
   const double dt = step_dt(a, t.inst, t.x0 == 0 && t.y0 == 0);
-  if (a.mk_in && isfinite(dt) && update_skip(a.mk_in, a.mk_out, t)) return;
+  if (a.mk_in && isfinite(dt) && update_skip(a.mk_in, t) &&
+      out_marked_zero<TX>(a.mk_out, t, a.zbytes))
+    return;
   update_tile<TX, face_threads<TX>(), true>(a, ref_of(t, tile), dt, L);
 }
 
@@ -1203,8 +1203,8 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_classify(AdjArgs a) {
   // the block record is read alongside the mark words (a skipped block
   // wastes its 64 bytes; a listed one saves a round trip)
   const BlockDev B = a.blocks[blockIdx.x];
-  if (a.mk_out &&
-      adjoint_skip(a.mk_U, a.dphi_part ? a.mk_lnext : nullptr, a.mk_out, (int)blockIdx.x))
+  if (a.mk_out && a.mk_out[blockIdx.x] == MARK_FULL &&
+      adjoint_skip(a.mk_U, a.dphi_part ? a.mk_lnext : nullptr, (int)blockIdx.x))
     return;
   __shared__ unsigned s_busy;
   if (threadIdx.x == 0) s_busy = 0u;
@@ -1516,7 +1516,9 @@ __global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint_tile(AdjArgs a) {
   __shared__ DualLds<TX, DPHI> L;
   const int tile = tile_of(a);
   const TileDev t = a.tiles[tile];
-  if (a.mk_out && adjoint_skip(a.mk_U, DPHI ? a.mk_lnext : nullptr, a.mk_out, t.mw)) return;
+  if (a.mk_out && adjoint_skip(a.mk_U, DPHI ? a.mk_lnext : nullptr, t.mw) &&
+      out_marked_zero<TX>(a.mk_out, t, a.l_bytes))
+    return;
   adjoint_tile<TX, DPHI, true>(a, ref_of(t, tile), L);
 }
 
