@@ -71,9 +71,10 @@ __device__ __forceinline__ Cell cell_of(const TileDev& t, const InstDev& I) {
 
 // ------------------------------------------------------------- zero marks --
 
-// Tile t is known to hold +0.0 in all three fields of a marked buffer: its
-// block's word is MARK_FULL, or its own byte is 1 and the bytes follow this
-// tile shape (bytes != 0).
+// Tile t is known to hold +0.0 in all three fields of a marked buffer that the
+// launch does not write (one that it writes: out_marked_zero): its block's word
+// is MARK_FULL, or its own byte is 1 and the bytes follow this tile shape
+// (bytes != 0).
 template <int TX>
 __device__ __forceinline__ bool tile_marked_zero(const uint32_t* mk, const TileDev& t,
                                                  int bytes) {
@@ -218,11 +219,12 @@ __global__ __launch_bounds__(BLOCK) void k32_update(StepArgsM<S> a) {
   // never do; a dt that is not finite makes every cell so and is reported by
   // the one that keeps the records, as the state it would give is.)
   const bool skip =
-      a.mk_in && a.mk_out && tile_marked_zero<TX>(a.mk_out, t, a.zbytes) &&
-      tile_marked_zero<TX>(a.mk_in, t, a.zbytes) && side_tile_zero<TX>(a.mk_in, t, I, 0, a.zbytes) &&
+      a.mk_in && a.mk_out && tile_marked_zero<TX>(a.mk_in, t, a.zbytes) &&
+      side_tile_zero<TX>(a.mk_in, t, I, 0, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 1, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 2, a.zbytes) &&
-      side_tile_zero<TX>(a.mk_in, t, I, 3, a.zbytes);
+      side_tile_zero<TX>(a.mk_in, t, I, 3, a.zbytes) &&
+      out_marked_zero<TX>(a.mk_out, t, a.zbytes);
   if (skip && !own) return;
   const double dt = step_dt(a, t.inst, own);
   if (own && threadIdx.x == 0 && !isfinite(dt)) atomicOr(a.err, 1);
@@ -840,7 +842,8 @@ __device__ __forceinline__ bool adjoint32_void(const AdjArgsM<S>& a, const TileD
                                                const Cell& q) {
   if (a.mk_out && tile_marked_zero<TX>(a.mk_U, t, a.u_bytes) &&
       (!a.dphi_part || tile_marked_zero<TX>(a.mk_lnext, t, a.l_bytes))) {
-    if (tile_marked_zero<TX>(a.mk_out, t, a.l_bytes)) return true;
+    if (out_marked_zero<TX>(a.mk_out, t, a.l_bytes)) return true;
+    __syncthreads();  // every wave has read the byte that thread 0 stores below
   } else {
     bool busy = false;
     if (q.act) {

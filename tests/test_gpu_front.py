@@ -10,6 +10,7 @@ import sys
 import numpy as np
 import pytest
 
+from discrete_adjoint_amd import _lib
 from discrete_adjoint_amd.solver import Simulation
 from helpers import analytic_problem, paraboloid
 
@@ -134,3 +135,29 @@ def test_a_tile_is_left_alone_by_its_own_mark(oracle_lib):
             short.append(cells)
     assert short[1][1] - short[0][1] == 64 * 4   # update
     assert short[1][2] - short[0][2] == 64 * 4   # reverse step
+
+
+@pytest.mark.parametrize("precision", [_lib.TG_FP32, _lib.TG_MIXED, _lib.TG_FWD64_ADJ32])
+@pytest.mark.parametrize("nx,ny,i0,j0", MESHES)
+def test_front_in_fp32_modes(nx, ny, i0, j0, precision):
+    """The FP32 reverse sweeps, whose marks leave tiles alone, equal their own
+    single reverse steps from uploaded states, which have no marks, bit for bit:
+    a cell left unwritten under a mark that says +0.0 would keep an earlier
+    step's lambda."""
+    _say(f"case fp32 front {nx}x{ny} precision {precision}")
+    pb = _embedded(_problem(), nx, ny, i0, j0)
+    w = _grow(_weights(_problem()), nx, ny, i0, j0)
+    with Simulation(pb, precision=precision, checkpoint_every=9) as sim:
+        for _ in range(2):  # the second time over the buffers of the first
+            sim.set_state(pb.h, pb.hu, pb.hv)
+            sim.run()
+            got = [sim.dual_solver(w, want_dphi=d)[0] for d in (False, True)]
+        dts = sim.dt_record()
+        with Simulation(pb, precision=precision, max_steps=STEPS) as one:
+            lam = w
+            for s in range(STEPS - 1, -1, -1):
+                one.set_state(*sim.trajectory_state(s))
+                lam = one.adjoint_step(s, dts[s], lam)
+    assert np.isfinite(lam).all() and np.abs(lam).max() > 1.0
+    for g in got:
+        assert np.array_equal(g, lam)
