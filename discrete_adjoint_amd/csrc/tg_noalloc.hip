@@ -23,7 +23,8 @@ namespace {
 
 constexpr long long NA_MAX_CELLS = TG_NOALLOC_MAX_CELLS;
 constexpr int NA_MAX_TILES = TG_NOALLOC_MAX_CELLS / 256 * 2;  // 64x4 tiles, partial edges
-constexpr int NA_MAX_BLOCKS = NA_MAX_TILES / 2;                // 64x16 mark blocks
+// 64x16 mark blocks: a block of at most four rows has one for each of its tiles
+constexpr int NA_MAX_BLOCKS = NA_MAX_TILES;
 constexpr int NA_MAX_DEVICES = 64;
 
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }

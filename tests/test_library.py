@@ -162,3 +162,19 @@ def test_fractal_dem_is_seeded_and_scaled():
     c = problems.fractal_dem(129, 800.0, 0.8, 8)
     assert np.array_equal(a, b) and not np.array_equal(a, c)
     assert a.min() == 0.0 and a.max() == pytest.approx(800.0, rel=1e-6)
+
+
+def test_noalloc_scratch_holds_every_accepted_block():
+    """tg_step_noalloc accepts up to 2^20 cells in up to 8192 tiles of 64 x 4
+    cells; its fixed array holds, for every such shape, kact of the cells, a
+    48-byte record and a 40-byte list entry per tile and a 64-byte record per
+    64 x 16 mark block.  A block of at most four rows has as many mark blocks as
+    tiles."""
+    lib = _lib.load()
+    up = lambda a, b: -(-a // b)
+    for nx, ny in [(524288, 1), (524288, 2), (262208, 3), (262144, 4), (64, 16384), (1024, 1024)]:
+        tiles, blocks = up(nx, 64) * up(ny, 4), up(nx, 64) * up(ny, 16)
+        assert nx * ny <= 1 << 20 and blocks <= tiles <= 8192
+        # (8192 tiles and 2^20 cells whatever the shape)
+        need = (8 << 20) + 8192 * (48 + 40) + blocks * 64
+        assert lib.tg_noalloc_scratch_bytes() >= need, (nx, ny)

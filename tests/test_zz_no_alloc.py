@@ -11,7 +11,7 @@ import pytest
 
 from discrete_adjoint_amd import _lib
 from discrete_adjoint_amd.solver import Simulation
-from helpers import small_flow_problem
+from helpers import analytic_problem, small_flow_problem
 from hipmem import DeviceArray, synchronize
 
 pytestmark = pytest.mark.gpu
@@ -84,3 +84,22 @@ def test_noalloc_rejects_blocks_beyond_its_scratch():
                              8, None, C.byref(dt))
     assert rc == _lib.TG_ERR_TOO_LARGE
     assert lib.tg_noalloc_scratch_bytes() < 16 << 20
+
+
+@pytest.mark.parametrize("nx,ny", [(524288, 1), (262208, 3), (64, 16384)])
+def test_noalloc_step_of_the_flattest_blocks(nx, ny):
+    """The accepted shapes with the most mark blocks (8192 and 4097: one for
+    every tile) and the fewest, mostly dry."""
+    _say(f"case noalloc {nx}x{ny}")
+    pb = analytic_problem(nx, ny, 10.0, slope_x_deg=20.0, slope_y_deg=3.0, phi_int=32.0,
+                          phi_bed=15.0, nsteps=3)
+    rng = np.random.default_rng(nx)
+    at = rng.integers(0, pb.n, 400)[:, None] + np.arange(6)   # short piles all over it
+    pb.h[at[at < pb.n]] = 3.0
+    pb.h[-3:] = 2.0                                           # and in the last tile
+    cfg, prm, ref = _reference(pb, 3)
+    got = _noalloc_chain(pb, cfg, prm, 3)
+    for s, ((U, dt), (Ur, dtr, _)) in enumerate(zip(got, ref)):
+        assert dt == dtr and 0 < dt < 1, s
+        for a, b in zip(U, Ur):
+            assert np.array_equal(a, b), s
