@@ -925,10 +925,10 @@ __device__ __forceinline__ double swap_pair(double v) {
 // zero (rows 0 and n have no t column), then the gather lambda^s = g -
 // sum_j J_j^T lambda_j, whose running sum the pair hands back and forth in the
 // reference's order self, S, E, N, W (neighbor[0..3] with positive_x_side =
-// 1).  The products left out are exact zeros, and adding a zero to a running
-// sum that starts at +0.0 changes nothing, so the result is the reference's
-// bit for bit.  The bed-friction gradient's face fluxes come out of the same
-// evaluation.
+// 1).  The products left out are exact zeros where lambda^{s+1} is finite, and
+// adding a zero to a running sum that starts at +0.0 changes nothing, so the
+// result is the reference's bit for bit.  The bed-friction gradient's face
+// fluxes come out of the same evaluation.
 //
 // What bounds it: FP64 instruction issue (52 % of the issue slots at 128
 // VGPRs, four waves per SIMD) and, per tile, three round trips to memory (list
@@ -1448,7 +1448,13 @@ __device__ __forceinline__ void adjoint_tile(const AdjArgs& a, const TileRef& t,
         };
         const double A1 = isx ? An0 : At0l, A2 = isx ? At0l : An0;
         const double A1n = isx ? Ann : Atn, A2n = isx ? Atn : Ann;
-        const double A0 = a0 * (sA * A.a00), A0n = a0 * (pA * A.a0n), Att = at * (sA * A.att);
+        const double A0 = a0 * (sA * A.a00), A0n = a0 * (pA * A.a0n);
+        const double B0 = b0 * (sB * B.a00), B0n = b0 * (pB * B.a0n);
+        double Att = at * (sA * A.att), Btt = bt * (sB * B.att);
+        if (!isfinite(a0 + an + b0 + bn)) {  // 0 * inf: the products left out count
+          Att += 0. * a0 + 0. * an;
+          Btt += 0. * b0 + 0. * bn;
+        }
         auto addA = [&]() {
           r0 += A0; rn += A0n; rt += Att;
           r0 += A1; rn += A1n;
@@ -1456,7 +1462,6 @@ __device__ __forceinline__ void adjoint_tile(const AdjArgs& a, const TileRef& t,
         };
         const double B1 = isx ? Bn0 : Bt0l, B2 = isx ? Bt0l : Bn0;
         const double B1n = isx ? Bnn : Btn, B2n = isx ? Btn : Bnn;
-        const double B0 = b0 * (sB * B.a00), B0n = b0 * (pB * B.a0n), Btt = bt * (sB * B.att);
         auto addB = [&]() {
           r0 += B0; rn += B0n; rt += Btt;
           r0 += B1; rn += B1n;

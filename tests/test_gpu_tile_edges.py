@@ -142,3 +142,33 @@ def test_fp32_reverse_step_at_tile_edges(oracle_lib, nx, ny, tile, thin):
             assert np.array_equal(sim.adjoint_step(s, dt, lam), got), s
             scale = np.abs(lam).sum() * max(np.abs(pb.hu).max(), np.abs(pb.hv).max(), 1.0) * dt
             assert abs(g - dphi) <= 1e-4 * max(abs(dphi), scale), s
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("nx,ny", [(66, 33), (513, 512)])
+def test_reverse_step_of_a_lambda_that_is_not_finite(oracle_lib, nx, ny, value):
+    """An infinite or undefined entry of lambda^{s+1} (an adjoint that has
+    overflowed) reaches every cell with h != 0 that the reference's full 3 x 3
+    products carry it to: 0 * inf is not a zero that may be left out.  Void
+    cells are +0.0 whatever lambda^{s+1} is."""
+    _say(f"case reverse step {nx}x{ny} lambda {value}")
+    pb = _problem(nx, ny, nx)
+    if nx > 100:
+        j, i = np.divmod(np.arange(pb.n), nx)
+        away = np.hypot(i - nx // 2, j - ny // 2) > 40
+        pb.h[away] = pb.hu[away] = pb.hv[away] = 0.0
+    orc = oracle_lib.Oracle.from_problem(pb)
+    rng = np.random.default_rng(nx + ny)
+    on = pb.h != 0.0
+    with Simulation(pb, max_steps=64) as sim:
+        for k in range(3):
+            lam = rng.normal(size=(3, pb.n))
+            lam[k, rng.choice(np.flatnonzero(on), 5, replace=False)] = value
+            lam[k, np.flatnonzero(on)[[0, -1]]] = value
+            lam[k, [0, nx - 1, pb.n - 1]] = value   # the member's corners
+            ref, _ = orc.adjoint_step([pb.h, pb.hu, pb.hv], 60, 0.05, lam)
+            ref = np.where(on, ref, 0.0)
+            assert 0 < np.count_nonzero(~np.isfinite(ref)) < 200
+            for got in (sim.adjoint_step(60, 0.05, lam), sim.adjoint_step_grad(60, 0.05, lam)[0]):
+                bad = np.argwhere((got != ref) & ~(np.isnan(got) & np.isnan(ref)))
+                assert len(bad) == 0, (k, len(bad), bad[:3], got[tuple(bad[0])], ref[tuple(bad[0])])
