@@ -780,11 +780,28 @@ int d2h_fields(tg_ctx* ctx, void* const f[3], long long off, long long count,
   return TG_OK;
 }
 
+// What the steps' error check said of `steps` recorded steps.  Where their
+// passes leave tiles alone without a look at dt, a dt that was not finite still
+// has to reach those.
+int steps_failed(tg_ctx* ctx, int steps, int rc) {
+  if (rc != TG_ERR_NONFINITE || ctx->leaves || (fwd64(ctx) && tile_launch(ctx, 0) != 0)) return rc;
+  uint32_t* mk = marks_of(ctx, ctx->U);
+  if (ctx->es == 8)
+    launch_spoil_members(ctx->inst_d, ctx->ninst, ctx->dt_rec, ctx->cfg.max_steps, steps,
+                         (double*)ctx->U[0], (double*)ctx->U[1], (double*)ctx->U[2], mk,
+                         ctx->stream);
+  else
+    launch_spoil_members(ctx->inst_d, ctx->ninst, ctx->dt_rec, ctx->cfg.max_steps, steps,
+                         (float*)ctx->U[0], (float*)ctx->U[1], (float*)ctx->U[2], mk, ctx->stream);
+  (void)hipGetLastError();  // (rc is what the caller has to hear of)
+  return rc;
+}
+
 // The error check of what was enqueued, and the stats of the state after
 // `steps` recorded steps (st null: the check alone), with one wait.
 int finish_steps(tg_ctx* ctx, int steps, tg_stats* st, int nst) {
   HIPCHK(ctx, hipGetLastError());
-  if (!st) return check_err(ctx);
+  if (!st) return steps_failed(ctx, steps, check_err(ctx));
   if (ctx->leaves)
     launch_leaf_stats(ctx->leaf,
                       Fields{(double*)ctx->U[0], (double*)ctx->U[1], (double*)ctx->U[2]},
@@ -805,7 +822,7 @@ int finish_steps(tg_ctx* ctx, int steps, tg_stats* st, int nst) {
                        ctx->time_d, dt ? ctx->dt_rec : nullptr, ctx->cfg.max_steps, steps - 1,
                        ctx->err_d, ctx->red_host, ctx->stream);
   const int rc = wait_reduced(ctx);
-  if (rc) return rc;
+  if (rc) return steps_failed(ctx, steps, rc);
   const double* r = ctx->red_host;
   for (int b = 0; b < nst && b < nm; b++) {
     st[b].dt = dt ? r[3 * nm + b] : 0.;

@@ -541,6 +541,11 @@ void launch_member_reduce(const double* sum_part, const double* max_part, const 
                           long long stride, int col, const int* err, double* out, hipStream_t s);
 // time[b] = t of n members, and *err (given) cleared
 void launch_set_time(double* time, int n, double t, int* err, hipStream_t s);
+// NaN in every cell, and nothing known in the zero marks mk (or null), of the
+// members with a dt that is not finite among dt_rec[b * stride + 0..steps)
+template <class S>
+void launch_spoil_members(const InstDev* inst, int n, const double* dt_rec, long long stride,
+                          int steps, S* h, S* hu, S* hv, uint32_t* mk, hipStream_t s);
 // What one reverse step of its own starts from, in one launch: dt_rec[b *
 // stride] = dt of n members, n0 words at z0 and n1 at z1 cleared
 void launch_reverse_setup(double* dt_rec, long long stride, int n, double dt, uint32_t* z0,

@@ -725,7 +725,7 @@ __device__ __forceinline__ void update_dry_tile(const StepArgs& a, const TileRef
 // Second pass on large meshes: a fixed grid walks the full list, then the dry
 // one.  The first workgroups also keep the members' records (step_dt); a dt
 // that is not finite makes every cell so, the unlisted ones too, so it is
-// reported here as the state it would give is.
+// reported here as the state it would give is (see k_spoil_members).
 template <int TX>
 __global__ __launch_bounds__(record_threads<TX>(), 5) void k_update(StepArgs a) {
   __shared__ FaceLds<TX> L;
@@ -888,6 +888,27 @@ __global__ void k_set_time(double* time, int n, double t, int* err) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b < n) time[b] = t;
   if (b == 0 && err) *err = 0;
+}
+
+// After a step whose dt was not finite (one of `steps` recorded ones): every
+// cell of the member is NaN, as inf - inf makes it.  The passes that leave tiles
+// of +0.0 alone do so without a look at dt; looking there costs every step (2 %
+// of 64 members' steps by its registers alone), this only the failing call.
+constexpr int SPOIL_GRID = 64;  // workgroups a member
+template <class S>
+__global__ __launch_bounds__(BLOCK) void k_spoil_members(const InstDev* inst, const double* dt_rec,
+                                                         long long stride, int steps, S* h, S* hu,
+                                                         S* hv, uint32_t* mk) {
+  const int b = (int)blockIdx.x / SPOIL_GRID;
+  bool bad = false;
+  for (int s = (int)threadIdx.x; s < steps; s += BLOCK) bad = bad || !isfinite(dt_rec[b * stride + s]);
+  if (!__syncthreads_or(bad)) return;
+  const InstDev I = inst[b];
+  const long long n = (long long)I.nx * I.ny, m = (long long)I.nsx * I.nsy;
+  const long long first = (long long)(blockIdx.x % SPOIL_GRID) * BLOCK + threadIdx.x;
+  for (long long i = first; i < n; i += SPOIL_GRID * BLOCK)
+    h[I.off + i] = hu[I.off + i] = hv[I.off + i] = (S)NAN;
+  for (long long i = first; mk && i < m; i += SPOIL_GRID * BLOCK) mk[I.soff + i] = 0u;
 }
 
 // (one launch for a copy and two fills; with the three fields of lambda in one
@@ -1665,6 +1686,16 @@ void launch_member_reduce(const double* sum_part, const double* max_part, const 
 void launch_set_time(double* time, int n, double t, int* err, hipStream_t s) {
   hipLaunchKernelGGL(k_set_time, dim3((n + 63) / 64), dim3(64), 0, s, time, n, t, err);
 }
+template <class S>
+void launch_spoil_members(const InstDev* inst, int n, const double* dt_rec, long long stride,
+                          int steps, S* h, S* hu, S* hv, uint32_t* mk, hipStream_t s) {
+  hipLaunchKernelGGL(k_spoil_members<S>, dim3(n * SPOIL_GRID), dim3(BLOCK), 0, s, inst, dt_rec,
+                     stride, steps, h, hu, hv, mk);
+}
+template void launch_spoil_members<double>(const InstDev*, int, const double*, long long, int,
+                                           double*, double*, double*, uint32_t*, hipStream_t);
+template void launch_spoil_members<float>(const InstDev*, int, const double*, long long, int,
+                                          float*, float*, float*, uint32_t*, hipStream_t);
 void launch_reverse_setup(double* dt_rec, long long stride, int n, double dt, uint32_t* z0,
                           long long n0, uint32_t* z1, long long n1, hipStream_t s) {
   long long m = n0 > n1 ? n0 : n1;

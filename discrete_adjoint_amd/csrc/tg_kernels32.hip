@@ -217,7 +217,8 @@ __global__ __launch_bounds__(BLOCK) void k32_update(StepArgsM<S> a) {
   // a finite dt; nothing to do when the output tile is marked +0.0 already.
   // (Looked at before dt is made, which most workgroups of a large mesh then
   // never do; a dt that is not finite makes every cell so and is reported by
-  // the one that keeps the records, as the state it would give is.)
+  // the one that keeps the records, as the state it would give is: see
+  // k_spoil_members.)
   const bool skip =
       a.mk_in && a.mk_out && tile_marked_zero<TX>(a.mk_in, t, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 0, a.zbytes) &&

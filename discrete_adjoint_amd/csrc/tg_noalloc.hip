@@ -208,7 +208,13 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   Misc back{};
   NA_CHK(hipMemcpyAsync(&back, md, sizeof(Misc), hipMemcpyDeviceToHost, s));
   NA_CHK(hipStreamSynchronize(s));
-  if (back.err & 1) return TG_ERR_NONFINITE;
+  if (back.err & 1) {
+    if (!a.by_tile) {  // the dry tiles were written before dt was known
+      launch_spoil_members(a.inst, 1, a.dt_rec, 1, 1, d_h_out, d_hu_out, d_hv_out, nullptr, s);
+      NA_CHK(hipStreamSynchronize(s));
+    }
+    return TG_ERR_NONFINITE;
+  }
   if (back.err & 2) return TG_ERR_EIGEN;
   if (dt_out) *dt_out = back.dt_rec;
   return TG_OK;

@@ -27,7 +27,9 @@ typedef enum tg_status {
   TG_ERR_HIP = -2,          /* HIP runtime error                             */
   TG_ERR_STATE = -3,        /* call out of order (no mesh, no forward run)   */
   TG_ERR_NOMEM = -4,        /* device allocation failed                      */
-  TG_ERR_NONFINITE = -5,    /* NaN/Inf in the state (residual.C:137-147)     */
+  TG_ERR_NONFINITE = -5,    /* NaN/Inf in the state (residual.C:137-147); a
+                               dt that is not finite leaves no finite cell in
+                               its member                                    */
   TG_ERR_EIGEN = -6,        /* eigenvalue > 1e9 (get_coef_and_eigen.C:144)   */
   TG_ERR_UNSUPPORTED = -7,  /* mesh kind / mode not built                    */
   TG_ERR_NODEVICE = -8,     /* no HIP device                                 */

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from discrete_adjoint_amd import _lib
-from discrete_adjoint_amd.solver import Simulation, TgError
+from discrete_adjoint_amd.solver import Ensemble, Simulation, TgError
 from helpers import small_flow_problem
 
 pytestmark = pytest.mark.gpu
@@ -82,3 +82,52 @@ def test_replayed_negative_dt(oracle_lib):
     with Simulation(pb, max_steps=8, use_graph=0) as sim:
         sim.replay(np.array(dts))
         assert _same(sim.get_state(), U)
+
+
+@pytest.mark.parametrize("ny", [300, 1500])   # 225 tiles, 1125 tiles
+@pytest.mark.parametrize("precision", [_lib.TG_FP64, _lib.TG_FWD64_ADJ32, _lib.TG_MIXED,
+                                       _lib.TG_FP32])
+def test_dt_not_finite_leaves_no_finite_cell(precision, ny):
+    """A step whose dt is not finite makes every cell so, those of blocks that
+    the marks let the steps before leave alone too, on meshes of either launch:
+    replayed, and as a single step."""
+    nx = 192
+    _say(f"case dt edge: dt not finite {nx}x{ny} precision {precision}")
+    pb = small_flow_problem(nx, ny, 10)
+    with Simulation(pb, precision=precision, max_steps=8, use_graph=0) as sim:
+        for bad in (np.inf, np.nan):
+            sim.set_state(pb.h, pb.hu, pb.hv)
+            sim.replay(np.array([0.02, 0.03]))
+            assert np.isfinite(sim.get_state()).all()
+            sim.set_state(pb.h, pb.hu, pb.hv)
+            with pytest.raises(TgError) as e:
+                sim.replay(np.array([0.02, 0.03, bad]))
+            assert e.value.code == _lib.TG_ERR_NONFINITE
+            assert not np.isfinite(sim.get_state()).all(axis=0).any(), bad
+        sim.set_state(pb.h, pb.hu, pb.hv)
+        sim.run(2)
+        sim.params.maxtime = -np.inf      # the next dt: maxtime - time
+        with pytest.raises(TgError) as e:
+            sim.step()
+        assert e.value.code == _lib.TG_ERR_NONFINITE
+        assert not np.isfinite(sim.get_state()).all(axis=0).any()
+
+
+def test_members_beside_one_whose_dt_is_not_finite(oracle_lib):
+    """An ensemble of more than 1024 tiles with an all-dry member: its dt is
+    infinite and its cells become NaN; the others' states are their own."""
+    mem = [small_flow_problem(70, 45, 3), small_flow_problem(40, 30, 3),
+           small_flow_problem(192, 1500, 3)]
+    for f in (mem[1].h, mem[1].hu, mem[1].hv):
+        f[:] = 0.0
+    _say("case dt edge: all-dry member of an ensemble")
+    with Ensemble(mem, precision=_lib.TG_FP64, max_steps=4) as ens:
+        with pytest.raises(TgError) as e:
+            ens.run(3)
+        assert e.value.code == _lib.TG_ERR_NONFINITE
+        assert np.isnan(ens.member_state(1)).all()
+        for b in (0, 2):
+            orc = oracle_lib.Oracle.from_problem(mem[b])
+            U = [mem[b].h.copy(), mem[b].hu.copy(), mem[b].hv.copy()]
+            orc.run(U, 3)
+            assert _same(ens.member_state(b), U), b

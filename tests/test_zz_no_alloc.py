@@ -103,3 +103,26 @@ def test_noalloc_step_of_the_flattest_blocks(nx, ny):
         assert dt == dtr and 0 < dt < 1, s
         for a, b in zip(U, Ur):
             assert np.array_equal(a, b), s
+
+
+@pytest.mark.parametrize("nx,ny", [(70, 45), (515, 513)])   # 24 tiles, 1161
+def test_noalloc_step_of_a_dry_block_without_a_time_limit(nx, ny):
+    """Nothing wet and nothing to end the step: dt is infinite, which is
+    reported, and every output cell is NaN whichever launch the size takes."""
+    _say(f"case noalloc all dry {nx}x{ny}")
+    lib = _lib.load()
+    cfg, prm = _lib.tg_config(), _lib.tg_params()
+    lib.tg_config_default(C.byref(cfg))
+    assert lib.tg_params_from_angles(0.5, 0.3, 1.0, 1.0, C.byref(prm)) == _lib.TG_OK
+    n = nx * ny
+    arrays = [DeviceArray.of(np.ones(7 * n))] + [DeviceArray.of(np.zeros(n)) for _ in range(6)]
+    try:
+        blk = _lib.tg_noalloc_block(nx, ny, 1.0, 1.0, arrays[0].ptr)
+        dt = C.c_double()
+        rc = lib.tg_step_noalloc(C.byref(cfg), C.byref(blk), C.byref(prm), 0, 0.0,
+                                 *[b.ptr for b in arrays[1:]], None, C.byref(dt))
+        assert rc == _lib.TG_ERR_NONFINITE
+        assert all(np.isnan(b.numpy()).all() for b in arrays[4:])
+    finally:
+        for b in arrays:
+            b.free()
