@@ -472,13 +472,20 @@ int tg_tile_variant(int variant, int* tile_x, int* tile_y, int* xcd_banded);
 
 /* Times every variant for each kernel (coef, update, adjoint; `reps` launches
  * each on the current state, after a completed tg_forward_run) and selects
- * the fastest per kernel for the rest of the context's life.
+ * the fastest per kernel for the rest of the context's life.  On meshes of
+ * more than 1024 tiles (64x4) the FP64 coefficient pass also lists the
+ * update's tiles and runs in the update's variant: the two are chosen
+ * together, by the sum of their times.
  * variant_out [3] (may be NULL); ms_out [3 * TG_NUM_TILE_VARIANTS] average
  * launch times (may be NULL).  Overwrites the adjoint buffers. */
 int tg_autotune(tg_ctx* ctx, const tg_params* prm, int reps, int* variant_out, double* ms_out);
 
 /* Variants in use per kernel (coef, update, adjoint); set them explicitly
- * (e.g. to reproduce an earlier autotune). */
+ * (e.g. to reproduce an earlier autotune).  variant[0] has no effect where the
+ * coefficient pass runs in the update's variant (tg_autotune), which is then
+ * what tg_get_tile_selection gives for it.  Without a choice (by these calls or
+ * tg_config's tile_x, tile_y) every kernel runs variant 0, but both FP64
+ * forward passes on meshes of more than 1024 tiles, which run variant 3. */
 int tg_get_tile_selection(const tg_ctx* ctx, int* variant_out);
 int tg_set_tile_selection(tg_ctx* ctx, const int* variant);
 
