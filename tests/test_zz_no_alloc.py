@@ -126,3 +126,38 @@ def test_noalloc_step_of_a_dry_block_without_a_time_limit(nx, ny):
     finally:
         for b in arrays:
             b.free()
+
+
+def test_noalloc_step_with_dry_cells_by_the_list(oracle_lib):
+    """A ragged block of more than 1024 tiles, whose dry tiles the first pass
+    writes itself: negative depths, -0.0 and momenta below tiny among them.
+    Equal to tg_forward_step and to the oracle, signs included; then with the
+    clock at and past its end (dt = 0, dt < 0), where no dry tile may be copied
+    before dt is known."""
+    pb = small_flow_problem(515, 513, 4)
+    _say("case noalloc 515x513 dry cells")
+    rng = np.random.default_rng(8)
+    dry = np.flatnonzero(pb.h == 0)
+    for f in (pb.h, pb.hu, pb.hv):
+        f[rng.choice(dry, 4000, replace=False)] = -0.0
+    pb.h[rng.choice(dry, 50, replace=False)] = -1e-3
+    some = rng.choice(dry, 300, replace=False)
+    pb.h[some], pb.hu[some], pb.hv[some] = 6e-5, -2e-6, 3e-7
+    cfg, prm, ref = _reference(pb, 4)
+    got = _noalloc_chain(pb, cfg, prm, 4)
+    orc = oracle_lib.Oracle.from_problem(pb)
+    U = [pb.h.copy(), pb.hu.copy(), pb.hv.copy()]
+    for s, ((V, dt), (Vr, dtr, _)) in enumerate(zip(got, ref)):
+        assert dt == dtr == orc.step(U, s)[0], s
+        for a, b, c in zip(V, Vr, U):
+            assert np.array_equal(a, b) and np.array_equal(a, c), s
+            assert np.array_equal(np.signbit(a), np.signbit(c)), s
+    for end in (0.0, -0.25):   # the first step starts at time 0
+        prm.maxtime = end
+        orc = oracle_lib.Oracle.from_problem(pb)
+        orc.params.maxtime = end
+        U = [pb.h.copy(), pb.hu.copy(), pb.hv.copy()]
+        (V, dt), = _noalloc_chain(pb, cfg, prm, 1)
+        assert dt == orc.step(U, 0)[0] == end
+        for a, c in zip(V, U):
+            assert np.array_equal(a, c) and np.array_equal(np.signbit(a), np.signbit(c)), end
