@@ -2,9 +2,10 @@
 tile less, equal and more than each tile shape, the thinnest ones, whole rows
 of boundary cells -- and on both sides of the line between a workgroup per
 tile (1024 tiles) and the tile list, against the oracle.  Bar: states, dt and
-lambda bit-identical (every product and sum in the reference's order), the
-bed-friction gradient's contribution to rtol 1e-12 (a sum over cells in
-another order)."""
+lambda bit-identical (every product and sum in the reference's order), a step's
+bed-friction gradient to 1e-12 of the absolute sum of its terms lambda .
+dU/dphi (each is rounded some 30 times and they are added in another order); the
+FP32 modes' bars stand at their tests."""
 import sys
 
 import numpy as np
@@ -43,8 +44,13 @@ def _problem(nx, ny, seed):
     return pb
 
 
+def _terms(orc, pb, s, dt, lam):
+    """The absolute sum of a reverse step's gradient terms."""
+    return np.abs(lam * orc.dstep_dphi([pb.h, pb.hu, pb.hv], s, dt)).sum()
+
+
 @pytest.mark.parametrize("tile", [(64, 4), (32, 8), (16, 16)])
-@pytest.mark.parametrize("nx,ny", SIZES)
+@pytest.mark.parametrize("nx,ny", SIZES + [(513, 512)])
 def test_reverse_step_at_tile_edges(oracle_lib, nx, ny, tile):
     _say(f"case reverse step {nx}x{ny} tile {tile}")
     pb = _problem(nx, ny, 100 * nx + ny)
@@ -57,10 +63,7 @@ def test_reverse_step_at_tile_edges(oracle_lib, nx, ny, tile):
             got, g = sim.adjoint_step_grad(s, dt, lam)
             assert np.array_equal(got, np.asarray(ref).reshape(3, -1)), s
             assert np.array_equal(sim.adjoint_step(s, dt, lam), got), s
-            # the sum's own cancellation: its terms are at most their count
-            # times the largest, rounded once each
-            scale = np.abs(lam).sum() * max(np.abs(pb.hu).max(), np.abs(pb.hv).max(), 1.0) * dt
-            assert abs(g - dphi) <= 1e-12 * max(abs(dphi), scale), s
+            assert abs(g - dphi) <= 1e-12 * _terms(orc, pb, s, dt, lam), s
 
 
 @pytest.mark.parametrize("tile", [(0, 0), (64, 4), (32, 8), (16, 16)])
@@ -91,7 +94,7 @@ def test_forward_steps_at_tile_edges(oracle_lib, nx, ny, tile):
 
 def test_reverse_sweep_on_both_launches(oracle_lib):
     """A sweep over 1024 tiles and one over more, checkpoints and recompute:
-    lambda bit-identical to the oracle's."""
+    lambda bit-identical to the oracle's, the gradient to rtol 1e-12."""
     for nx in (512, 513):
         _say(f"case reverse sweep {nx}x512")
         pb = _problem(nx, 512, nx)
@@ -100,13 +103,15 @@ def test_reverse_sweep_on_both_launches(oracle_lib):
         pb.h[away] = pb.hu[away] = pb.hv[away] = 0.0
         w = pb.box_weights((nx * 2.0, nx * 6.0, 1500.0, 3500.0))
         orc = oracle_lib.Oracle.from_problem(pb)
-        _, dts, lam_ref, _ = orc.forward_adjoint([pb.h.copy(), pb.hu.copy(), pb.hv.copy()], 5, w)
+        _, dts, lam_ref, dphi_ref = orc.forward_adjoint([pb.h.copy(), pb.hu.copy(), pb.hv.copy()],
+                                                        5, w, want_dphi=True)
         for graph in (0, 1):
             with Simulation(pb, max_steps=5, checkpoint_every=2, use_graph=graph) as sim:
                 sim.run(5)
                 assert np.array_equal(sim.dt_record(), dts)
-                lam, _ = sim.dual_solver(w, want_dphi=True)
+                lam, dphi = sim.dual_solver(w, want_dphi=True)
                 assert np.array_equal(lam, lam_ref), (nx, graph)
+                assert dphi == pytest.approx(dphi_ref, rel=1e-12), (nx, graph)
 
 
 @pytest.mark.parametrize("thin", [0.1, 0.5])
@@ -140,8 +145,7 @@ def test_fp32_reverse_step_at_tile_edges(oracle_lib, nx, ny, tile, thin):
             got, g = sim.adjoint_step_grad(s, dt, lam)
             assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref), s
             assert np.array_equal(sim.adjoint_step(s, dt, lam), got), s
-            scale = np.abs(lam).sum() * max(np.abs(pb.hu).max(), np.abs(pb.hv).max(), 1.0) * dt
-            assert abs(g - dphi) <= 1e-4 * max(abs(dphi), scale), s
+            assert abs(g - dphi) <= 1e-4 * _terms(orc, pb, s, dt, lam), s
 
 
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
@@ -172,3 +176,40 @@ def test_reverse_step_of_a_lambda_that_is_not_finite(oracle_lib, nx, ny, value):
             for got in (sim.adjoint_step(60, 0.05, lam), sim.adjoint_step_grad(60, 0.05, lam)[0]):
                 bad = np.argwhere((got != ref) & ~(np.isnan(got) & np.isnan(ref)))
                 assert len(bad) == 0, (k, len(bad), bad[:3], got[tuple(bad[0])], ref[tuple(bad[0])])
+
+
+@pytest.mark.parametrize("tile", [(64, 4), (32, 8), (16, 16)])
+@pytest.mark.parametrize("nx,ny", [(66, 33), (513, 512)])
+def test_fp32_gradient_term_of_one_cell(oracle_lib, nx, ny, tile):
+    """lambda^{s+1} in one cell only: its gradient term alone, at the corners and
+    edges of the tiles and of the member and next to thin cells, so that no term
+    of a cell or of a face beyond the tile can be lost in a sum over all.
+    Bar: 1e-4 of the term's three products, some hundred FP32 roundings each with
+    up to ten times their size cancelling between the faces; every one of them
+    far above it."""
+    _say(f"case fp32 gradient of one cell {nx}x{ny} tile {tile}")
+    pb = _problem(nx, ny, 3 * nx + ny)
+    i0, j0 = (0, 0) if nx < 100 else (tile[0] * (256 // tile[0]), 256)
+    if nx > 100:
+        j, i = np.divmod(np.arange(pb.n), nx)
+        away = np.hypot(i - i0, j - j0) > 80
+        pb.h[away] = pb.hu[away] = pb.hv[away] = 0.0
+    orc = oracle_lib.Oracle.from_problem(pb)
+    at = [(i0 + a * tile[0] + di, j0 + b * tile[1] + dj)
+          for a, b in ((0, 0), (1, 1)) for di in (0, tile[0] - 1) for dj in (0, tile[1] - 1)]
+    at += [(0, 0), (nx - 1, 0), (0, ny - 1), (nx - 1, ny - 1)] if nx < 100 else []
+    cells = [j * nx + i for i, j in at if i < nx and j < ny]
+    thin = np.flatnonzero((pb.h > 0) & (pb.h < 1e-3))
+    cells += [c + 1 for c in thin[::max(1, len(thin) // 6)] if c + 1 < pb.n]
+    checked = 0
+    with Simulation(pb, max_steps=64, tile_x=tile[0], tile_y=tile[1],
+                    precision=_lib.TG_FWD64_ADJ32) as sim:
+        for c in cells:
+            lam = np.zeros((3, pb.n))
+            lam[:, c] = 1.0, -0.7, 0.4
+            _, dphi = orc.adjoint_step([pb.h, pb.hu, pb.hv], 60, 0.05, lam, want_dphi=True)
+            _, g = sim.adjoint_step_grad(60, 0.05, lam)
+            terms = _terms(orc, pb, 60, 0.05, lam)
+            assert abs(g - dphi) <= 1e-4 * terms, (c % nx, c // nx, g, dphi)
+            checked += abs(dphi) > 1e-2 * terms > 0
+    assert checked >= 6
