@@ -90,7 +90,7 @@ struct tg_ctx {
   bool box_on = false;  // a region is set (it may hold no cell)
   long long box_version = 0;  // changes with every tg_set_maxh_region
   double* box_rec = nullptr;
-  RedDev* red = nullptr;     // 2 * ninst: steps alternate
+  RedDev* red = nullptr;     // 2 * ninst * NRED: steps alternate
   double* dt_rec = nullptr;  // ninst * max_steps
   double* time_d = nullptr;  // ninst
   // ninst * (max_steps + 1): each member's time before each recorded step of
@@ -526,8 +526,8 @@ StepArgsM<S> step_args_m(tg_ctx* ctx, void* const in[3], void* const out[3], int
   a.U = FieldsT<S>{(S*)in[0], (S*)in[1], (S*)in[2]};
   a.S32 = statics32(ctx);
   a.kact = (float*)ctx->kact; a.dt_rec = ctx->dt_rec; a.time = ctx->time_d;
-  a.red = ctx->red + (s & 1) * ctx->ninst;
-  a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst;
+  a.red = ctx->red + (s & 1) * ctx->ninst * NRED;
+  a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst * NRED;
   a.clock = ctx->clock_d;
   a.cfl_inner = ctx->cfg.cfl_inner; a.cfl_outer = ctx->cfg.cfl_outer;
   a.max_steps = ctx->cfg.max_steps; a.step = s; a.ft = frict_tiny(ctx, s);
@@ -602,7 +602,7 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
                   at<double>(ctx->statics, 2, n), at<double>(ctx->statics, 3, n),
                   at<double>(ctx->statics, 4, n), at<double>(ctx->statics, 5, n),
                   at<double>(ctx->statics, 6, n)};
-    a.kact = (double*)ctx->kact; a.red = ctx->red; a.dt_rec = ctx->dt_rec; a.time = ctx->time_d;
+    a.kact = (double*)ctx->kact; a.dt_rec = ctx->dt_rec; a.time = ctx->time_d;
     a.clock = ctx->clock_d;
     a.max_steps = ctx->cfg.max_steps; a.step = s; a.ft = frict_tiny(ctx, s);
     a.tiny = ctx->cfg.tiny; a.gamma = ctx->cfg.gamma;
@@ -617,8 +617,8 @@ void enqueue_step(tg_ctx* ctx, void* const in[3], void* const out[3], int s, boo
     a.mk_out = marks_of(ctx, out);
     a.zbytes = !ctx->bytes_off && SHAPE_TX[ctx->sel[1]] == ctx->mk_tx[0];
     a.fold = compute_dt;
-    a.red = ctx->red + (s & 1) * ctx->ninst;
-    a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst;
+    a.red = ctx->red + (s & 1) * ctx->ninst * NRED;
+    a.red_next = ctx->red + ((s + 1) & 1) * ctx->ninst * NRED;
     if (ctx->leaves) {
       a.mat = ctx->mat_d;
       a.mtab = ctx->mtab_d;
@@ -782,11 +782,11 @@ int d2h_fields(tg_ctx* ctx, void* const f[3], long long off, long long count,
   return TG_OK;
 }
 
-// What the steps' error check said of `steps` recorded steps.  Where their
-// passes leave tiles alone without a look at dt, a dt that was not finite still
-// has to reach those.
+// What the steps' error check said of `steps` recorded steps.  Their passes
+// leave tiles alone without a look at dt (uniform meshes): a dt that was not
+// finite still has to reach those.
 int steps_failed(tg_ctx* ctx, int steps, int rc) {
-  if (rc != TG_ERR_NONFINITE || ctx->leaves || (fwd64(ctx) && tile_launch(ctx, 0) != 0)) return rc;
+  if (rc != TG_ERR_NONFINITE || ctx->leaves) return rc;
   uint32_t* mk = marks_of(ctx, ctx->U);
   if (ctx->es == 8)
     launch_spoil_members(ctx->inst_d, ctx->ninst, ctx->dt_rec, ctx->cfg.max_steps, steps,
@@ -1612,7 +1612,7 @@ int set_members(tg_ctx* ctx, int nm, const tg_mesh* meshes, const tg_params* par
   for (int b = 0; b < nm; b++) any_mat |= meshes[b].mat != nullptr;
   if (!rc && any_mat) rc = dalloc(ctx, (void**)&ctx->mat_d, (size_t)n);
   if (!rc && any_mat) rc = dalloc(ctx, (void**)&ctx->mtab_d, sizeof(MatDev) * MAX_MAT * nm);
-  if (!rc) rc = dalloc(ctx, (void**)&ctx->red, sizeof(RedDev) * 2 * nm);
+  if (!rc) rc = dalloc(ctx, (void**)&ctx->red, sizeof(RedDev) * 2 * nm * NRED);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->time_d, sizeof(double) * nm);
   if (!rc) rc = dalloc(ctx, (void**)&ctx->dt_rec, sizeof(double) * nm * ctx->cfg.max_steps);
   if (!rc)

@@ -83,10 +83,17 @@ struct BlockDev {
 // Per-instance CFL reduction cells: bit patterns of non-negative doubles
 // (IEEE order of non-negative doubles equals unsigned-integer order, so
 // integer atomic min/max is an exact FP64 min/max).
-struct alignas(128) RedDev {  // a cache line each: members' atomics do not share one
+struct alignas(128) RedDev {  // a cache line each: atomics on two do not wait for each other
   unsigned long long min_ev;  // min over wet cells of min(dx,dy)/evalue
   unsigned long long hmax;    // max over wet cells of h
 };
+// Cells of one member, which its workgroups take in turn.  Atomics on one line
+// take 12 ns each, one after another, and a workgroup per tile adds two: with
+// one cell a forward step of 448 x 400 (512 x 512) wet cells took 39.8 (52.5) us,
+// with two 32.8 (42.1), with four 29.1 (36.4).  But every tile of a step reads
+// them all: four cost 64 members and 1531 x 1207 cells 1 to 2 % where two cost
+// nothing.
+constexpr int NRED = 2;
 
 constexpr int BLOCK = 256;
 // Tile variants (one tile table each): tile width TX (height BLOCK / TX)
@@ -177,8 +184,8 @@ struct StepArgs {
   Fields U;
   Statics S;
   double* kact;          // [n] forward kact of U
-  RedDev* red;           // [ninst] of this step
-  RedDev* red_next;      // [ninst] of the next step (fold)
+  RedDev* red;           // [ninst * NRED] of this step
+  RedDev* red_next;      // [ninst * NRED] of the next step (fold)
   double* dt_rec;        // [ninst * max_steps]
   double* time;          // [ninst] after the last step taken
   double* clock;         // [ninst * (max_steps + 1)]: before each step (fold)
@@ -244,6 +251,18 @@ __device__ __forceinline__ double cfl_dt(const A& a, const InstDev& I, const Red
   return dt;
 }
 
+// A workgroup's terms into one of the member's cells, workgroups in turn.
+__device__ __forceinline__ void red_add(RedDev* red, int b, double minev, double hmax) {
+  RedDev* r = red + (long long)b * NRED + blockIdx.x % NRED;
+  if (minev < HUGE_VAL) atomicMin(&r->min_ev, (unsigned long long)__double_as_longlong(minev));
+  if (hmax > 0.) atomicMax(&r->hmax, (unsigned long long)__double_as_longlong(hmax));
+}
+// cell k of member b, empty (get_coef_and_eigen.C:35)
+__device__ __forceinline__ void red_clear(RedDev* red, int b, int k) {
+  red[(long long)b * NRED + k] =
+      RedDev{(unsigned long long)__double_as_longlong(10000000.), 0ull};
+}
+
 // The dt of member b at this step.  a.fold: it is made here, by every workgroup
 // alike, from the reduction cells the coefficient pass filled, instead of in a
 // launch of its own (4.4 us of every step); one workgroup of the member
@@ -256,14 +275,19 @@ __device__ __forceinline__ double step_dt(const A& a, int b, bool own) {
   double* rec = a.dt_rec + (long long)b * a.max_steps + a.step;
   if (!a.fold) return *rec;
   const InstDev& I = a.inst[b];
-  const RedDev R = a.red[b];
+  RedDev R = a.red[(long long)b * NRED];
+#pragma unroll
+  for (int k = 1; k < NRED; k++) {
+    const RedDev q = a.red[(long long)b * NRED + k];
+    R.min_ev = q.min_ev < R.min_ev ? q.min_ev : R.min_ev;
+    R.hmax = q.hmax > R.hmax ? q.hmax : R.hmax;
+  }
   double* clock = a.clock + (long long)b * (a.max_steps + 1) + a.step;
   const double dt = cfl_dt(a, I, R, *clock);
+  if (own && threadIdx.x < NRED) red_clear(a.red_next, b, (int)threadIdx.x);
   if (own && threadIdx.x == 0) {
     *rec = dt;
     clock[1] = a.time[b] = *clock + dt;
-    a.red_next[b].min_ev = (unsigned long long)__double_as_longlong(10000000.);
-    a.red_next[b].hmax = 0ull;
   }
   return dt;
 }
@@ -407,12 +431,22 @@ constexpr int THIN_GRID = 512;
 // the listed tiles spread over every CU (1024, 2048, 4096 and 8192 measured
 // on the 256-member ensemble: 4096 about 1 % ahead)
 constexpr int LIST_GRID = 4096;
-// Up to this many tiles each FP64 pass launches a workgroup per tile: two
-// launches per forward and one per reverse step instead of four and three
-// (512 x 512 cells, 1024 tiles: 14.4 us of kernels per forward step against
-// 34, 13 against 40 per reverse step).  Beyond it the workgroups of empty
-// tiles, held to three a CU by their LDS, queue: the block passes leave a
-// block after a few words and only listed tiles take that LDS.
+// Up to this many tiles each FP64 pass, and the FP32 reverse step, launches a
+// workgroup per tile: two launches per forward and one per reverse step, where
+// the block passes and the list take two and two.  us per step by tile / by list,
+// forward and reverse, of a mesh with a small pile and of one all wet:
+//   tiles   pile fwd     rev          wet fwd       rev
+//    700    13.9 / 21.7  11.8 / 19.5  32.3 / 28.5   22.8 /  33.5
+//   1024    18.4 / 22.2  17.1 / 19.7  42.3 / 35.2   28.8 /  42.2
+//   1500    19.0 / 22.5  17.3 / 19.7  62.6 / 44.7   40.7 /  56.7
+//   2496    22.1 / 23.3  21.1 / 20.6  97.8 / 60.9   63.6 /  87.0
+//   4096    42.7 / 23.1  32.7 / 22.0   159 / 91.5   98.5 / 140.6
+// Beyond it the workgroups of empty tiles, held to three a CU by their LDS,
+// queue, and a wet forward step loses to the list what a pile's gains.  (The
+// reverse step alone would gain up to 2496 tiles; all passes of a mesh share one
+// line.  The FP32 reverse step goes the same way: 1024 tiles 38.4 / 48.2 with a
+// pile, 35.0 / 58.2 wet; 2496 40.9 / 51.1 and 87.5 / 121; 4096 63.5 / 53.4 and
+// 132 / 201.)
 constexpr int TILE_LAUNCH_MAX = 1024;
 // workgroups of the FP64 adjoint's list walk
 constexpr int ADJ_GRID = 2048;
@@ -502,7 +536,7 @@ void launch_leaf_stats(const LeafDev& L, Fields U, double* part_mass, double* pa
 void launch_coef(const StepArgs& a, bool reduce, hipStream_t s);
 void launch_update(const StepArgs& a, hipStream_t s);
 void launch_adjoint(const AdjArgs& a, hipStream_t s);
-// clears both sets of reduction cells (red [2 * ninst]); clock (or null):
+// clears both sets of reduction cells (red [2 * ninst * NRED]); clock (or null):
 // clock[b * stride] = time[b]
 void launch_reset_red(RedDev* red, int ninst, const double* time, double* clock, long long stride,
                       hipStream_t s);

@@ -200,7 +200,8 @@ __device__ __forceinline__ void coef_cell(const StepArgs& a, const InstDev& I, i
 
 // The workgroup's CFL terms into the member's reduction cells (every thread
 // calls it; any: some thread has one).
-__device__ __forceinline__ void coef_reduce(RedDev* red, double minev, double hmax, bool any) {
+__device__ __forceinline__ void coef_reduce(RedDev* red, int b, double minev, double hmax,
+                                            bool any) {
   if (!__syncthreads_or(any)) return;
   __shared__ double smin[BLOCK / 64], smax[BLOCK / 64];
   minev = wave_min(minev);
@@ -213,8 +214,7 @@ __device__ __forceinline__ void coef_reduce(RedDev* red, double minev, double hm
       minev = (smin[k] < minev) ? smin[k] : minev;
       hmax = (smax[k] > hmax) ? smax[k] : hmax;
     }
-    if (minev < HUGE_VAL) atomicMin(&red->min_ev, dbits(minev));
-    if (hmax > 0.) atomicMax(&red->hmax, dbits(hmax));
+    red_add(red, b, minev, hmax);
   }
 }
 
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
   for (int k = (int)threadIdx.x; k < n; k += BLOCK)
     coef_cell(a, I, B.x0 + s_cell[k] % MARK_W, B.y0 + s_cell[k] / MARK_W, s_h[k], reduce, minev,
               hmax);
-  if (reduce) coef_reduce(&a.red[B.inst], minev, hmax, (int)threadIdx.x < n);
+  if (reduce) coef_reduce(a.red, B.inst, minev, hmax, (int)threadIdx.x < n);
 }
 
 // the tile of a workgroup of the passes over every tile
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(BLOCK) void k_coef_tile(StepArgs a, int reduce) {
     const int cnt = __syncthreads_count(act && !wet);
     if (threadIdx.x == 0 && cnt) atomicAdd(a.short_cells, (unsigned long long)cnt);
   }
-  if (reduce) coef_reduce(&a.red[t.inst], minev, hmax, wet);
+  if (reduce) coef_reduce(a.red, t.inst, minev, hmax, wet);
 }
 
 // Both sets of reduction cells, and each member's clock slot of the step about
@@ -385,8 +385,10 @@ __global__ void k_reset_red(RedDev* red, int ninst, const double* time, double* 
                             long long stride) {
   int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b < ninst) {
-    red[b].min_ev = red[ninst + b].min_ev = dbits(10000000.);  // get_coef_and_eigen.C:35
-    red[b].hmax = red[ninst + b].hmax = dbits(0.);
+    for (int k = 0; k < NRED; k++) {
+      red_clear(red, b, k);
+      red_clear(red, ninst + b, k);
+    }
     if (clock) clock[b * stride] = time[b];
   }
 }
@@ -755,10 +757,14 @@ __global__ __launch_bounds__(face_threads<TX>()) void k_update_tile(StepArgs a) 
   __shared__ FaceLds<TX> L;
   const int tile = tile_of(a);
   const TileDev t = a.tiles[tile];
-  const double dt = step_dt(a, t.inst, t.x0 == 0 && t.y0 == 0);
-  if (a.mk_in && isfinite(dt) && update_skip(a.mk_in, t) &&
-      out_marked_zero<TX>(a.mk_out, t, a.zbytes))
-    return;
+  const bool own = t.x0 == 0 && t.y0 == 0;  // keeps the member's records
+  // (looked at before dt is made, which the workgroups of empty tiles then never
+  // do; a dt that is not finite: see k_spoil_members)
+  const bool skip = a.mk_in && update_skip(a.mk_in, t) && out_marked_zero<TX>(a.mk_out, t, a.zbytes);
+  if (skip && !own) return;
+  const double dt = step_dt(a, t.inst, own);
+  if (own && threadIdx.x == 0 && !isfinite(dt)) atomicOr(a.err, 1);
+  if (skip && isfinite(dt)) return;
   update_tile<TX, face_threads<TX>(), true>(a, ref_of(t, tile), dt, L);
 }
 

@@ -25,9 +25,6 @@ namespace {
 template <class S>
 using Wt = typename std::conditional<std::is_same<S, double>::value, double, float>::type;
 
-__device__ __forceinline__ unsigned long long dbits(double v) {
-  return (unsigned long long)__double_as_longlong(v);
-}
 __device__ __forceinline__ double wave_min(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -174,8 +171,7 @@ __global__ __launch_bounds__(BLOCK) void k32_coef(StepArgsM<S> a, int reduce) {
         minev = (smin[k] < minev) ? smin[k] : minev;
         hmax = (smax[k] > hmax) ? smax[k] : hmax;
       }
-      if (minev < HUGE_VAL) atomicMin(&a.red[t.inst].min_ev, dbits(minev));
-      if (hmax > 0.) atomicMax(&a.red[t.inst].hmax, dbits(hmax));
+      red_add(a.red, t.inst, minev, hmax);
     }
   }
 }
@@ -981,7 +977,7 @@ void k32_adjoint(AdjArgsM<S> a) {
 // record has a thread of its own and nothing is spilled (389 x 301 cells, 457
 // tiles, mixed: 16 us against 5.3 for the classifying pass, 22 for the gather
 // and 4.4 for emptying the list).  The line to the two passes is the FP64
-// kernels' (TILE_LAUNCH_MAX): past it the LDS of empty tiles queues.
+// kernels', measured with theirs (TILE_LAUNCH_MAX).
 template <int TX>
 constexpr int adj32_threads() {
   return BLOCK + (2 * TX + 2 * (BLOCK / TX) + 63) / 64 * 64;

@@ -127,8 +127,7 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_coef(StepArgs a, LeafDev L, int 
         minev = (smin[k] < minev) ? smin[k] : minev;
         hmax = (smax[k] > hmax) ? smax[k] : hmax;
       }
-      if (minev < HUGE_VAL) atomicMin(&a.red[0].min_ev, lbits(minev));
-      if (hmax > 0.) atomicMax(&a.red[0].hmax, lbits(hmax));
+      red_add(a.red, 0, minev, hmax);
     }
   }
 }

@@ -1,8 +1,9 @@
 // tg_step_noalloc: one order-1 forward step of a uniform block with every
 // intermediate kept in a fixed device array of this file (no device memory
 // is allocated or freed by the call).  It runs the kernels of
-// tg_forward_step -- coefficient / CFL pass and update -- on caller-owned device arrays, so its results are those of
-// tg_forward_step on the same state, bit for bit.
+// tg_forward_step -- coefficient / CFL pass and update -- on caller-owned
+// device arrays, so its results are those of tg_forward_step on the same
+// state, bit for bit.
 //
 // Scratch: the member record, the tile and mark-block tables of the 64x4
 // row-major tile variant, the CFL reduction cells, the dt / time / error
@@ -32,7 +33,7 @@ constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 // byte offsets into the scratch array
 constexpr size_t OFF_INST = 0;
 constexpr size_t OFF_RED = OFF_INST + align256(sizeof(InstDev));
-constexpr size_t OFF_MISC = OFF_RED + align256(2 * sizeof(RedDev));  // dt, time, err, count
+constexpr size_t OFF_MISC = OFF_RED + align256(2 * NRED * sizeof(RedDev));  // dt, time, err, count
 constexpr size_t OFF_TILES = OFF_MISC + 256;
 constexpr size_t OFF_BLOCKS = OFF_TILES + align256(sizeof(TileDev) * NA_MAX_TILES);
 constexpr size_t OFF_LIST = OFF_BLOCKS + align256(sizeof(BlockDev) * NA_MAX_BLOCKS);
@@ -75,11 +76,8 @@ __global__ __launch_bounds__(256) void k_noalloc_setup(InstDev I, Misc m, InstDe
   if (i == 0) {
     *inst = I;
     *misc = m;
-    for (int k = 0; k < 2; k++) {
-      red[k].min_ev = (unsigned long long)__double_as_longlong(10000000.);  // get_coef_and_eigen.C:35
-      red[k].hmax = 0ull;
-    }
   }
+  if (i < NRED) red_clear(red, 0, i);
   const int nsx = I.nsx;
   if (i < ntiles) {
     const int bx = i % ntx, ty = i / ntx, by = ty / ROWS, mw = by * nsx + bx;
@@ -180,7 +178,7 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.kact = (double*)(base + OFF_KACT);
   a.red = (RedDev*)(base + OFF_RED);
   a.dt_rec = &md->dt_rec;
-  a.red_next = a.red + 1;
+  a.red_next = a.red + NRED;
   a.time = &md->time;
   a.clock = md->clock;
   a.fold = 1;
