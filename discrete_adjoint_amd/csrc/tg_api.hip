@@ -2479,6 +2479,14 @@ int time_kernel_variant(tg_ctx* ctx, int which, int v, int reps, double* avg_ms)
       else launch_update_m<float>(a, ctx->stream);
     }
   };
+  // the scratch buffers carry marks in the timed variant's shape: none before
+  // and none after
+  auto forget = [&] {
+    if (!ctx->marks) return;
+    clear_marks(ctx, ctx->Ut[0]);
+    clear_marks(ctx, ctx->lam[1][0]);
+  };
+  forget();
   one(0);  // kact of the current state
   one(which);  // untimed first launch of this variant
   int rc = TG_OK;
@@ -2501,11 +2509,7 @@ int time_kernel_variant(tg_ctx* ctx, int which, int v, int reps, double* avg_ms)
   }
   for (int k = 0; k < 3; k++) ctx->sel[k] = keep[k];
   ctx->bytes_off = false;
-  // the scratch buffers carry marks in the timed variant's shape
-  if (ctx->marks) {
-    clear_marks(ctx, ctx->Ut[0]);
-    clear_marks(ctx, ctx->lam[1][0]);
-  }
+  forget();
   if (rc) return rc;
   *avg_ms = ms / reps;
   return check_err(ctx);

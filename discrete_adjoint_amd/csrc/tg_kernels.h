@@ -148,15 +148,15 @@ __device__ __forceinline__ int mark_byte(const T& t) {
 }
 
 // Whether the tile of this workgroup holds +0.0 in a buffer that the launch
-// writes, per its marks (every thread calls it and all get the same answer).
-// The word's other bytes are stored by other workgroups of the same launch, so
-// only the tile's own byte is looked at, which this workgroup alone stores, and
-// not before a barrier.  bytes 0 (timing: the bytes follow another shape): the
-// whole word, read once for all waves.
+// writes, per its marks, whose bytes follow the launch's own shape.  The word's
+// other bytes are stored by other workgroups of the same launch, so only the
+// tile's own byte counts, which this workgroup alone stores, and not before a
+// barrier that every wave passes after it has read it.  (No barrier here: past
+// one, the compiler reads the tile's and the member's records by vector loads,
+// which cost the FP32 update of 256 members 2 % and more.)
 template <int TX, class T>
-__device__ __forceinline__ bool out_marked_zero(const uint32_t* mk, const T& t, int bytes) {
-  if (bytes) return ((const unsigned char*)(mk + t.mw))[mark_byte<TX>(t)] == 1;
-  return __syncthreads_or(threadIdx.x == 0 && mk[t.mw] == MARK_FULL);
+__device__ __forceinline__ bool out_marked_zero(const uint32_t* mk, const T& t) {
+  return ((mk[t.mw] >> (8 * mark_byte<TX>(t))) & 0xffu) == 1u;
 }
 
 struct Fields {

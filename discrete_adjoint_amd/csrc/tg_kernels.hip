@@ -760,7 +760,7 @@ __global__ __launch_bounds__(face_threads<TX>()) void k_update_tile(StepArgs a) 
   const bool own = t.x0 == 0 && t.y0 == 0;  // keeps the member's records
   // (looked at before dt is made, which the workgroups of empty tiles then never
   // do; a dt that is not finite: see k_spoil_members)
-  const bool skip = a.mk_in && update_skip(a.mk_in, t) && out_marked_zero<TX>(a.mk_out, t, a.zbytes);
+  const bool skip = a.mk_in && update_skip(a.mk_in, t) && out_marked_zero<TX>(a.mk_out, t);
   if (skip && !own) return;
   const double dt = step_dt(a, t.inst, own);
   if (own && threadIdx.x == 0 && !isfinite(dt)) atomicOr(a.err, 1);
@@ -1549,7 +1549,7 @@ __global__ __launch_bounds__(ADJ_THREADS, 4) void k_adjoint_tile(AdjArgs a) {
   const int tile = tile_of(a);
   const TileDev t = a.tiles[tile];
   if (a.mk_out && adjoint_skip(a.mk_U, DPHI ? a.mk_lnext : nullptr, t.mw) &&
-      out_marked_zero<TX>(a.mk_out, t, a.l_bytes))
+      out_marked_zero<TX>(a.mk_out, t))
     return;
   adjoint_tile<TX, DPHI, true>(a, ref_of(t, tile), L);
 }

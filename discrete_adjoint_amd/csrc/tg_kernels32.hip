@@ -216,12 +216,12 @@ __global__ __launch_bounds__(BLOCK) void k32_update(StepArgsM<S> a) {
   // the one that keeps the records, as the state it would give is: see
   // k_spoil_members.)
   const bool skip =
-      a.mk_in && a.mk_out && tile_marked_zero<TX>(a.mk_in, t, a.zbytes) &&
+      a.mk_in && a.mk_out && out_marked_zero<TX>(a.mk_out, t) &&
+      tile_marked_zero<TX>(a.mk_in, t, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 0, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 1, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 2, a.zbytes) &&
-      side_tile_zero<TX>(a.mk_in, t, I, 3, a.zbytes) &&
-      out_marked_zero<TX>(a.mk_out, t, a.zbytes);
+      side_tile_zero<TX>(a.mk_in, t, I, 3, a.zbytes);
   if (skip && !own) return;
   const double dt = step_dt(a, t.inst, own);
   if (own && threadIdx.x == 0 && !isfinite(dt)) atomicOr(a.err, 1);
@@ -839,7 +839,7 @@ __device__ __forceinline__ bool adjoint32_void(const AdjArgsM<S>& a, const TileD
                                                const Cell& q) {
   if (a.mk_out && tile_marked_zero<TX>(a.mk_U, t, a.u_bytes) &&
       (!a.dphi_part || tile_marked_zero<TX>(a.mk_lnext, t, a.l_bytes))) {
-    if (out_marked_zero<TX>(a.mk_out, t, a.l_bytes)) return true;
+    if (out_marked_zero<TX>(a.mk_out, t)) return true;
     __syncthreads();  // every wave has read the byte that thread 0 stores below
   } else {
     bool busy = false;
