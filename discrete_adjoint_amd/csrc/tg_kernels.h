@@ -91,8 +91,9 @@ struct alignas(128) RedDev {  // a cache line each: atomics on two do not wait f
 // take 12 ns each, one after another, and a workgroup per tile adds two: with
 // one cell a forward step of 448 x 400 (512 x 512) wet cells took 39.8 (52.5) us,
 // with two 32.8 (42.1), with four 29.1 (36.4).  But every tile of a step reads
-// them all: four cost 64 members and 1531 x 1207 cells 1 to 2 % where two cost
-// nothing.
+// them all: four cost 1531 x 1207 cells 2 %, and two cost 256 members of 90,000
+// cells 0.7 % and gain them nothing.  So there are two where members hold more
+// than 512 tiles (64 x 4) each, else one.
 constexpr int NRED = 2;
 
 constexpr int BLOCK = 256;
@@ -186,6 +187,7 @@ struct StepArgs {
   double* kact;          // [n] forward kact of U
   RedDev* red;           // [ninst * NRED] of this step
   RedDev* red_next;      // [ninst * NRED] of the next step (fold)
+  int nred;              // cells of a member in use (reduction_cells)
   double* dt_rec;        // [ninst * max_steps]
   double* time;          // [ninst] after the last step taken
   double* clock;         // [ninst * (max_steps + 1)]: before each step (fold)
@@ -252,8 +254,9 @@ __device__ __forceinline__ double cfl_dt(const A& a, const InstDev& I, const Red
 }
 
 // A workgroup's terms into one of the member's cells, workgroups in turn.
-__device__ __forceinline__ void red_add(RedDev* red, int b, double minev, double hmax) {
-  RedDev* r = red + (long long)b * NRED + blockIdx.x % NRED;
+template <class A>
+__device__ __forceinline__ void red_add(const A& a, int b, double minev, double hmax) {
+  RedDev* r = a.red + (long long)b * NRED + (int)blockIdx.x % a.nred;
   if (minev < HUGE_VAL) atomicMin(&r->min_ev, (unsigned long long)__double_as_longlong(minev));
   if (hmax > 0.) atomicMax(&r->hmax, (unsigned long long)__double_as_longlong(hmax));
 }
@@ -262,6 +265,8 @@ __device__ __forceinline__ void red_clear(RedDev* red, int b, int k) {
   red[(long long)b * NRED + k] =
       RedDev{(unsigned long long)__double_as_longlong(10000000.), 0ull};
 }
+
+inline int reduction_cells(int ntiles, int ninst) { return ntiles > 512LL * ninst ? NRED : 1; }
 
 // The dt of member b at this step.  a.fold: it is made here, by every workgroup
 // alike, from the reduction cells the coefficient pass filled, instead of in a
@@ -276,9 +281,9 @@ __device__ __forceinline__ double step_dt(const A& a, int b, bool own) {
   if (!a.fold) return *rec;
   const InstDev& I = a.inst[b];
   RedDev R = a.red[(long long)b * NRED];
-#pragma unroll
-  for (int k = 1; k < NRED; k++) {
-    const RedDev q = a.red[(long long)b * NRED + k];
+  static_assert(NRED == 2, "one more cell");
+  if (a.nred > 1) {
+    const RedDev q = a.red[(long long)b * NRED + 1];
     R.min_ev = q.min_ev < R.min_ev ? q.min_ev : R.min_ev;
     R.hmax = q.hmax > R.hmax ? q.hmax : R.hmax;
   }
@@ -360,6 +365,7 @@ struct StepArgsM {
   float* kact;
   RedDev* red;           // as in StepArgs, down to fold
   RedDev* red_next;
+  int nred;
   double* dt_rec;
   double* time;
   double* clock;

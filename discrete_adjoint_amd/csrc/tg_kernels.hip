@@ -200,7 +200,7 @@ __device__ __forceinline__ void coef_cell(const StepArgs& a, const InstDev& I, i
 
 // The workgroup's CFL terms into the member's reduction cells (every thread
 // calls it; any: some thread has one).
-__device__ __forceinline__ void coef_reduce(RedDev* red, int b, double minev, double hmax,
+__device__ __forceinline__ void coef_reduce(const StepArgs& a, int b, double minev, double hmax,
                                             bool any) {
   if (!__syncthreads_or(any)) return;
   __shared__ double smin[BLOCK / 64], smax[BLOCK / 64];
@@ -214,7 +214,7 @@ __device__ __forceinline__ void coef_reduce(RedDev* red, int b, double minev, do
       minev = (smin[k] < minev) ? smin[k] : minev;
       hmax = (smax[k] > hmax) ? smax[k] : hmax;
     }
-    red_add(red, b, minev, hmax);
+    red_add(a, b, minev, hmax);
   }
 }
 
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(BLOCK) void k_coef(StepArgs a, int reduce) {
   for (int k = (int)threadIdx.x; k < n; k += BLOCK)
     coef_cell(a, I, B.x0 + s_cell[k] % MARK_W, B.y0 + s_cell[k] / MARK_W, s_h[k], reduce, minev,
               hmax);
-  if (reduce) coef_reduce(a.red, B.inst, minev, hmax, (int)threadIdx.x < n);
+  if (reduce) coef_reduce(a, B.inst, minev, hmax, (int)threadIdx.x < n);
 }
 
 // the tile of a workgroup of the passes over every tile
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(BLOCK) void k_coef_tile(StepArgs a, int reduce) {
     const int cnt = __syncthreads_count(act && !wet);
     if (threadIdx.x == 0 && cnt) atomicAdd(a.short_cells, (unsigned long long)cnt);
   }
-  if (reduce) coef_reduce(a.red, t.inst, minev, hmax, wet);
+  if (reduce) coef_reduce(a, t.inst, minev, hmax, wet);
 }
 
 // Both sets of reduction cells, and each member's clock slot of the step about

@@ -171,7 +171,7 @@ __global__ __launch_bounds__(BLOCK) void k32_coef(StepArgsM<S> a, int reduce) {
         minev = (smin[k] < minev) ? smin[k] : minev;
         hmax = (smax[k] > hmax) ? smax[k] : hmax;
       }
-      red_add(a.red, t.inst, minev, hmax);
+      red_add(a, t.inst, minev, hmax);
     }
   }
 }

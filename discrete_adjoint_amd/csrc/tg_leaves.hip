@@ -127,7 +127,7 @@ __global__ __launch_bounds__(BLOCK) void k_leaf_coef(StepArgs a, LeafDev L, int 
         minev = (smin[k] < minev) ? smin[k] : minev;
         hmax = (smax[k] > hmax) ? smax[k] : hmax;
       }
-      red_add(a.red, 0, minev, hmax);
+      red_add(a, 0, minev, hmax);
     }
   }
 }

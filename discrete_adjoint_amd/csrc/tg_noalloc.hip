@@ -179,6 +179,7 @@ int step_on_device(const tg_config* cfg, const tg_noalloc_block* blk, const tg_p
   a.red = (RedDev*)(base + OFF_RED);
   a.dt_rec = &md->dt_rec;
   a.red_next = a.red + NRED;
+  a.nred = reduction_cells(ntiles, 1);
   a.time = &md->time;
   a.clock = md->clock;
   a.fold = 1;
