@@ -431,6 +431,11 @@ struct AdjArgsM {
 // most workgroups of the FP64 thin-layer adjoint pass (strides over its list):
 // as many as the chip holds of them at once
 constexpr int THIN_GRID = 512;
+// past this many tiles the cells that take a thread each have a kernel of their
+// own (k32_adjoint_thin_many).  Reverse steps of an ensemble in one kernel / two:
+// 96 members, 32,688 tiles 301 / 309 us, 128 members, 45,344 tiles 403 / 386,
+// 192 members 557 / 538 (TG_FP32; TG_MIXED the same way)
+constexpr int THIN_MANY_TILES = 32768;
 // workgroups of the update / adjoint passes that stride over the compacted
 // list of tiles taking the full path (a fixed grid, for graph capture):
 // 16 per CU, so that the workgroups left without a tile exit early while

@@ -1072,7 +1072,7 @@ __device__ __forceinline__ void thin_by_thread(const AdjArgsM<S>& a, int n) {
 }
 
 template <class S, int TX>
-__global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
+__global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a, int many) {
   using F = double;
   __shared__ ThinLds L;
   const bool want_dphi = a.dphi_part != nullptr;
@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
   const int n = *a.thin_count;
   if (blockIdx.x == 0 && threadIdx.x == 0) *a.tile_count = *a.thin_next = 0;
   if (n > THIN_CELLS * (int)gridDim.x) {
-    thin_by_thread<S, TX>(a, n);
+    if (!many) thin_by_thread<S, TX>(a, n);
     return;
   }
 #pragma unroll 1
@@ -1153,6 +1153,17 @@ __global__ __launch_bounds__(BLOCK) void k32_adjoint_thin(AdjArgsM<S> a) {
   }
 }
 
+// The threads' way in a kernel of its own for the largest meshes.  Beside the
+// lanes' way it gets one wave a SIMD, which is all that a thread for each of up
+// to 65,536 cells needs (bounded to two the lanes' way spills: 20.1 -> 21.5 us);
+// past that a second one counts (a reverse step of 256 members, 23 M cells, FP32:
+// 141 us against 128 and 5 for the lanes' launch, which finds too many).
+template <class S, int TX>
+__global__ __launch_bounds__(BLOCK, 2) void k32_adjoint_thin_many(AdjArgsM<S> a) {
+  const int n = *a.thin_count;
+  if (n > THIN_CELLS * THIN_GRID) thin_by_thread<S, TX>(a, n);
+}
+
 }  // namespace
 
 #define TG_LAUNCH_TX(shape, KERNEL, S, GRID, ...)                                       \
@@ -1189,7 +1200,9 @@ void launch_adjoint_m(const AdjArgsM<S>& a, hipStream_t s) {
   }
   // (a tile's 256 cells are eight rounds of a workgroup; most tiles have none)
   const int g = 4LL * a.ntiles < THIN_GRID ? 4 * a.ntiles : THIN_GRID;
-  TG_LAUNCH_TX(a.shape, k32_adjoint_thin, S, dim3(g), s, a);
+  const int many = a.ntiles > THIN_MANY_TILES;
+  TG_LAUNCH_TX(a.shape, k32_adjoint_thin, S, dim3(g), s, a, many);
+  if (many) TG_LAUNCH_TX(a.shape, k32_adjoint_thin_many, S, dim3(2 * THIN_GRID), s, a);
 }
 template void launch_coef_m<float>(const StepArgsM<float>&, bool, hipStream_t);
 template void launch_coef_m<double>(const StepArgsM<double>&, bool, hipStream_t);

@@ -243,3 +243,33 @@ def test_reverse_steps_by_the_list(oracle_lib, tile):
             terms = np.abs(lam * orc.dstep_dphi(_U(pb), s, dt).reshape(3, -1)).sum()
             assert abs(g - dphi) <= 1e-12 * terms, s
             assert abs(dphi) > 1e-6 * terms
+
+
+@pytest.mark.parametrize("rows", [300, 3000])   # 2400 and 24,000 thin cells
+def test_fp32_thin_cells_of_a_very_large_mesh(oracle_lib, rows):
+    """Past 32,768 tiles the cells next to a thin layer go to one of two kernels,
+    by their number (16,384).  Bar: that of the FP32 reverse step elsewhere, 1e-4
+    in norm; a second step repeats the first bit for bit."""
+    nx, ny = 8, 131200
+    _say(f"case list path fp32 thin cells {nx}x{ny} rows {rows}")
+    pb = small_flow_problem(nx, ny, 4)
+    rng = np.random.default_rng(rows)
+    at = np.arange(pb.n) // nx
+    thin = (at >= 700) & (at < 700 + rows)
+    pb.h[thin], pb.hu[thin], pb.hv[thin] = 5e-4, 3e-3, -2e-3
+    lam = rng.normal(size=(3, pb.n)) * (pb.h > 0)
+    orc = oracle_lib.Oracle.from_problem(pb)
+    ref, dphi = orc.adjoint_step(_U(pb), 60, 0.05, lam, want_dphi=True)
+    terms = np.abs(lam * orc.dstep_dphi(_U(pb), 60, 0.05)).sum()
+    ref = np.asarray(ref).reshape(3, -1)
+    with Simulation(pb, max_steps=64, precision=_lib.TG_FWD64_ADJ32) as sim:
+        got, g = sim.adjoint_step_grad(60, 0.05, lam)
+        assert np.linalg.norm(got - ref) <= 1e-4 * np.linalg.norm(ref)
+        assert np.linalg.norm((got - ref)[:, thin]) <= 1e-4 * np.linalg.norm(ref[:, thin])
+        assert abs(g - dphi) <= 1e-4 * terms
+        again, _ = sim.adjoint_step_grad(60, 0.05, lam)
+        assert np.array_equal(again, got)
+        lam[:, thin] = 0.0                            # and after one without them
+        sim.adjoint_step(60, 0.05, lam)
+        assert np.array_equal(sim.adjoint_step(60, 0.05, lam),
+                              sim.adjoint_step_grad(60, 0.05, lam)[0])
