@@ -195,11 +195,14 @@ __device__ __forceinline__ Hfv rec_hfv32(const Lds32<W, TX>& L, int dir, int r) 
              L.g[r], L.wet[r] != 0);
 }
 
-// One workgroup per tile, which also makes dt (step_dt): a pass of its own
-// cost 4.4 us beside this one's 8.4 (389 x 301 cells).  A tile whose cells and frame are all below tiny
-// has every face flux zero and no sources: its cells take the update's own
-// arithmetic with zero fluxes, without the flux and slope work.
-template <class S, int TX>
+// One workgroup per tile.  FOLD: it also makes dt (step_dt); a pass of its own
+// cost 4.4 us beside this one's 8.4 (389 x 301 cells).  A recomputed or replayed
+// step has its dt and loads it in a kernel without that code, which held up every
+// tile (256 members of 23 M cells, TG_FP32: 131 us a recomputed step against 140).
+// A tile whose cells and frame are all below tiny has every face flux zero and no
+// sources: its cells take the update's own arithmetic with zero fluxes, without
+// the flux and slope work.
+template <class S, int TX, bool FOLD>
 __global__ __launch_bounds__(BLOCK) void k32_update(StepArgsM<S> a) {
   using W = Wt<S>;
   using L32 = Lds32<W, TX>;
@@ -215,17 +218,23 @@ __global__ __launch_bounds__(BLOCK) void k32_update(StepArgsM<S> a) {
   // never do; a dt that is not finite makes every cell so and is reported by
   // the one that keeps the records, as the state it would give is: see
   // k_spoil_members.)
+  double dt = 0.;
+  if constexpr (!FOLD) dt = a.dt_rec[(long long)t.inst * a.max_steps + a.step];
   const bool skip =
-      a.mk_in && a.mk_out && out_marked_zero<TX>(a.mk_out, t) &&
+      (FOLD || isfinite(dt)) && a.mk_in && a.mk_out && out_marked_zero<TX>(a.mk_out, t) &&
       tile_marked_zero<TX>(a.mk_in, t, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 0, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 1, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 2, a.zbytes) &&
       side_tile_zero<TX>(a.mk_in, t, I, 3, a.zbytes);
-  if (skip && !own) return;
-  const double dt = step_dt(a, t.inst, own);
-  if (own && threadIdx.x == 0 && !isfinite(dt)) atomicOr(a.err, 1);
-  if (skip && isfinite(dt)) return;
+  if constexpr (FOLD) {
+    if (skip && !own) return;
+    dt = step_dt(a, t.inst, own);
+    if (own && threadIdx.x == 0 && !isfinite(dt)) atomicOr(a.err, 1);
+    if (skip && isfinite(dt)) return;
+  } else {
+    if (skip) return;
+  }
   const Cell q = cell_of<TX>(t, I);
   const long long nx = I.nx;
   const W tiny = (W)a.tiny, gamma = (W)a.gamma;
@@ -1181,7 +1190,17 @@ void launch_coef_m(const StepArgsM<S>& a, bool reduce, hipStream_t s) {
 }
 template <class S>
 void launch_update_m(const StepArgsM<S>& a, hipStream_t s) {
-  TG_LAUNCH_TX(a.shape, k32_update, S, dim3(a.ntiles), s, a);
+#define TG_UPD32(TX)                                                                            \
+  if (a.fold)                                                                                  \
+    hipLaunchKernelGGL((k32_update<S, TX, true>), dim3(a.ntiles), dim3(BLOCK), 0, s, a);       \
+  else                                                                                         \
+    hipLaunchKernelGGL((k32_update<S, TX, false>), dim3(a.ntiles), dim3(BLOCK), 0, s, a)
+  switch (SHAPE_TX[a.shape]) {
+    case 64: TG_UPD32(64); break;
+    case 32: TG_UPD32(32); break;
+    default: TG_UPD32(16); break;
+  }
+#undef TG_UPD32
 }
 template <class S>
 void launch_adjoint_m(const AdjArgsM<S>& a, hipStream_t s) {
