@@ -1016,9 +1016,9 @@ __global__ __launch_bounds__(adj32_threads<TX>()) void k32_adjoint_tile(AdjArgsM
 // thread per cell walks for the neighbours' records one after another, three
 // times over (a front of some thousand cells, 389 x 301: 34.5 us against 19.6).
 // More cells than that (16,384): a thread each.  The lanes' time goes up by a
-// round at a time, the threads' stays one chain until 131,072 (96 members of
+// round at a time, the threads' stays one chain until 65,536 (96 members of
 // 64 to 512 cells a side, 32,768 to 65,536 thin cells: 73 us by lanes alone,
-// 52 by threads).
+// 52 by threads; beyond: k32_adjoint_thin_many).
 constexpr int THIN_LANES = 8, THIN_CELLS = BLOCK / THIN_LANES;
 struct ThinLds {
   DualInfoT<double> self[THIN_CELLS];
